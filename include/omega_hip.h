@@ -75,7 +75,9 @@ typedef struct omg_geom_desc {
      * their backprojection into y-fastest buffers, where the lanes of a wave share cache lines);
      * reserved[4] is the device-memory budget in MiB of projectors 2 and 3's tube lists (each
      * measurement range's voxel indices and table weights, traced once and then streamed by the
-     * projections; 0: 16384 MiB, < 0: off, every call traces the tubes).
+     * projections; 0: 16384 MiB, < 0: off, every call traces the tubes), and of the lists that subset
+     * iterations of direct-plane sinograms keep (the voxels and lengths of one plane, shared by all planes;
+     * projectors 1, 2 and 4, built by a handle's first iteration that may allocate).
      * Zero = automatic. */
     int32_t reserved[8];
     /* measurement-level subsets of PET sinograms (subset types 1-5: indexMaker's `index`,
@@ -200,7 +202,8 @@ int omg_ct_osem_subset_iteration(const omg_geom* g, int64_t first, int64_t n_mea
 
 /* omg_osem_subset_iteration_ex without allocation. No counterpart in the reference: it is for callers that
  * cannot allocate device memory (code under HIP graph capture, serving loops, harnesses that forbid
- * hipMalloc). The same kernels in the same order, with every work buffer (OSL gradient, rhs image, slice map,
+ * hipMalloc). The same kernels in the same order (a direct-plane handle without its lists -- they are built by
+ * an allocating iteration -- takes the tracing kernels, whose sums differ in rounding), with every work buffer (OSL gradient, rhs image, slice map,
  * the direct-plane kernels' per-workgroup partial slices, the voxel-driven path's per-LOR buffers) carved
  * out of one library-owned device array of 64 MiB (16,777,216 floats) that each GPU holds until the process
  * ends. A call that needs more (2 N + Nz floats for an image of N voxels and Nz slices, plus, on the

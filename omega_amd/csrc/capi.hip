@@ -1,5 +1,6 @@
 // capi.hip -- geometry handles, error text and version of libomega_hip.so.
 #include "geom.hpp"
+#include "plane.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -64,6 +65,10 @@ static int fixed_need(const omg_geom* g, size_t floats, const char* what) {
 float* scratch_ptr(const omg_geom* g) { return t_fixed ? t_fixed->base + fixed_work_floats(g) : g->scratch; }
 float* work_ptr(const omg_geom* g) { return t_fixed ? t_fixed->base : g->work; }
 float* q_ptr(const omg_geom* g) { return t_fixed ? t_fixed->base + fixed_work_floats(g) : g->vbp_q; }
+
+bool scratch_fits(const omg_geom* g, size_t floats) {
+    return !t_fixed || fixed_work_floats(g) + floats <= t_fixed->floats;
+}
 
 int scratch_reserve(omg_geom* g, size_t floats) {
     if (t_fixed) return fixed_need(g, floats, "partial images");
@@ -351,6 +356,7 @@ extern "C" int omg_geom_destroy(omg_geom* g) {
     bdd_release(g);
     orth_release(g);
     vbp_release(g);
+    plane_release(g);
     delete g;
     return OMG_OK;
 }

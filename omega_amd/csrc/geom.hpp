@@ -5,6 +5,8 @@
 
 #include <vector>
 
+namespace omg { struct PlanePlan; }
+
 struct omg_geom {
     omg_geom_desc d;          // caller's description (host table pointers cleared after upload)
     float* x_dev = nullptr;   // coordinate tables on the device
@@ -37,6 +39,9 @@ struct omg_geom {
     // Projectors 2 and 3: the tube lists of the measurement ranges used so far, kept on the device
     // (orth.hip; omg_geom_desc.reserved[4] sets the budget).
     struct TubeCache* tubes = nullptr;
+    // Direct-plane sinograms: the one 2-D system's lists (plane.hip), built by the first subset iteration that
+    // may allocate.
+    omg::PlanePlan* plane = nullptr;
     // Workgroups per plane for the planar kernels (omg_geom_desc.reserved[1]; 0 = automatic).
     int32_t planar_groups = 0;
     // Library-owned scratch (floats) for partial images; grown on demand, freed with the handle.
@@ -99,6 +104,10 @@ static inline SidArgs make_sid_args(const omg_geom* g, int64_t first, int64_t n)
     return a;
 }
 
+// grad = beta * RDP gradient of u with the zero boundary (image.hip; omg_rdp_gradient adds to grad instead).
+int rdp_write(const float* u, float* grad, uint32_t Nx, uint32_t Ny, uint32_t Nz, float gamma, float epps, float beta,
+              hipStream_t s);
+
 // Time-of-flight projections (tof.hip): measurement arrays hold tof_bins blocks of n values.
 int tof_forward(const omg_geom* g, int64_t first, int64_t n, const float* img, float* y, hipStream_t s);
 int tof_backward(const omg_geom* g, int64_t first, int64_t n, const float* yin, float* rhs, float* sens,
@@ -140,6 +149,9 @@ bool fixed_region_active();
 // Ensures scratch_ptr(g) holds at least `floats` floats (hipMalloc on growth; synchronises the device then).
 int scratch_reserve(omg_geom* g, size_t floats);
 float* scratch_ptr(const omg_geom* g);
+
+// False when a held fixed region is too small for scratch_reserve(g, floats).
+bool scratch_fits(const omg_geom* g, size_t floats);
 
 // Ensures work_ptr(g) holds the fused-iteration buffers for an image of N voxels.
 int work_reserve(omg_geom* g, uint32_t N);

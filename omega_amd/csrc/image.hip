@@ -12,7 +12,8 @@ constexpr int kEB = 256;
 
 // RDP gradient (source/cpp/RDP.h:4-78; source/opencl/auxKernels.cl:802-871).
 // Neighbour pairs are evaluated as the reference's float2 lanes: lane 0 = (+x, +y, +z),
-// lane 1 = (-x, -y, -z), each summed x, y, z; NaN lanes -> 0; grad += beta * (lane0 + lane1).
+// lane 1 = (-x, -y, -z), each summed x, y, z; NaN lanes -> 0; grad += beta * (lane0 + lane1), or = without ADD.
+template <bool ADD>
 __global__ __launch_bounds__(kEB) void k_rdp(const float* __restrict__ u, float* __restrict__ grad, uint32_t Nx,
                                              uint32_t Ny, uint32_t Nz, float gamma, float epps, float beta, int clamp) {
     const uint32_t Nxy = Nx * Ny;
@@ -44,7 +45,8 @@ __global__ __launch_bounds__(kEB) void k_rdp(const float* __restrict__ u, float*
     l1 = l1 + rdp_term(uj, zm, gamma, epps);
     if (isnan(l0)) l0 = 0.f;
     if (isnan(l1)) l1 = 0.f;
-    grad[n] += beta * (l0 + l1);
+    if (ADD) grad[n] += beta * (l0 + l1);
+    else grad[n] = beta * (l0 + l1);
 }
 
 __global__ __launch_bounds__(kEB) void k_ratio(const float* __restrict__ y, float* __restrict__ r, int64_t n, float epps) {
@@ -190,6 +192,14 @@ static unsigned stream_grid(int64_t n) {
     return (unsigned)(g < 8192 ? (g > 0 ? g : 1) : 8192);
 }
 
+int rdp_write(const float* u, float* grad, uint32_t Nx, uint32_t Ny, uint32_t Nz, float gamma, float epps, float beta,
+              hipStream_t s) {
+    hipLaunchKernelGGL(k_rdp<false>, dim3(grid_for((int64_t)Nx * Ny * Nz, kEB)), dim3(kEB), 0, s, u, grad, Nx, Ny, Nz,
+                       gamma, epps, beta, 0);
+    OMG_CHECK_LAUNCH();
+    return OMG_OK;
+}
+
 }  // namespace omg
 
 using namespace omg;
@@ -200,7 +210,7 @@ extern "C" int omg_rdp_gradient(const float* u, float* grad, uint32_t Nx, uint32
     OMG_REQUIRE(Nx > 0 && Ny > 0 && Nz > 0, "empty image");
     OMG_REQUIRE((uint64_t)Nx * Ny * Nz < (1ull << 32), "image exceeds 2^32 voxels");
     OMG_REQUIRE(boundary == 0 || boundary == 1, "boundary must be 0 (zero) or 1 (clamp)");
-    hipLaunchKernelGGL(k_rdp, dim3(grid_for((int64_t)Nx * Ny * Nz, kEB)), dim3(kEB), 0, as_stream(stream), u, grad, Nx, Ny, Nz,
+    hipLaunchKernelGGL(k_rdp<true>, dim3(grid_for((int64_t)Nx * Ny * Nz, kEB)), dim3(kEB), 0, as_stream(stream), u, grad, Nx, Ny, Nz,
                        gamma, epps, beta, (int)boundary);
     OMG_CHECK_LAUNCH();
     return OMG_OK;

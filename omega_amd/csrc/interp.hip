@@ -26,6 +26,7 @@
 // bit-identical to the oracle's restatement; the oracle's exp is the host's, so attenuation factors agree to
 // float rounding.
 #include "geom.hpp"
+#include "plane.hpp"
 
 namespace omg {
 
@@ -577,6 +578,78 @@ static InterpArgs make_interp_args(const omg_geom* g, int64_t first, int64_t n) 
     ia.atn_image = d.atten_mode == 1;
     ia.a.atten_lor = d.atten_mode == 2;
     return ia;
+}
+
+// ---- the 2-D system's lists of a direct-plane sinogram (plane.hip) ------------------------------------
+// Forward samples (the four corners' first pixel, the steps to the others, the fractions) and the voxels of the
+// backprojection's samples, relative to the plane's slice.
+__global__ __launch_bounds__(kInterpBlock) void k_interp_plane(InterpArgs ia, PlaneFill f) {
+    const uint32_t row = blockIdx.x * kInterpBlock + threadIdx.x;
+    if ((int64_t)row >= ia.a.nmeas) return;
+    const uint32_t Nx = ia.a.Nx, Ny = ia.a.Ny;
+    Samples S;
+    uint32_t k = 0, m = 0;
+    if (interp_samples(ia, row, S)) {
+        interp_walk(ia, S, S.t0, S.n, [&](IF3 p) {
+            if (f.samp) {
+                uint32_t x0, x1, y0, y1;
+                float a, b;
+                tex_axis(p.x, Nx, x0, x1, a);
+                tex_axis(p.y, Ny, y0, y1, b);
+                f.samp[(size_t)f.soff[row / kLI] + m * kLI + row % kLI] =
+                    make_uint4((y0 * Nx + x0) | (x1 - x0) << 30 | (y1 - y0) << 31, __float_as_uint(a),
+                               __float_as_uint(b), __float_as_uint(S.stepLen));
+            }
+            m++;
+        });
+        float t0 = S.t0;
+        uint32_t n = S.n;
+        if (ia.a.atten && ia.atn_image && ia.dL > 0.f) {
+            t0 = S.tStart + S.tStep / 10.f;
+            n = t0 <= S.tEnd ? (uint32_t)((S.tEnd - t0) / S.tStep) + 1u : 0u;
+        }
+        interp_walk(ia, S, t0, n, [&](IF3 p) {
+            const uint32_t ind = (uint32_t)fmaxf(p.x * (float)Nx, 0.f) + (uint32_t)fmaxf(p.y * (float)Ny, 0.f) * Nx;
+            plane_put(f, row, k, f.slice_base + ind, S.stepLen);
+        });
+    }
+    f.cnt[row] = k;
+    f.scnt[row] = m;
+}
+
+__global__ __launch_bounds__(kInterpBlock) void k_interp_weight(InterpArgs ia, float* __restrict__ w) {
+    const int64_t lo = (int64_t)blockIdx.x * kInterpBlock + threadIdx.x;
+    if (lo >= ia.a.nmeas) return;
+    Samples S;
+    w[lo] = interp_samples(ia, lo, S) ? interp_weight(ia, lo, S.L, true) : 0.f;
+}
+
+int interp_plane_trace(const omg_geom* g, uint32_t plane, const PlaneFill& f, hipStream_t s) {
+    const uint32_t per = g->d.size_x * g->d.size_y;
+    const InterpArgs ia = make_interp_args(g, plane, per);
+    hipLaunchKernelGGL(k_interp_plane, dim3(grid_for(per, kInterpBlock)), dim3(kInterpBlock), 0, s, ia, f);
+    OMG_CHECK_LAUNCH();
+    return OMG_OK;
+}
+
+int interp_plane_weights(const omg_geom* g, float* w, hipStream_t s) {
+    const int64_t n = (int64_t)g->d.size_x * g->d.size_y * g->d.n_proj;
+    const InterpArgs ia = make_interp_args(g, 0, n);
+    hipLaunchKernelGGL(k_interp_weight, dim3(grid_for(n, kInterpBlock)), dim3(kInterpBlock), 0, s, ia, w);
+    OMG_CHECK_LAUNCH();
+    return OMG_OK;
+}
+
+// The slice that the walk's arithmetic gives for a plane's z; planes on or outside the image's end faces miss.
+void interp_plane_slices(const omg_geom* g, std::vector<int32_t>& out) {
+    const InterpArgs ia = make_interp_args(g, 0, 0);
+    out.resize(g->d.n_proj);
+    for (uint32_t p = 0; p < g->d.n_proj; p++) {
+        const float z = g->z_host[2 * (size_t)p];
+        const float pz = ((0.f + z) - ia.b.z) * ia.scale.z;
+        const uint32_t zb = (uint32_t)fmaxf(pz * (float)g->d.Nz, 0.f);
+        out[p] = z > ia.b.z && z < ia.bmax.z && zb < g->d.Nz ? (int32_t)zb : -1;
+    }
 }
 
 // LDS of the TOF kernels: FP [bins: the LOR's sums][bins: one ray's sums][bins: weights], BP the first two

@@ -27,6 +27,7 @@
 #include <type_traits>
 
 #include "geom.hpp"
+#include "plane.hpp"
 
 #include <algorithm>
 #include <vector>
@@ -271,6 +272,19 @@ __device__ __forceinline__ int o_sweep(const T& t, int tempi, float cx, int temp
     return uu;
 }
 
+// Corrections in the reference kernel's order: factors made from an attenuation image first (-DATN,
+// projectorType123.cl:975-976); given per-LOR factors (-DATNM) after the global factor (:986-988), or
+// before it on the axis-parallel path (perpendicular_elements, general_opencl_functions.h:1722-1734).
+__device__ __forceinline__ float orth_chain(const SidArgs& g, int64_t lo, float w, bool perp) {
+    if (g.atten && !g.atten_lor) w *= g.atten[lo];
+    if (g.norm) w *= g.norm[lo];
+    if (g.scat) w *= g.scat[lo];
+    if (g.atten && g.atten_lor && perp) w *= g.atten[lo];
+    w *= g.global_factor;
+    if (g.atten && g.atten_lor && !perp) w *= g.atten[lo];
+    return w;
+}
+
 // One LOR: visit(ind, w) for every voxel of its tube. Returns the LOR weight temp (0: ray skipped); with
 // temp_out, temp is also stored there before the first visit (for callers whose visit applies it).
 // No time of flight: nothing to do per stretch of the centre ray.
@@ -309,18 +323,7 @@ __device__ __forceinline__ float orth_lor_t(const OrthArgs& oa, int64_t lo, V&& 
         t.bmax = oa.bmax;
         t.vmax = oa.vmax;
     }
-    // corrections in the reference kernel's order: factors made from an attenuation image first (-DATN,
-    // projectorType123.cl:975-976); given per-LOR factors (-DATNM) after the global factor (:986-988), or
-    // before it on the axis-parallel path (perpendicular_elements, general_opencl_functions.h:1722-1734)
-    auto chain = [&](float w, bool perp) {
-        if (g.atten && !g.atten_lor) w *= g.atten[lo];
-        if (g.norm) w *= g.norm[lo];
-        if (g.scat) w *= g.scat[lo];
-        if (g.atten && g.atten_lor && perp) w *= g.atten[lo];
-        w *= g.global_factor;
-        if (g.atten && g.atten_lor && !perp) w *= g.atten[lo];
-        return w;
-    };
+    auto chain = [&](float w, bool perp) { return orth_chain(g, lo, w, perp); };
     // projector 3: TotV = L * (1/pi) * R^2 (projectorType123.cl:505); an axis-parallel ray's weight is the
     // corrections' product times 1 / TotV (:641-643), any other ray's starts from 1 / TotV (:952)
     const float inv_v = vol ? 1.f / (L * (float)M_1_PI * oa.width * oa.width) : 1.f;
@@ -1146,11 +1149,8 @@ using namespace omg;
 // with the axial sweep, the centres of the slices next to every plane's slice lie at least
 // 0.99 * width * (1 + 1e-3) from the plane, so no voxel of another slice passes the tube cut-off
 // (a voxel's distance to an in-plane LOR is at least its axial offset).
-static bool orth_planar_check(const omg_geom* g) {
+static bool orth_in_slice(const omg_geom* g) {
     const omg_geom_desc& d = g->d;
-    if (!g->planar || d.mode != OMG_MODE_PET_SINO || d.Nx % 4 != 0) return false;
-    const size_t Nyx = (size_t)d.Nx * d.Ny;
-    if (Nyx * 8 + sizeof(float) * (kPlanarTPB + kPlanarTPB / 64) > 160 * 1024) return false;
     if (!(d.orth_flags & 2)) return true;
     const double cut = (1.0 - (double)kOrthThr) * (double)d.orth_width * (1.0 + 1e-3);
     for (uint32_t p = 0; p < d.n_proj; p++) {
@@ -1165,6 +1165,71 @@ static bool orth_planar_check(const omg_geom* g) {
     }
     return true;
 }
+
+static bool orth_planar_check(const omg_geom* g) {
+    const omg_geom_desc& d = g->d;
+    if (!g->planar || d.mode != OMG_MODE_PET_SINO || d.Nx % 4 != 0) return false;
+    const size_t Nyx = (size_t)d.Nx * d.Ny;
+    if (Nyx * 8 + sizeof(float) * (kPlanarTPB + kPlanarTPB / 64) > 160 * 1024) return false;
+    return orth_in_slice(g);
+}
+
+// ---- the 2-D system's lists of a direct-plane sinogram (plane.hip) ------------------------------------
+namespace omg {
+
+__global__ __launch_bounds__(kOrthBlock) void k_orth_plane(OrthArgs oa, PlaneFill f) {
+    const uint32_t row = blockIdx.x * kOrthBlock + threadIdx.x;
+    if ((int64_t)row >= oa.a.nmeas) return;
+    uint32_t k = 0;
+    orth_lor<false>(oa, row, [&](int64_t ind, float w) { plane_put(f, row, k, (uint32_t)ind, w); });
+    f.cnt[row] = k;
+}
+
+// The LOR weight orth_lor returns, without its walk (a LOR that misses the image has no list entries).
+__global__ __launch_bounds__(kOrthBlock) void k_orth_weight(OrthArgs oa, float* __restrict__ w) {
+    const int64_t lo = (int64_t)blockIdx.x * kOrthBlock + threadIdx.x;
+    if (lo >= oa.a.nmeas) return;
+    Ray r;
+    fetch_ray(oa.a, lo, r);
+    const bool perp = fabsf(r.zd - r.zs) < 1e-6f && (fabsf(r.yd - r.ys) < 1e-6f || fabsf(r.xd - r.xs) < 1e-6f);
+    w[lo] = orth_chain(oa.a, lo, 1.f, perp);
+}
+
+int orth_plane_trace(const omg_geom* g, uint32_t plane, const PlaneFill& f, hipStream_t s) {
+    const uint32_t per = g->d.size_x * g->d.size_y;
+    OrthArgs oa = make_orth_args(g, plane, per);
+    oa.a.norm = oa.a.atten = oa.a.scat = nullptr;
+    hipLaunchKernelGGL(k_orth_plane, dim3(grid_for(per, kOrthBlock)), dim3(kOrthBlock), 0, s, oa, f);
+    OMG_CHECK_LAUNCH();
+    return OMG_OK;
+}
+
+int orth_plane_weights(const omg_geom* g, float* w, hipStream_t s) {
+    const int64_t n = (int64_t)g->d.size_x * g->d.size_y * g->d.n_proj;
+    const OrthArgs oa = make_orth_args(g, 0, n);
+    hipLaunchKernelGGL(k_orth_weight, dim3(grid_for(n, kOrthBlock)), dim3(kOrthBlock), 0, s, oa, w);
+    OMG_CHECK_LAUNCH();
+    return OMG_OK;
+}
+
+bool orth_plane_ok(const omg_geom* g) {
+    const omg_geom_desc& d = g->d;
+    if (!g->planar || !orth_in_slice(g)) return false;
+    float off = 0.f;
+    bool any = false;
+    for (uint32_t p = 0; p < d.n_proj; p++) {
+        const float zs = g->z_host[2 * (size_t)p];
+        const int32_t tk = (int32_t)(fabsf(zs - d.bz) / d.dz);
+        if (tk < 0 || (uint32_t)tk >= d.Nz) continue;
+        const float o = (d.bz + (float)tk * d.dz + d.dz / 2.f) - zs;   // z of the slice centre above the plane
+        if (any && o != off) return false;
+        off = o;
+        any = true;
+    }
+    return true;
+}
+
+}  // namespace omg
 
 struct TubeEntry;
 static int tube_lists(const omg_geom* gc, int64_t first, int64_t n, hipStream_t s, const TubeEntry** out);

@@ -9,6 +9,7 @@
 // no CAS loop: built with -munsafe-fp-atomics) exactly where the reference CPU
 // uses `omp atomic` (source/cpp/projector_functions.h:652-656).
 #include "geom.hpp"
+#include "plane.hpp"
 
 #include <utility>
 #include <vector>
@@ -265,6 +266,49 @@ __global__ __launch_bounds__(kBlock) void k_siddon_trace(SidArgs a, int32_t* __r
         siddon_trace(a, lo, w, [&](uint32_t, float) { c++; });
     }
     counts[lo] = c;
+}
+
+// ---- the 2-D system's lists of a direct-plane sinogram (plane.hip) ------------------------------------
+__global__ __launch_bounds__(kBlock) void k_siddon_plane(SidArgs a, PlaneFill f) {
+    const uint32_t row = blockIdx.x * kBlock + threadIdx.x;
+    if ((int64_t)row >= a.nmeas) return;
+    uint32_t k = 0;
+    float w = 0.f;
+    siddon_trace(a, row, w, [&](uint32_t ind, float len) { plane_put(f, row, k, ind, len); });
+    f.cnt[row] = k;
+}
+
+__global__ __launch_bounds__(kBlock) void k_siddon_weight(SidArgs a, float* __restrict__ w) {
+    const int64_t lo = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (lo >= a.nmeas) return;
+    Walk wk;
+    float v = 0.f;
+    w[lo] = siddon_setup<false>(a, lo, wk, v) ? v : 0.f;
+}
+
+int siddon_plane_trace(const omg_geom* g, uint32_t plane, const PlaneFill& f, hipStream_t s) {
+    const uint32_t per = g->d.size_x * g->d.size_y;
+    SidArgs a = make_sid_args(g, plane, per);
+    a.norm = a.atten = a.scat = nullptr;   // lengths only
+    hipLaunchKernelGGL(k_siddon_plane, dim3(grid_for(per, kBlock)), dim3(kBlock), 0, s, a, f);
+    OMG_CHECK_LAUNCH();
+    return OMG_OK;
+}
+
+int siddon_plane_weights(const omg_geom* g, float* w, hipStream_t s) {
+    const int64_t n = (int64_t)g->d.size_x * g->d.size_y * g->d.n_proj;
+    const SidArgs a = make_sid_args(g, 0, n);
+    hipLaunchKernelGGL(k_siddon_weight, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, s, a, w);
+    OMG_CHECK_LAUNCH();
+    return OMG_OK;
+}
+
+void siddon_plane_slices(const omg_geom* g, std::vector<int32_t>& out) {
+    out.resize(g->d.n_proj);
+    for (uint32_t p = 0; p < g->d.n_proj; p++) {
+        const int32_t tk = (int32_t)(fabsf(g->z_host[2 * (size_t)p] - g->d.bz) / g->d.dz);
+        out[p] = tk < 0 || (uint32_t)tk >= g->d.Nz ? -1 : tk;
+    }
 }
 
 // ---- planar LDS kernels ---------------------------------------------------------------------------
@@ -926,12 +970,19 @@ int omg_osem_subset_iteration_impl(const omg_geom* g, int64_t first, int64_t n_m
     float* dU = nullptr;
     if (beta != 0.f) {
         dU = work_ptr(g);
-        hipLaunchKernelGGL(k_fill_f32, dim3(grid_for(N, 256)), dim3(256), 0, s, dU, N, 0.f);
-        OMG_CHECK_LAUNCH();
-        rc = omg_rdp_gradient(x, dU, g->d.Nx, g->d.Ny, g->d.Nz, gamma, epps, beta, 0, stream);
+        rc = rdp_write(x, dU, g->d.Nx, g->d.Ny, g->d.Nz, gamma, epps, beta, s);
         if (rc) return rc;
     }
     const uint32_t per = g->d.size_x * g->d.size_y;
+    // direct planes: two sparse products with the lists of their shared 2-D system
+    if (n_meas > 0 && !g->vbp_ok) {
+        if (const PlanePlan* pl = plane_plan(g, s)) {
+            bool done = false;
+            rc = plane_subset_iteration(gm, pl, first, n_meas, x, meas, additive, S, compute_sens, epps, dU, positivity,
+                                        s, &done);
+            if (rc || done) return rc;
+        }
+    }
     if (n_meas > 0 && g->d.projector_type == OMG_PROJ_SIDDON && planar_ok(g) && !g->force_generic &&
         unique_slices(g, first, (uint32_t)(n_meas / per))) {
         if (g->vbp_ok) {

@@ -19,6 +19,7 @@
 
 #include "common.hpp"
 #include "geom.hpp"
+#include "plane.hpp"
 #include "siddon_device.hpp"
 
 namespace omg {
@@ -195,6 +196,43 @@ __global__ __launch_bounds__(kTofBlock) void k_tof_osem(SidArgs a, const float* 
     tof_scatter(a, lo, acc, wl, c, rhs, sens);
 }
 
+// ---- the 2-D system's lists of a direct-plane sinogram (plane.hip) --------------------------------------
+__global__ __launch_bounds__(kTofBlock) void k_tof_plane(SidArgs a, PlaneFill f) {
+    const uint32_t row = blockIdx.x * kTofBlock + threadIdx.x;
+    if ((int64_t)row >= a.nmeas) return;
+    uint32_t k = 0;
+    float w = 0.f;
+    siddon_tof_trace(a, row, w, [&](uint32_t ind, float len, float, float, float) { plane_put(f, row, k, ind, len); });
+    f.cnt[row] = k;
+}
+
+// share[entry][b] = w_b / sum of the entry's voxel (the forward projection's weights and floored sum) and
+// lsum[entry] = length * sum_b share.
+__global__ __launch_bounds__(kTofBlock) void k_tof_shares(SidArgs a, PlaneFill f, uint32_t pitch,
+                                                          float* __restrict__ share, float* __restrict__ lsum) {
+    extern __shared__ float lds[];
+    const uint32_t row = blockIdx.x * kTofBlock + threadIdx.x;
+    if ((int64_t)row >= a.nmeas) return;
+    float* wl = lds + a.tof_bins * kTofBlock + threadIdx.x;
+    const TofCache c = tof_cache(a, lds);
+    *c.x = __builtin_nanf("");
+    uint32_t k = 0;
+    float w = 0.f;
+    siddon_tof_trace(a, row, w, [&](uint32_t, float len, float D, float DD, float esum) {
+        const float sum = tof_weights(a, esum, D, DD, wl, c);
+        if (esum != len) tof_weights(a, len, D, DD, wl, c);
+        const size_t pos = (size_t)f.off[row / kLI] + k * kLI + row % kLI;
+        float t = 0.f;
+        for (uint32_t b = 0; b < a.tof_bins; b++) {
+            const float q = wl[b * kTofBlock] / sum;
+            share[pos * pitch + b] = q;
+            t += q;
+        }
+        lsum[pos] = len * t;
+        k++;
+    });
+}
+
 // LDS per workgroup: [acc or yv: bins x lanes][wl: bins x lanes][cache p: bins x lanes][cache x: lanes]
 // and, with several rays per LOR, [tot: bins x lanes]: at most (4 * 64 + 1) * 64 * 4 B = 65,792 B.
 static size_t tof_lds(const SidArgs& a) {
@@ -213,6 +251,26 @@ static int tof_lds_attr() {
     OMG_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_tof_osem),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
     done = true;
+    return OMG_OK;
+}
+
+int tof_plane_trace(const omg_geom* g, uint32_t plane, const PlaneFill& f, hipStream_t s) {
+    const uint32_t per = g->d.size_x * g->d.size_y;
+    SidArgs a = make_sid_args(g, plane, per);
+    a.norm = a.atten = a.scat = nullptr;
+    hipLaunchKernelGGL(k_tof_plane, dim3(grid_for(per, kTofBlock)), dim3(kTofBlock), 0, s, a, f);
+    OMG_CHECK_LAUNCH();
+    return OMG_OK;
+}
+
+int tof_plane_shares(const omg_geom* g, uint32_t plane, const PlaneFill& f, uint32_t pitch, float* share, float* lsum,
+                     hipStream_t s) {
+    const uint32_t per = g->d.size_x * g->d.size_y;
+    SidArgs a = make_sid_args(g, plane, per);
+    a.norm = a.atten = a.scat = nullptr;
+    hipLaunchKernelGGL(k_tof_shares, dim3(grid_for(per, kTofBlock)), dim3(kTofBlock), tof_lds(a), s, a, f, pitch, share,
+                       lsum);
+    OMG_CHECK_LAUNCH();
     return OMG_OK;
 }
 

@@ -1,0 +1,107 @@
+"""Subset iterations of direct-plane sinograms from the shared 2-D system's lists (plane.hip) against the same
+iterations through the one-lane-per-LOR kernels (omg_geom_desc.reserved[0]).
+
+Both sum the same 32-bit products; the lists sum the backprojection in double, the other kernels in 32-bit
+atomics over at most ~400 LORs per voxel, so the images agree within about 400 * 2^-24 / sqrt(400) = 1.2e-6 per
+update; bar: 5e-6 relative L2 after two updates. Plane counts of 1, 2, 3, 5 and 9 per call cover every lane
+grouping and a second chunk of planes; images that are odd, non-square and smaller than one block; a plane
+outside the image; two planes of one slice (where the lists do not apply); every register group of TOF bins; the
+interpolation projector's far-face samples, which carry into the next slice.
+"""
+import numpy as np
+import pytest
+
+from omega_amd import _lib, geometry as G
+from tests.hip_helpers import make_geom, ptr, rel_l2
+
+pytestmark = pytest.mark.gpu
+EPPS = 1e-5
+
+
+def _scanner(nx, ny, nz, n_radial, n_angles, extra_z=()):
+    fov = 2.5 * max(nx, ny)
+    grid = G.Grid.from_fov(nx, ny, nz, fov, fov, 2.5 * nz)
+    x = G.ring_sinogram_xy(n_radial, n_angles, fov / n_radial, 1.25 * fov)
+    z = G.direct_planes_z(grid)
+    if extra_z:
+        z = np.concatenate([z, np.repeat(np.asarray(extra_z, np.float32), 2)])
+    return grid, x, z
+
+
+def _iterate(geom, grid, first, planes, per, meas, add, beta, seed):
+    import torch
+    rng = np.random.default_rng(seed)
+    x = torch.from_numpy((rng.random(grid.N) + 0.5).astype(np.float32)).cuda()
+    S = torch.zeros(grid.N, device="cuda")
+    for sens in (1, 0):
+        _lib.call("omg_osem_subset_iteration_ex", geom.handle, first, planes * per, ptr(x), ptr(meas), ptr(add),
+                  ptr(S), sens, EPPS, beta, 2.0, 1, None)
+    torch.cuda.synchronize()
+    return x.cpu().numpy(), S.cpu().numpy()
+
+
+def _compare(grid, x, z, n_radial, n_angles, first, planes, bins=1, beta=0.0, add=False, **kw):
+    import torch
+    per = n_radial * n_angles
+    rng = np.random.default_rng(planes + grid.Nx)
+    meas = torch.from_numpy(rng.poisson(3.0, planes * per * bins).astype(np.float32)).cuda()
+    a = torch.from_numpy((rng.random(planes * per) + 0.1).astype(np.float32)).cuda() if add else None
+    out = []
+    for generic in (False, True):
+        geom = make_geom(grid, x, z, n_radial, n_angles, generic=generic, **kw)
+        out.append(_iterate(geom, grid, first, planes, per, meas, a, beta, 3))
+        out.append(_iterate(geom, grid, first, planes, per, meas, a, beta, 3)) if not generic else None
+    (xa, Sa), (xb, _), (xg, Sg) = out
+    if bins <= 32:                  # more bins keep the one-lane-per-LOR kernels and their atomics
+        assert np.array_equal(xa, xb)   # the lists have a fixed order
+    e, es = rel_l2(xa, xg), rel_l2(Sa, Sg)
+    print(f"[plane] {grid.Nx}x{grid.Ny}x{grid.Nz} planes={planes} bins={bins} rel-L2 {e:.2e} sens {es:.2e}", flush=True)
+    assert e < 5e-6 and es < 5e-6
+    return xa
+
+
+@pytest.mark.parametrize("nx,ny,nz,n_radial,n_angles", [(32, 32, 11, 32, 40), (21, 34, 10, 29, 27), (5, 5, 9, 7, 9)])
+@pytest.mark.parametrize("planes", [1, 2, 3, 5, 9])
+def test_siddon(cuda, nx, ny, nz, n_radial, n_angles, planes):
+    grid, x, z = _scanner(nx, ny, nz, n_radial, n_angles)
+    norm = np.random.default_rng(0).random(n_radial * n_angles * nz).astype(np.float32) + 0.5
+    _compare(grid, x, z, n_radial, n_angles, 0 if planes == 9 else 1, planes, add=planes % 2 == 1,
+             beta=0.01 if planes > 2 else 0.0, norm=norm, global_factor=0.9)
+
+
+def test_plane_outside_and_shared_slice(cuda):
+    grid, x, z = _scanner(20, 20, 6, 24, 21, extra_z=(100.0, 1.25))   # beyond the image; slice 3's centre again
+    _compare(grid, x, z, 24, 21, 3, 4)      # planes 3, 4, 5 and the one outside
+    import torch
+    per = 24 * 21
+    geom = make_geom(grid, x, z, 24, 21)
+    gen = make_geom(grid, x, z, 24, 21, generic=True)
+    meas = torch.ones(8 * per, device="cuda")
+    a = _iterate(geom, grid, 0, 8, per, meas, None, 0.0, 5)[0]
+    b = _iterate(gen, grid, 0, 8, per, meas, None, 0.0, 5)[0]
+    assert rel_l2(a, b) < 5e-6
+
+
+@pytest.mark.parametrize("bins,planes", [(3, 2), (8, 9), (13, 1), (17, 5), (23, 3), (32, 2), (33, 2)])
+def test_tof(cuda, bins, planes):
+    grid, x, z = _scanner(22, 19, 10, 24, 21)
+    sigma = G.tof_sigma(300e-12)
+    centres = np.linspace(-40.0, 40.0, bins).astype(np.float32)
+    atten = np.full(grid.N, 0.004, np.float32)
+    _compare(grid, x, z, 24, 21, 1, planes, bins=bins, add=True, tof=(bins, sigma, centres, EPPS), atten=atten,
+             atten_mode=1)
+
+
+@pytest.mark.parametrize("n,flags,planes", [(32, 3, 5), (19, 3, 2), (20, 1, 9)])
+def test_orthogonal(cuda, n, flags, planes):
+    grid, x, z = _scanner(n, n, 10, 24, 20)
+    _compare(grid, x, z, 24, 20, 0, planes, projector_type=2, orth_width=2.4, orth_flags=flags,
+             norm=np.random.default_rng(1).random(24 * 20 * 10).astype(np.float32) + 0.5)
+
+
+@pytest.mark.parametrize("nx,ny,dl,atten", [(32, 32, 2.5, False), (21, 34, 1.7, True), (16, 16, -2.5, False)])
+@pytest.mark.parametrize("planes", [1, 4, 9])
+def test_interpolation(cuda, nx, ny, dl, atten, planes):
+    grid, x, z = _scanner(nx, ny, 10, 24, 20)
+    kw = dict(atten=np.full(grid.N, 0.004, np.float32), atten_mode=1) if atten else {}
+    _compare(grid, x, z, 24, 20, 0, planes, projector_type=4, interp=(dl, 0.0), beta=0.01, **kw)
