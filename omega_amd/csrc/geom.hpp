@@ -54,6 +54,7 @@ struct omg_geom {
     std::vector<float> z_host;
     // Branchless distance-driven projector: per-projection back-projection geometry (16 floats each).
     float* bdd_geom5 = nullptr;
+    float bdd_mag = 0.f;      // largest magnification of the image centre (sizes the backprojection's window)
     // Voxel-driven planar backprojection (vbp.hip): usable when every angle column is a parallel-beam set
     // of evenly spaced LORs with endpoints outside the image; per-angle parameters and q/w work buffers.
     bool vbp_ok = false;
