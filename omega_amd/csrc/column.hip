@@ -1,0 +1,930 @@
+// column.hip -- projections of 3-D (ring-pair) sinograms by image columns.
+//
+// Every plane of a sinogram repeats the same transaxial LORs: an oblique LOR crosses the x and y boundaries of the
+// image at the same parameters as its neighbours in the other planes, and between two of them it stays in one
+// column of voxels (fixed x, y), moving along z. So a wave takes one transaxial bin and 64 planes, one per lane:
+// the crossings of the bin (pixel, exit parameter) are traced once per handle and kept, and all lanes read them
+// through scalar loads; a lane keeps only its z walk, and the lanes' voxels lie within one column, which is
+// contiguous in a z-fastest image (Nz floats, a few cache lines) -- in the one-lane-per-LOR kernels every lane
+// gathers from, or adds to, a line of its own.
+//
+// Forward projection: z-fastest copy of the image, sums in the walk's order with its float operations
+// (bit-identical to the one-lane-per-LOR kernel). Backprojection: a workgroup owns a tile of columns and a share of
+// the segments (bin, entries inside the tile) of the lists, accumulates in LDS in 64-bit fixed point (as the
+// direct-plane kernels: float LDS atomics retire 15 times slower, and global float atomics at 21 G segments of 64
+// bytes per second however few lanes a segment serves), and adds the tile to the image once, in runs of
+// consecutive x.
+//
+// LORs whose set-up differs from their bin's (along an image axis in a direct plane, entering the image through an
+// end face, dropped or displaced by rounding) are listed and take the one-lane-per-LOR walk.
+#include "column.hpp"
+#include "geom.hpp"
+#include "siddon_device.hpp"
+
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+#include <vector>
+
+namespace omg {
+
+constexpr uint32_t kCL = 64;        // planes per wave
+
+struct ColStart { float tc, tx0, ty0; uint32_t xy; };   // where a bin's walk enters the image
+struct ColSeg { uint32_t bin, k0, k1; };                // entries [k0, k1) of the lists lie in one tile
+struct ColItem { uint32_t tile, s0, s1; };              // one workgroup's segments
+
+struct ColPlan {
+    int64_t first = 0, n = 0;
+    bool ok = false;
+    uint32_t bins = 0;
+    const uint32_t* bin_of = nullptr;   // measurement-level subsets: the range's first plane in the index table
+    uint32_t* off = nullptr;            // [bins + 1]
+    ColStart* start = nullptr;
+    uint2* ent = nullptr;               // {x | y << 16, exit parameter}
+    uint32_t tw = 0, th = 0, ntx = 0;   // tile width, height; tiles per row
+    ColSeg* seg = nullptr;
+    ColItem* item = nullptr;
+    uint32_t items = 0, max_segs = 0, tpb = 0;
+};
+
+struct ColView {
+    uint32_t bins, planes, tw, th, ntx, max_segs;
+    const uint32_t* off;
+    const ColStart* start;
+    const uint2* ent;
+    const ColSeg* seg;
+    const ColItem* item;
+};
+
+// ---- building ----------------------------------------------------------------------------------------
+__device__ __forceinline__ uint32_t col_tile(uint32_t xy, uint32_t tw, uint32_t th, uint32_t ntx) {
+    return (xy & 0xffffu) / tw + (xy >> 16) / th * ntx;
+}
+
+// The transaxial walk of bin j: visit(xy, exit parameter) for each pixel in order; false when the bin's LORs are
+// irregular in every plane or miss the image.
+template <typename Visit>
+__device__ __forceinline__ bool col_walk(const SidArgs& a, uint32_t j, ColStart& st, Visit&& visit) {
+    Ray r;
+    fetch_ray_base(a, j, r);
+    const float xdf = r.xd - r.xs, ydf = r.yd - r.ys;
+    st = ColStart{__builtin_nanf(""), 0.f, 0.f, 0u};
+    if (isinf(ydf) || isinf(xdf)) return false;
+    int32_t ti = 0, tj = 0, ux = 0, uy = 0;
+    float txu = 0.f, tyu = 0.f, tc = 0.f, tx0 = 1e8f, ty0 = 1e8f;
+    // a LOR along one image axis crosses that axis only (siddon_setup's branches for oblique planes)
+    auto along = [&](float b, float bmax, float d, float src, float dst, float diff, uint32_t N, int32_t& i, int32_t& u,
+                     float& t0, float& tu) {
+        t0 = (b - src) / diff;
+        const float tb = (bmax - src) / diff, tmin = mn(t0, tb), tmax = mx(t0, tb);
+        tc = tmin;
+        if (tc >= tmax) return false;
+        uint32_t vmin = 0, vmax = 0;
+        if (src < dst) axis_inc(tc, tmin, tmax, tmax, vmin, vmax, t0, u, diff, b, d, src, N);
+        else axis_dec(tc, tmin, tmax, tmax, vmin, vmax, t0, u, diff, b, d, src, N);
+        i = src < dst ? 0 : (int32_t)N - 1;
+        tu = d / fabsf(diff);
+        return true;
+    };
+    if (fabsf(ydf) < 1e-8f) {
+        tj = perp_start(a.by, r.yd, a.dy, a.Ny);
+        if (fabsf(xdf) < 1e-8f || r.yd > a.bmaxy || r.yd < a.by ||
+            !along(a.bx, a.bmaxx, a.dx, r.xs, r.xd, xdf, a.Nx, ti, ux, tx0, txu))
+            return false;
+    } else if (fabsf(xdf) < 1e-8f) {
+        ti = perp_start(a.bx, r.xd, a.dx, a.Nx);
+        if (r.xd > a.bmaxx || r.xd < a.bx ||
+            !along(a.by, a.bmaxy, a.dy, r.ys, r.yd, ydf, a.Ny, tj, uy, ty0, tyu))
+            return false;
+    } else {
+        uint32_t Np = 0;
+        if (preloop2(a.bx, a.by, xdf, ydf, a.bmaxx, a.bmaxy, a.dx, a.dy, a.Nx, a.Ny, ti, tj, txu, tyu, Np, r.ys, r.xs,
+                     r.yd, r.xd, tc, ux, uy, tx0, ty0))
+            return false;
+    }
+    st = ColStart{tc, tx0, ty0, (uint32_t)ti | (uint32_t)tj << 16};
+    while ((uint32_t)ti < a.Nx && (uint32_t)tj < a.Ny) {
+        const bool y = ty0 < tx0;
+        visit((uint32_t)ti | (uint32_t)tj << 16, y ? ty0 : tx0);
+        if (y) { tj += uy; ty0 += tyu; }
+        else { ti += ux; tx0 += txu; }
+    }
+    return true;
+}
+
+// One lane per bin. Counting pass (ent null): entries, and segments per tile. Filling pass: the lists, and the
+// segments in their tiles' ranges. The tiles' counters are shared by every bin, so a workgroup adds its own
+// counts (LDS, up to kTileLds tiles) once.
+constexpr uint32_t kTileLds = 2048;
+
+__global__ __launch_bounds__(256) void k_col_trace(SidArgs a, uint32_t bins, uint32_t tw, uint32_t th, uint32_t ntx,
+                                                   uint32_t tiles, uint32_t* __restrict__ cnt,
+                                                   uint32_t* __restrict__ tile_cnt, const uint32_t* __restrict__ off,
+                                                   ColStart* __restrict__ start, uint2* __restrict__ ent,
+                                                   const uint32_t* __restrict__ tile_off, ColSeg* __restrict__ seg) {
+    __shared__ uint32_t mine[kTileLds];
+    const uint32_t j = blockIdx.x * 256 + threadIdx.x;
+    const bool shared = tiles <= kTileLds;
+    for (uint32_t i = threadIdx.x; i < (shared ? tiles : 0u); i += 256) mine[i] = 0u;
+    __syncthreads();
+    ColStart st;
+    uint32_t n = 0, tile = 0xffffffffu;
+    if (j < bins && (shared || !ent)) {
+        col_walk(a, j, st, [&](uint32_t xy, float) {
+            const uint32_t t = col_tile(xy, tw, th, ntx);
+            if (t != tile) atomicAdd(shared ? mine + t : tile_cnt + t, 1u);
+            tile = t;
+            n++;
+        });
+        if (!ent) cnt[j] = n;
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < (shared ? tiles : 0u); i += 256)   // counts -> this workgroup's first slot
+        if (mine[i]) mine[i] = atomicAdd(tile_cnt + i, mine[i]);
+    if (!ent) return;
+    __syncthreads();
+    if (j >= bins) return;
+    const uint32_t o = off[j];
+    uint32_t k0 = o;
+    n = o;
+    tile = 0xffffffffu;
+    auto close = [&]() {
+        if (tile != 0xffffffffu)
+            seg[tile_off[tile] + atomicAdd(shared ? mine + tile : tile_cnt + tile, 1u)] = ColSeg{j, k0, n};
+    };
+    col_walk(a, j, st, [&](uint32_t xy, float tn) {
+        const uint32_t t = col_tile(xy, tw, th, ntx);
+        if (t != tile) {
+            close();
+            tile = t;
+            k0 = n;
+        }
+        ent[n++] = make_uint2(xy, __float_as_uint(tn));
+    });
+    close();
+    start[j] = st;
+}
+
+// *bad = 1 unless measurement i of the range is bin index[i % bins] of plane i / bins.
+__global__ __launch_bounds__(256) void k_col_check(const uint32_t* __restrict__ index, uint64_t n, uint32_t bins,
+                                                   uint32_t per, int32_t* __restrict__ bad) {
+    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t p = (uint32_t)(i / bins), c = index[i - (uint64_t)p * bins];
+    if (c >= per || index[i] != c + p * per) *bad = 1;
+}
+
+__global__ void k_col_zero(uint32_t* p, uint32_t n) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) p[i] = 0u;
+}
+
+// ---- running -----------------------------------------------------------------------------------------
+// dst[x + y Nx][z + lead] = src[x + y Nx + z Nx Ny], columns of `pitch` with zeros around the image's Nz; clears
+// the launch's state. grid = (ceil(Nx / 32), Ny, ceil(pitch / 32)), block = (32, 8).
+__global__ __launch_bounds__(256) void k_col_zfast(const float* __restrict__ src, float* __restrict__ dst, uint32_t Nx,
+                                                   uint32_t Ny, uint32_t Nz, uint32_t pitch, uint32_t lead,
+                                                   uint32_t* __restrict__ state) {
+    __shared__ float t[32][33];
+    const uint32_t x0 = blockIdx.x * 32, z0 = blockIdx.z * 32, y = blockIdx.y;
+    if (blockIdx.x + blockIdx.y + blockIdx.z == 0 && threadIdx.y == 0 && threadIdx.x < 4) state[threadIdx.x] = 0u;
+    for (uint32_t k = threadIdx.y; k < 32; k += 8) {
+        const uint32_t x = x0 + threadIdx.x, z = z0 + k - lead;
+        t[k][threadIdx.x] = x < Nx && z < Nz ? src[x + ((size_t)z * Ny + y) * Nx] : 0.f;
+    }
+    __syncthreads();
+    for (uint32_t k = threadIdx.y; k < 32; k += 8) {
+        const uint32_t x = x0 + k, z = z0 + threadIdx.x;
+        if (x < Nx && z < pitch) dst[(x + (size_t)y * Nx) * pitch + z] = t[threadIdx.x][k];
+    }
+}
+
+// The set-up of a LOR is its bin's: the bin's crossings are its own.
+__device__ __forceinline__ bool col_regular(const Walk& w, const ColStart& st) {
+    return !w.perp && w.tc == st.tc && w.tx0 == st.tx0 && w.ty0 == st.ty0 &&
+           ((uint32_t)w.ti | (uint32_t)w.tj << 16) == st.xy;
+}
+
+// More than one z crossing per column is possible only if they lie closer together than a column's faces.
+__device__ __forceinline__ bool col_steep(const Walk& w) {
+    const float t = w.txu == 0.f ? w.tyu : w.tyu == 0.f ? w.txu : fminf(w.txu, w.tyu);
+    return w.uz != 0 && w.tzu < 1.001f * t;
+}
+
+// A lane's z walk within the columns its wave passes. tk counts from `lead`; columns carry cells of no consequence in
+// front of the image and behind it. `left` counts the steps that the LOR's walk may still take (0: it has ended). A
+// lane that leaves the image stays in the end cell with tz0 = kColEnd; one that runs out of steps keeps tk and Lf = 0:
+// their terms vanish without a test. `tc` is the same for every lane after each column (its exit), so it lives outside.
+constexpr float kColEnd = 3e38f;
+struct ColLane {
+    float tz0, tzu, Lf;
+    int32_t tk, uz, left;
+};
+
+__device__ __forceinline__ void col_end(ColLane& l) {
+    l.left = 0;
+    l.Lf = 0.f;
+    l.tz0 = kColEnd;
+}
+
+// One column as the walk defines it: z crossings while they come first, then the exit. visit(parameter step, tk).
+template <typename Visit>
+__device__ __forceinline__ void col_step(ColLane& l, float tc, float tn, uint32_t Nz, uint32_t lead, Visit&& visit) {
+    float t = tc;
+    bool cross = l.left > 0 && l.tz0 < tn;
+    while (__any(cross)) {
+        if (cross) {
+            visit(l.tz0 - t, l.tk);
+            t = l.tz0;
+            l.tz0 += l.tzu;
+            l.tk += l.uz;
+            l.left--;
+            if ((uint32_t)l.tk - lead >= Nz || l.left == 0) col_end(l);
+        }
+        cross = l.left > 0 && l.tz0 < tn;
+    }
+    if (l.left > 0) {
+        visit(tn - t, l.tk);
+        if (--l.left == 0) col_end(l);
+    }
+}
+
+// True when no lane can run out of steps in the next four columns (two per column, see `steep`).
+__device__ __forceinline__ bool col_free(const ColLane& l) { return !__any(l.left > 0 && l.left <= 8); }
+
+// Four entries of a list from k on by one scalar load (the lists never change); the allocation ends four later.
+__device__ __forceinline__ void col_four(const uint2* ent, uint32_t k, uint2 (&e)[4]) {
+    const auto* p = (const __attribute__((address_space(4))) uint32_t*)(uintptr_t)(ent + k);
+#pragma unroll
+    for (int j = 0; j < 4; j++) e[j] = make_uint2(p[2 * j], p[2 * j + 1]);
+}
+
+// One column of a lane that crosses at most one z plane in it: the pieces before and behind the crossing, piece(length,
+// tk) and other(length, tk, crossed); an absent one has length 0. CHECK: the lane may run out of steps here.
+template <bool CHECK, typename Piece, typename Other>
+__device__ __forceinline__ void col_pair(ColLane& l, float tc, float tn, uint32_t Nz, uint32_t lead, Piece&& piece,
+                                         Other&& other) {
+    const bool cross = l.tz0 < tn;
+    piece(fmaxf((cross ? l.tz0 : tn) - tc, 0.f) * l.Lf, l.tk);
+    l.tk += cross ? l.uz : 0;
+    if (CHECK) {
+        l.left -= cross ? 1 : 0;
+        l.Lf = cross && l.left <= 0 ? 0.f : l.Lf;
+    }
+    other(fmaxf(tn - l.tz0, 0.f) * l.Lf, l.tk, cross);
+    l.tz0 = cross ? l.tz0 + l.tzu : l.tz0;
+    l.tz0 = (uint32_t)l.tk - lead < Nz ? l.tz0 : kColEnd;
+    if (CHECK && --l.left <= 0) {
+        l.left = 0;
+        l.Lf = 0.f;
+        l.tz0 = kColEnd;
+    }
+}
+
+// a * b, and 0 where a factor is 0 whatever the other one is
+__device__ __forceinline__ float mul_or_zero(float a, float b) {
+    float r;
+    asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+enum { COL_FP = 0, COL_OSEM = 1, COL_BP = 2 };
+
+// One wave per bin and 64 planes, BPW bins one after the other. COL_FP: y = A img. COL_BP: the lanes' records for
+// k_col_bp, {z walk, length, y * weight (weight alone when y is null)}, and with wrec the weights beside them.
+// COL_OSEM: forward projection, ratio, records. state: {largest |value| of the records as float bits, irregular LORs
+// listed in `rest`, largest weight}. Measurements pass through LDS (a wave's lanes are a whole plane apart in
+// them). A column of up to 64 NR - 1 slices is loaded into the wave's registers, lane z holding slice z, and every
+// lane picks its slices by ds_bpermute; NR 0: lanes gather from memory. What bounds the forward projection: VALU,
+// about 22 operations per column and 64 LORs besides 690 per LOR's set-up. 64 planes of 224 x 224 bins, 128 x 128 x 63:
+// 217 us; 383 us with gathers (16 clocks of the texture address unit each, two per column) and 484 us by one lane per
+// LOR.
+template <int MODE, int BPW, int NR>
+__global__ __launch_bounds__(256, MODE == COL_FP && NR < 2 ? 6 : 4) void k_col_fp(
+    ColView c, SidArgs a, uint32_t plane0, const float* __restrict__ Xz, const float* __restrict__ yin,
+    float* __restrict__ yout, float4* __restrict__ rec, float* __restrict__ wrec, uint32_t* __restrict__ state,
+    uint32_t* __restrict__ rest, float epps) {
+    constexpr uint32_t NB = 4 * BPW;
+    __shared__ float ys[kCL][NB + 1];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const uint32_t bin0 = blockIdx.x * NB, pg = plane0 + blockIdx.y * kCL;
+    if (MODE != COL_FP && yin) {
+        for (uint32_t t = threadIdx.x; t < kCL * NB; t += 256) {
+            const uint32_t b = t % NB, q = t / NB;
+            ys[q][b] = bin0 + b < c.bins && pg + q < c.planes ? yin[(int64_t)(pg + q) * c.bins + bin0 + b] : 0.f;
+        }
+        __syncthreads();
+    }
+    const uint32_t p = pg + lane;
+    const bool in = p < c.planes;
+    constexpr uint32_t lead = NR ? 0u : 1u;
+    const uint32_t zp = NR ? 64u * NR : a.Nz + 2;
+    const __amdgpu_buffer_rsrc_t cols = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(Xz), 0, NR ? (int)(a.Nx * a.Ny * 256u * NR) : 0, 0x00027000);
+    uint32_t top = 0, topw = 0;
+    for (uint32_t i = 0; i < BPW; i++) {
+        const uint32_t b = wave * BPW + i, bin = bin0 + b;
+        if (bin >= c.bins) break;
+        const int64_t lo = (int64_t)p * c.bins + bin;
+        const ColStart st = c.start[bin];
+        Walk w;
+        float weight = 0.f, yhat = 0.f;
+        const bool hit = in && siddon_setup<false>(a, lo, w, weight);
+        const bool reg = hit && col_regular(w, st);
+        {   // irregular LORs: a list for k_col_rest
+            const uint64_t m = __ballot(hit && !reg);
+            if (m) {
+                uint32_t o = 0;
+                if (lane == 0) o = atomicAdd(state + 1, (uint32_t)__popcll(m));
+                o = __builtin_amdgcn_readfirstlane(o);
+                if (hit && !reg) rest[o + __popcll(m & ((1ull << lane) - 1))] = (uint32_t)lo;
+            }
+        }
+        if (MODE != COL_BP) {
+            float ax = 0.f;
+            if (__any(reg)) {
+                ColLane l{w.tz0, w.tzu, w.L, w.tk + (int32_t)lead, w.uz, (int32_t)w.left};
+                if (!reg) {
+                    l.tk = 0;
+                    l.uz = 0;
+                    col_end(l);
+                }
+                const bool steep = __any(reg && col_steep(w));
+                float tc = st.tc;
+                const uint32_t e1 = __builtin_amdgcn_readfirstlane(c.off[bin + 1]);
+                uint32_t k = __builtin_amdgcn_readfirstlane(c.off[bin]);
+                while (k < e1) {
+                    if (!steep) {
+                        // straight line, four columns at a time, the next four loading meanwhile; behind the list's
+                        // end its last column again, where no length is left
+                        uint2 e[4], en[4];
+                        float r0[4], r1[4], n0[4], n1[4];
+                        auto load = [&](uint32_t kk, uint2 (&ee)[4], float* q0, float* q1) {
+                            col_four(c.ent, kk, ee);
+#pragma unroll
+                            for (int j = 1; j < 4; j++) ee[j] = kk + j < e1 ? ee[j] : ee[j - 1];
+#pragma unroll
+                            for (int j = 0; j < 4 && NR; j++) {
+                                const int32_t o =
+                                    (int32_t)(((ee[j].x & 0xffffu) + (ee[j].x >> 16) * a.Nx) * (256u * NR));
+                                auto slice = [&](uint32_t z) {
+                                    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(cols, 4 * z, o, 0));
+                                };
+                                q0[j] = slice(lane);
+                                if (NR > 1) q1[j] = slice(64 + lane);
+                            }
+                        };
+                        auto batch = [&](auto check) {
+                            float l1[4], l2[4], v1[4], v2[4];
+                            const int32_t tk0 = l.tk;
+#pragma unroll
+                            for (int j = 0; j < 4; j++) {
+                                const float tn = __uint_as_float(e[j].y);
+                                const char* col = reinterpret_cast<const char*>(
+                                    Xz + (size_t)((e[j].x & 0xffffu) + (e[j].x >> 16) * a.Nx) * zp);
+                                auto voxel = [&](int32_t tk) {
+                                    if (!NR) return *reinterpret_cast<const float*>(col + 4u * (uint32_t)tk);
+                                    auto pick = [&](float q) {
+                                        return __int_as_float(__builtin_amdgcn_ds_bpermute(4 * tk, __float_as_int(q)));
+                                    };
+                                    if (NR < 2) return pick(r0[j]);
+                                    const float q0 = pick(r0[j]), q1 = pick(r1[j]);
+                                    return (tk & 64) ? q1 : q0;
+                                };
+                                col_pair<decltype(check)::value>(
+                                    l, tc, tn, a.Nz, lead,
+                                    [&](float len, int32_t tk) { l1[j] = len; v1[j] = voxel(tk); },
+                                    [&](float len, int32_t tk, bool) { l2[j] = len; v2[j] = voxel(tk); });
+                                tc = tn;
+                            }
+                            // steps taken; a lane that has ended stays at 0
+                            if (!decltype(check)::value) l.left = max(l.left - 4 - abs(l.tk - tk0), 0);
+                            if ((uint32_t)l.tk - lead >= a.Nz) col_end(l);
+#pragma unroll
+                            for (int j = 0; j < 4; j++) {   // 0 times anything is 0 here: no term for an empty piece
+                                ax += mul_or_zero(l1[j], v1[j]);
+                                ax += mul_or_zero(l2[j], v2[j]);
+                            }
+                        };
+                        load(k, e, r0, r1);
+                        for (; k < e1; k += 4) {
+                            load(k + 4 < e1 ? k + 4 : k, en, n0, n1);
+                            __builtin_amdgcn_sched_barrier(0);
+                            if (col_free(l)) batch(std::false_type());
+                            else batch(std::true_type());
+#pragma unroll
+                            for (int j = 0; j < 4; j++) {
+                                e[j] = en[j];
+                                r0[j] = n0[j];
+                                r1[j] = n1[j];
+                            }
+                        }
+#pragma unroll
+                        for (int j = 0; j < 4 && NR; j++) {   // a use on the way out keeps the loads ahead of the sums
+                            asm volatile("" ::"v"(r0[j]));
+                            if (NR > 1) asm volatile("" ::"v"(r1[j]));
+                        }
+                    } else {
+                        const uint32_t ke = min(k + 4, e1);
+                        for (; k < ke; k++) {
+                            const uint2 e = c.ent[k];
+                            const float tn = __uint_as_float(e.y);
+                            const float* col = Xz + (size_t)((e.x & 0xffffu) + (e.x >> 16) * a.Nx) * zp;
+                            col_step(l, tc, tn, a.Nz, lead, [&](float dt, int32_t tk) {
+                                const float len = dt * l.Lf;
+                                if (len > 0.f) ax += len * col[tk];
+                            });
+                            tc = tn;
+                        }
+                    }
+                }
+            }
+            yhat = hit ? ax * weight : 0.f;
+            if (MODE == COL_FP) {
+                ys[lane][b] = yhat;
+                continue;
+            }
+        }
+        float v = 1.f;
+        if (MODE == COL_OSEM) {
+            v = 0.f;
+            if (hit) {
+                v = ys[lane][b] / ratio_den(a, lo, yhat, epps);
+                if (isnan(v) || isinf(v)) v = epps;
+            }
+        } else if (yin) {
+            v = ys[lane][b];
+        }
+        const float keep = reg ? v * weight : 0.f;
+        // bit 15 of tk: more than one z crossing per column is possible
+        const uint32_t steep = reg && col_steep(w) ? 0x8000u : 0u;
+        rec[((size_t)blockIdx.y * c.bins + bin) * kCL + lane] =
+            make_float4(w.tz0, w.L, keep, __uint_as_float((uint32_t)(w.tk + 1) | steep | w.left << 16));
+        top = max(top, __float_as_uint(keep) & 0x7fffffffu);   // NaN and Inf order above every number
+        if (wrec) {
+            const float kw = reg ? weight : 0.f;
+            wrec[((size_t)blockIdx.y * c.bins + bin) * kCL + lane] = kw;
+            topw = max(topw, __float_as_uint(kw) & 0x7fffffffu);
+        }
+    }
+    if (MODE == COL_FP) {
+        __syncthreads();
+        for (uint32_t t = threadIdx.x; t < kCL * NB; t += 256) {
+            const uint32_t b = t % NB, q = t / NB;
+            if (bin0 + b < c.bins && pg + q < c.planes) yout[(int64_t)(pg + q) * c.bins + bin0 + b] = ys[q][b];
+        }
+        return;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        top = max(top, (uint32_t)__shfl_xor((int)top, o, 64));
+        topw = max(topw, (uint32_t)__shfl_xor((int)topw, o, 64));
+    }
+    auto raise = [&](uint32_t* at, uint32_t v) {
+        if (lane == 0 && v > __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(at, v);
+    };
+    raise(state, top);
+    if (wrec) raise(state + 2, topw);
+}
+
+// The irregular LORs of a k_col_fp launch, one per lane, by the walk of the one-lane-per-LOR kernels: thread `i` of
+// `step`.
+struct ColRest {
+    const uint32_t* list;
+    const float* img;        // image (x fastest); null: backprojection of yin alone
+    const float* yin;
+    float* yout;             // forward projection
+    float *rhs, *sens;
+    float epps;
+};
+
+__device__ __forceinline__ void col_rest(const SidArgs& a, const ColRest& r, uint32_t n, uint32_t i, uint32_t step) {
+    for (; i < n; i += step) {
+        const int64_t lo = r.list[i];
+        float v = !r.img && r.yin ? r.yin[lo] : 1.f, weight = 0.f;
+        if (r.img) {
+            float ax = 0.f;
+            const bool hit = siddon_gather<false>(a, lo, r.img, ax, weight);
+            const float yhat = hit ? ax * weight : 0.f;
+            if (r.yout) {
+                r.yout[lo] = yhat;
+                continue;
+            }
+            v = r.yin[lo] / ratio_den(a, lo, yhat, r.epps);
+            if (isnan(v) || isinf(v)) v = r.epps;
+        }
+        if (v == 0.f && !r.sens) continue;
+        siddon_trace(a, lo, weight, [&](uint32_t ind, float len) {
+            const float lw = len * weight;
+            unsafeAtomicAdd(r.rhs + ind, v * lw);
+            if (r.sens) unsafeAtomicAdd(r.sens + ind, lw);
+        });
+    }
+}
+
+__global__ __launch_bounds__(64) void k_col_rest(SidArgs a, const uint32_t* __restrict__ state, ColRest r) {
+    col_rest(a, r, state[1], blockIdx.x * 64 + threadIdx.x, gridDim.x * 64);
+}
+
+// Backprojection. Blocks [0, rest_blocks) of x take the irregular LORs (first, as theirs are the longest chains);
+// every other block one item: LDS accumulators [tile pixel][Nz + 2], int64 fixed point; the end cells are dropped.
+// blockIdx.z 1: the weights into sens instead of the records' values into rhs. What bounds it: the LDS atomics (64
+// lanes over one column's cells) and about 35 VALU operations per column and 64 LORs. 64 planes of 224 x 224 bins,
+// 128 x 128 x 63: 281 us, with the records' launch 355 us; 5690 us by one lane per LOR (global float atomics).
+__global__ __launch_bounds__(1024, 8) void k_col_bp(ColView c, SidArgs a, uint32_t plane0, uint32_t rest_blocks,
+                                                    ColRest rest, const float4* __restrict__ rec,
+                                                    const float* __restrict__ wrec,
+                                                    const uint32_t* __restrict__ state) {
+    extern __shared__ unsigned long long acc64[];
+    if (blockIdx.x < rest_blocks) {
+        if (blockIdx.y + blockIdx.z == 0)
+            col_rest(a, rest, state[1], blockIdx.x * blockDim.x + threadIdx.x, rest_blocks * blockDim.x);
+        return;
+    }
+    const bool sens = blockIdx.z != 0;
+    float* __restrict__ rhs = sens ? rest.sens : rest.rhs;
+    const ColItem it = c.item[blockIdx.x - rest_blocks];
+    const uint32_t x0 = it.tile % c.ntx * c.tw, y0 = it.tile / c.ntx * c.th;
+    const uint32_t zp = a.Nz + 2, cells = c.tw * c.th * zp;
+    for (uint32_t i = threadIdx.x; i < cells; i += blockDim.x) acc64[i] = 0ull;
+    const uint32_t pk = state[sens ? 2 : 0];
+    bool finite = pk < 0x7f800000u;
+    // |term| <= peak * voxel diagonal; a segment adds at most two terms to a voxel per lane, and an item holds at
+    // most max_segs segments of 64 lanes
+    double up, down;
+    {
+        const float diag = sqrtf(a.dx * a.dx + a.dy * a.dy + a.dz * a.dz) * (1.f + 0x1p-10f);
+        const float bt = finite ? __uint_as_float(pk) * diag : 1.f;
+        const float bs = bt * (2.f * kCL * (float)c.max_segs);
+        finite = finite && bs < __builtin_inff();
+        fixed_scale(bt, bs, up, down);
+    }
+    __syncthreads();
+    const uint32_t lane = threadIdx.x & 63, p = plane0 + blockIdx.y * kCL + lane;
+    ColLane l;
+    float tzi = 0.f;
+    l.tzu = 0.f;
+    l.uz = 0;
+    if (p < c.planes) {
+        const float2 zz = *reinterpret_cast<const float2*>(a.z + (a.plane_col + p) * 2);
+        l.tzu = a.dz / fabsf(zz.y - zz.x);
+        tzi = fabsf(zz.y - zz.x) / a.dz;
+        l.uz = zz.x < zz.y ? 1 : -1;
+    }
+    const int32_t uz = l.uz;
+    const uint32_t waves = blockDim.x >> 6;
+    uint32_t s = it.s0 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const size_t group = (size_t)blockIdx.y * c.bins * kCL + lane;
+    auto fetch = [&](uint32_t q) {
+        const size_t o = group + (size_t)c.seg[q].bin * kCL;
+        float4 r = rec[o];
+        if (sens) r.z = wrec[o];
+        return r;
+    };
+    float4 nx = s < it.s1 ? fetch(s) : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (; s < it.s1; s += waves) {
+        const ColSeg sg = c.seg[s];
+        const float4 r = nx;
+        if (s + waves < it.s1) nx = fetch(s + waves);   // in flight during this segment
+        const uint32_t o = c.off[sg.bin];
+        const uint32_t bits = __float_as_uint(r.w);
+        const float Lw = r.y * r.z;                       // length * record value; a term is a parameter step times it
+        float tc = sg.k0 > o ? __uint_as_float(c.ent[sg.k0 - 1].y) : c.start[sg.bin].tc;
+        l.tz0 = r.x;
+        l.uz = uz;
+        l.Lf = Lw;
+        l.tk = (int32_t)(bits & 0x7fffu);
+        l.left = (int32_t)(bits >> 16);
+        if (r.z == 0.f) {
+            l.tk = 0;
+            l.uz = 0;
+            col_end(l);
+        }
+        if (!__any(l.left > 0)) continue;
+        const bool steep = __any(l.left > 0 && (bits & 0x8000u));
+        if (l.tz0 < tc) {             // the z crossings before the tile
+            const float n = fminf(floorf((tc - l.tz0) * tzi) + 1.f, (float)l.left);
+            l.tz0 = __builtin_fmaf(n, l.tzu, l.tz0);
+            l.tk += l.uz * (int32_t)n;
+            l.left -= (int32_t)n;
+            if ((uint32_t)(l.tk - 1) >= a.Nz) col_end(l);
+        }
+        l.left -= (int32_t)(sg.k0 - o);
+        if (l.left <= 0) col_end(l);
+        if (l.left > 0) {
+            for (uint32_t k = sg.k0; k < sg.k1; k += 4) {
+                if (finite && !steep) {
+                    uint2 e[4];
+                    col_four(c.ent, k, e);
+                    auto batch = [&](auto check) {
+                        const int32_t tk0 = l.tk;
+#pragma unroll
+                        for (uint32_t j = 0; j < 4; j++) {
+                            if (j && k + j >= sg.k1) break;
+                            const float tn = __uint_as_float(e[j].y);
+                            unsigned long long* col =
+                                acc64 + (((e[j].x >> 16) - y0) * c.tw + ((e[j].x & 0xffffu) - x0)) * zp;
+                            col_pair<decltype(check)::value>(
+                                l, tc, tn, a.Nz, 1u, [&](float len, int32_t tk) { lds_add_fixed(col + tk, len, up); },
+                                [&](float len, int32_t tk, bool cross) {
+                                    if (cross) lds_add_fixed(col + tk, len, up);
+                                });
+                            tc = tn;
+                        }
+                        if (!decltype(check)::value) l.left = max(l.left - 4 - abs(l.tk - tk0), 0);
+                        if ((uint32_t)(l.tk - 1) >= a.Nz) col_end(l);
+                    };
+                    if (col_free(l)) batch(std::false_type());
+                    else batch(std::true_type());
+                } else {
+                    for (uint32_t j = k; j < min(k + 4, sg.k1); j++) {
+                        const uint2 e = c.ent[j];
+                        const float tn = __uint_as_float(e.y);
+                        const uint32_t ex = e.x & 0xffffu, ey = e.x >> 16;
+                        unsigned long long* col = acc64 + ((ey - y0) * c.tw + (ex - x0)) * zp;
+                        col_step(l, tc, tn, a.Nz, 1u, [&](float dt, int32_t tk) {
+                            if (!(dt > 0.f)) return;
+                            if (finite) lds_add_fixed(col + tk, dt * l.Lf, up);
+                            else unsafeAtomicAdd(rhs + ex + (size_t)(ey + (size_t)(tk - 1) * a.Ny) * a.Nx, dt * l.Lf);
+                        });
+                        tc = tn;
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();
+    if (!finite) return;
+    // x fastest, so a wave's adds fall on runs of tw consecutive voxels
+    for (uint32_t i = threadIdx.x; i < c.tw * c.th * a.Nz; i += blockDim.x) {
+        const uint32_t lx = i % c.tw, q = i / c.tw, ly = q % c.th, z = q / c.th;
+        const unsigned long long v = acc64[(ly * c.tw + lx) * zp + z + 1];
+        if (v != 0ull) unsafeAtomicAdd(rhs + x0 + lx + (size_t)(y0 + ly + (size_t)z * a.Ny) * a.Nx, fixed_value(v, down));
+    }
+}
+
+// ---- host ----------------------------------------------------------------------------------------------
+struct ColCache { std::vector<ColPlan*> e; };
+
+static void col_free(ColPlan* p) {
+    hipFree(p->off); hipFree(p->start); hipFree(p->ent); hipFree(p->seg); hipFree(p->item);
+    p->off = nullptr; p->start = nullptr; p->ent = nullptr; p->seg = nullptr; p->item = nullptr;
+}
+
+template <typename T>
+static bool col_alloc(T** p, uint64_t n) {
+    return hipMalloc(reinterpret_cast<void**>(p), (size_t)std::max<uint64_t>(n, 1) * sizeof(T)) == hipSuccess;
+}
+
+constexpr size_t kColLds = 76 * 1024;   // two workgroups of 16 waves per CU (one of 152 KB: 376 us, four of 38 KB: 310 us)
+constexpr size_t kColPlans = 64;        // subsets of an index table that keep their lists
+constexpr uint32_t kColRest = 32;       // workgroups of k_col_bp for the irregular LORs
+
+// Columns per tile whose int64 accumulators fit LDS: 16 x 16 (64-byte runs of x) down to 1 x 1; 0: none.
+static bool col_tile_size(uint32_t Nz, uint32_t* tw, uint32_t* th) {
+    const size_t m = kColLds / (8 * ((size_t)Nz + 2));
+    uint32_t w = 16, h = 16;
+    while ((size_t)w * h > m && (w > 1 || h > 1)) {
+        if (h >= w) h /= 2;
+        else w /= 2;
+    }
+    *tw = w;
+    *th = h;
+    return (size_t)w * h <= m;
+}
+
+static size_t col_lds(uint32_t tw, uint32_t th, uint32_t Nz) { return (size_t)tw * th * (Nz + 2) * 8; }
+
+// Lanes per workgroup of k_col_bp: a tile's LDS decides how many share a CU, 32 waves on it either way.
+static uint32_t col_tpb(uint32_t tw, uint32_t th, uint32_t Nz) {
+    const size_t lds = col_lds(tw, th, Nz);
+    return lds > 38 * 1024 ? 1024 : lds > 19 * 1024 ? 512 : 256;
+}
+
+static bool col_build(const omg_geom* g, ColPlan* p, hipStream_t s) {
+    const omg_geom_desc& d = g->d;
+    const uint32_t per = d.size_x * d.size_y;
+    if (!col_tile_size(d.Nz, &p->tw, &p->th) ||
+        hipFuncSetAttribute(reinterpret_cast<const void*>(k_col_bp), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)kColLds) != hipSuccess)
+        return false;
+    p->ntx = (d.Nx + p->tw - 1) / p->tw;
+    const uint32_t tiles = p->ntx * ((d.Ny + p->th - 1) / p->th);
+    uint32_t *cnt = nullptr, *tile_cnt = nullptr, *tile_off = nullptr;
+    bool ok = true;
+    if (g->index_dev) {      // the range has to be the same bins of every plane
+        p->bins = d.n_proj && p->n % d.n_proj == 0 ? (uint32_t)(p->n / d.n_proj) : 0u;
+        if (p->bins == 0 || p->bins > per) return false;
+        p->bin_of = g->index_dev + p->first;
+        int32_t bad = 0;
+        ok = col_alloc(&cnt, 1);
+        if (ok) {
+            hipLaunchKernelGGL(k_col_zero, dim3(1), dim3(256), 0, s, cnt, 1u);
+            hipLaunchKernelGGL(k_col_check, dim3(grid_for(p->n, 256)), dim3(256), 0, s, p->bin_of, (uint64_t)p->n, p->bins,
+                               per, reinterpret_cast<int32_t*>(cnt));
+            ok = hipMemcpyAsync(&bad, cnt, 4, hipMemcpyDeviceToHost, s) == hipSuccess &&
+                 hipStreamSynchronize(s) == hipSuccess && !bad;
+        }
+        hipFree(cnt);
+        cnt = nullptr;
+        if (!ok) return false;
+    } else {
+        p->bins = per;
+    }
+    SidArgs a = make_sid_args(g, g->index_dev ? p->first : 0, p->bins);
+    const dim3 grid(grid_for(p->bins, 256)), block(256);
+    std::vector<uint32_t> hc(p->bins), ht(tiles), off((size_t)p->bins + 1), toff(tiles);
+    ok = col_alloc(&cnt, p->bins) && col_alloc(&tile_cnt, tiles);
+    if (ok) {
+        hipLaunchKernelGGL(k_col_zero, dim3(grid_for(tiles, 256)), dim3(256), 0, s, tile_cnt, tiles);
+        hipLaunchKernelGGL(k_col_trace, grid, block, 0, s, a, p->bins, p->tw, p->th, p->ntx, tiles, cnt, tile_cnt, nullptr,
+                           nullptr, nullptr, nullptr, nullptr);
+        ok = hipMemcpyAsync(hc.data(), cnt, p->bins * 4ull, hipMemcpyDeviceToHost, s) == hipSuccess &&
+             hipMemcpyAsync(ht.data(), tile_cnt, tiles * 4ull, hipMemcpyDeviceToHost, s) == hipSuccess &&
+             hipStreamSynchronize(s) == hipSuccess;
+    }
+    uint64_t total = 0, segs = 0;
+    for (uint32_t j = 0; j < p->bins && ok; j++) {
+        off[j] = (uint32_t)total;
+        total += hc[j];
+        if (total >= 0xFFFFFFF0ull) ok = false;
+    }
+    off[p->bins] = (uint32_t)total;
+    for (uint32_t t = 0; t < tiles; t++) {
+        toff[t] = (uint32_t)segs;
+        segs += ht[t];
+    }
+    ok = ok && total * 8 + segs * 12 <= (2ull << 30);
+    // equal shares of the segments: one per wave at least (an item clears and adds its whole tile)
+    std::vector<ColItem> items;
+    p->tpb = col_tpb(p->tw, p->th, d.Nz);
+    while (p->tpb > 256 && segs < 8 * 4096) p->tpb /= 2;    // few segments: more, smaller workgroups
+    const uint64_t slots = 256 * (2048 / p->tpb);
+    // four rounds of workgroups even out (294 us with two, 345 us with one)
+    uint64_t share = std::max<uint64_t>(p->tpb / 64, (segs + 4 * slots - 1) / (4 * slots));
+    for (uint64_t parts = ~0ull; share < segs && parts > 4 * slots - kColRest; share += (share + 63) / 64) {
+        parts = 0;
+        for (uint32_t t = 0; t < tiles; t++) parts += (ht[t] + share - 1) / share;
+    }
+    for (uint32_t t = 0; t < tiles; t++) {
+        const uint32_t parts = (uint32_t)((ht[t] + share - 1) / share);
+        for (uint32_t q = 0; q < parts; q++) {
+            const uint32_t s0 = (uint32_t)((uint64_t)ht[t] * q / parts), s1 = (uint32_t)((uint64_t)ht[t] * (q + 1) / parts);
+            items.push_back(ColItem{t, toff[t] + s0, toff[t] + s1});
+            p->max_segs = std::max(p->max_segs, s1 - s0);
+        }
+    }
+    p->items = (uint32_t)items.size();
+    ok = ok && p->items > 0 && col_alloc(&p->off, off.size()) && col_alloc(&p->start, p->bins) &&
+         col_alloc(&p->ent, total + 4) &&
+         col_alloc(&p->seg, segs) && col_alloc(&p->item, items.size()) && col_alloc(&tile_off, tiles) &&
+         hipMemcpy(p->off, off.data(), off.size() * 4, hipMemcpyHostToDevice) == hipSuccess &&
+         hipMemcpy(tile_off, toff.data(), tiles * 4ull, hipMemcpyHostToDevice) == hipSuccess &&
+         hipMemcpy(p->item, items.data(), items.size() * sizeof(ColItem), hipMemcpyHostToDevice) == hipSuccess;
+    if (ok) {
+        hipLaunchKernelGGL(k_col_zero, dim3(grid_for(tiles, 256)), dim3(256), 0, s, tile_cnt, tiles);
+        hipLaunchKernelGGL(k_col_trace, grid, block, 0, s, a, p->bins, p->tw, p->th, p->ntx, tiles, cnt, tile_cnt, p->off,
+                           p->start, p->ent, tile_off, p->seg);
+        ok = hipGetLastError() == hipSuccess && hipStreamSynchronize(s) == hipSuccess;
+    }
+    hipFree(cnt); hipFree(tile_cnt); hipFree(tile_off);
+    if (!ok) {
+        (void)hipGetLastError();
+        col_free(p);
+    }
+    return ok;
+}
+
+const ColPlan* col_plan(const omg_geom* gc, int64_t first, int64_t n, hipStream_t s) {
+    omg_geom* g = const_cast<omg_geom*>(gc);
+    const omg_geom_desc& d = g->d;
+    // fewer planes than half a wave leave most lanes idle; without the ring property a walk's lengths need the
+    // general expression; the records hold z in 15 bits and the steps left in 16
+    if (d.mode != OMG_MODE_PET_SINO || d.projector_type != OMG_PROJ_SIDDON || d.tof_bins > 1 || g->force_generic ||
+        d.reserved[3] != 0 || d.reserved[4] < 0 || !g->ring || d.n_proj < 32 ||
+        (uint64_t)d.Nx + d.Ny + d.Nz + 3 > 65535 || d.Nz > 32000 || n > 0xffffffffll ||
+        (uint64_t)std::max(d.rays_xy, 1u) * std::max(d.rays_z, 1u) != 1)
+        return nullptr;
+    const uint64_t per = (uint64_t)d.size_x * d.size_y;
+    if (!g->index_dev && ((uint64_t)n < 32 * per || (uint64_t)n % per)) return nullptr;
+    if (!g->columns) {
+        if (fixed_region_active()) return nullptr;
+        g->columns = new ColCache();
+    }
+    for (ColPlan* p : g->columns->e)
+        if (!g->index_dev || (p->first == first && p->n == n)) return p->ok ? p : nullptr;
+    if (fixed_region_active() || g->columns->e.size() >= kColPlans) return nullptr;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return nullptr;
+    ColPlan* p = new ColPlan();
+    p->first = first;
+    p->n = n;
+    g->columns->e.push_back(p);
+    p->ok = col_build(g, p, s);
+    return p->ok ? p : nullptr;
+}
+
+void col_release(omg_geom* g) {
+    if (!g->columns) return;
+    for (ColPlan* p : g->columns->e) {
+        col_free(p);
+        delete p;
+    }
+    delete g->columns;
+    g->columns = nullptr;
+}
+
+// Work memory: [z-fastest image: Nx Ny pitch][records: 4 floats x bins x 64 x plane groups per pass][weights, with
+// sens][irregular LORs][state: 4].
+constexpr uint64_t kColRecords = 8ull << 20;      // records per pass (128 MB): plane groups beyond take more passes
+
+// Bins per wave: one where the wave walks (a lane's chain of columns is long, so the last waves would leave the chip
+// idle: 218 us for the forward projection against 299 us with four), four for the records alone (longer runs of y:
+// 73 against 84 us with two).
+template <int MODE>
+static void col_launch_fp(const ColView& c, const SidArgs& a, uint32_t g0, uint32_t groups, uint32_t nr, const float* Xz,
+                          const float* yin, float* yout, float4* rec, float* wrec, uint32_t* state, uint32_t* rest,
+                          float epps, hipStream_t s) {
+    auto launch = [&](auto kern, uint32_t nb) {
+        hipLaunchKernelGGL(kern, dim3((c.bins + nb - 1) / nb, groups), dim3(256), 0, s, c, a, g0 * kCL, Xz, yin, yout, rec,
+                           wrec, state, rest, epps);
+    };
+    if (MODE == COL_BP) launch(k_col_fp<MODE, MODE == COL_BP ? 4 : 1, 1>, 16);
+    else if (nr == 1) launch(k_col_fp<MODE, 1, 1>, 4);
+    else if (nr == 2) launch(k_col_fp<MODE, 1, 2>, 4);
+    else launch(k_col_fp<MODE, 1, 0>, 4);
+}
+
+// The plane groups of a call, pass after pass. yout: forward projection of img. Otherwise rhs (and sens) += the
+// backprojection of the ratios (img given) or of yin (null: ones).
+static int col_run(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* img, const float* yin,
+                   float* yout, const float* add, float* rhs, float* sens, float epps, hipStream_t s, bool* done) {
+    const omg_geom_desc& d = g->d;
+    const ColView c{pl->bins, (uint32_t)(n / pl->bins), pl->tw, pl->th, pl->ntx, pl->max_segs,
+                    pl->off, pl->start, pl->ent, pl->seg, pl->item};
+    SidArgs a = make_sid_args(g, first, n);
+    a.plane_col = g->index_dev ? 0 : first;   // the z table's first plane (an index table's range holds every plane)
+    a.add = add;
+    const bool small = (uint64_t)d.Nx * d.Ny * (d.Nz <= 63 ? 256 : 512) <= 0xffffffffull;   // a buffer's offsets
+    const uint32_t nr = !small ? 0 : d.Nz <= 63 ? 1 : d.Nz <= 127 ? 2 : 0, pitch = nr ? 64 * nr : d.Nz + 2;
+    const uint32_t all = (c.planes + kCL - 1) / kCL;
+    const uint64_t per = (uint64_t)c.bins * kCL;
+    const uint32_t pass = (uint32_t)std::min<uint64_t>(all, std::max<uint64_t>(1, kColRecords / per));
+    const size_t nimg = img ? ((size_t)d.Nx * d.Ny * pitch + 3) & ~(size_t)3 : 0, nrec = rhs ? 4 * per * pass : 0;
+    const size_t nw = sens ? per * pass : 0, need = nimg + nrec + nw + per * pass + 4;
+    *done = false;
+    if (!scratch_fits(g, need)) return OMG_OK;
+    int rc = scratch_reserve(const_cast<omg_geom*>(g), need);
+    if (rc) return rc;
+    *done = true;
+    float* Xz = scratch_ptr(g);
+    float4* rec = reinterpret_cast<float4*>(Xz + nimg);
+    float* wrec = sens ? Xz + nimg + nrec : nullptr;
+    uint32_t* rest = reinterpret_cast<uint32_t*>(Xz + nimg + nrec + nw);
+    uint32_t* state = rest + per * pass;
+    const size_t lds = col_lds(c.tw, c.th, d.Nz);
+    hipEvent_t stop;
+    timing_begin(s, &stop);
+    if (img)
+        hipLaunchKernelGGL(k_col_zfast, dim3((d.Nx + 31) / 32, d.Ny, (pitch + 31) / 32), dim3(32, 8), 0, s, img, Xz, d.Nx,
+                           d.Ny, d.Nz, pitch, nr ? 0u : 1u, state);
+    OMG_CHECK_LAUNCH();
+    for (uint32_t g0 = 0; g0 < all; g0 += pass) {
+        const uint32_t groups = std::min(pass, all - g0);
+        if (!img || g0) {
+            hipLaunchKernelGGL(k_col_zero, dim3(1), dim3(256), 0, s, state, 4u);
+            OMG_CHECK_LAUNCH();
+        }
+        if (yout) col_launch_fp<COL_FP>(c, a, g0, groups, nr, Xz, yin, yout, rec, wrec, state, rest, epps, s);
+        else if (img) col_launch_fp<COL_OSEM>(c, a, g0, groups, nr, Xz, yin, yout, rec, wrec, state, rest, epps, s);
+        else col_launch_fp<COL_BP>(c, a, g0, groups, nr, Xz, yin, yout, rec, wrec, state, rest, epps, s);
+        OMG_CHECK_LAUNCH();
+        const ColRest r{rest, img, yin, yout, rhs, sens, epps};
+        if (yout) {
+            hipLaunchKernelGGL(k_col_rest, dim3(1024), dim3(64), 0, s, a, state, r);
+        } else {
+            hipLaunchKernelGGL(k_col_bp, dim3(kColRest + pl->items, groups, sens ? 2 : 1), dim3(pl->tpb), lds, s,
+                               c, a, g0 * kCL, kColRest, r, rec, wrec, state);
+        }
+        OMG_CHECK_LAUNCH();
+    }
+    timing_end(s, stop);
+    return OMG_OK;
+}
+
+int col_forward(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* img, float* y,
+                hipStream_t s, bool* done) {
+    return col_run(g, pl, first, n, img, nullptr, y, nullptr, nullptr, nullptr, 0.f, s, done);
+}
+
+int col_backward(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* y, float* rhs, float* sens,
+                 hipStream_t s, bool* done) {
+    return col_run(g, pl, first, n, nullptr, y, nullptr, nullptr, rhs, sens, 0.f, s, done);
+}
+
+int col_osem(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* img, const float* meas,
+             const float* add, float* rhs, float* sens, float epps, hipStream_t s, bool* done) {
+    return col_run(g, pl, first, n, img, meas, nullptr, add, rhs, sens, epps, s, done);
+}
+
+}  // namespace omg

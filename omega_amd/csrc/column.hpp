@@ -1,0 +1,26 @@
+// column.hpp -- 3-D sinogram projections by image columns (column.hip).
+#pragma once
+#include "common.hpp"
+
+struct omg_geom;
+
+namespace omg {
+
+struct ColPlan;
+
+// The transaxial lists that serve measurements [first, first + n) of g, built on the first call that may allocate
+// and wait; null when they do not apply or do not fit.
+const ColPlan* col_plan(const omg_geom* g, int64_t first, int64_t n, hipStream_t s);
+void col_release(omg_geom* g);
+
+// y = A img.
+int col_forward(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* img, float* y,
+                hipStream_t s, bool* done);
+// rhs += A^T y (y null: A^T 1); with sens also sens += A^T 1.
+int col_backward(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* y, float* rhs, float* sens,
+                 hipStream_t s, bool* done);
+// rhs += A^T (meas / (A img + epps (+ add))), NaN and Inf ratios -> epps; with sens also sens += A^T 1.
+int col_osem(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* img, const float* meas,
+             const float* add, float* rhs, float* sens, float epps, hipStream_t s, bool* done);
+
+}  // namespace omg

@@ -5,7 +5,7 @@
 
 #include <vector>
 
-namespace omg { struct PlanePlan; }
+namespace omg { struct PlanePlan; struct ColCache; }
 
 struct omg_geom {
     omg_geom_desc d;          // caller's description (host table pointers cleared after upload)
@@ -42,6 +42,8 @@ struct omg_geom {
     // Direct-plane sinograms: the one 2-D system's lists (plane.hip), built by the first subset iteration that
     // may allocate.
     omg::PlanePlan* plane = nullptr;
+    // 3-D sinograms: the transaxial crossing lists of column.hip, per measurement range used with an index table.
+    omg::ColCache* columns = nullptr;
     // Workgroups per plane for the planar kernels (omg_geom_desc.reserved[1]; 0 = automatic).
     int32_t planar_groups = 0;
     // Library-owned scratch (floats) for partial images; grown on demand, freed with the handle.

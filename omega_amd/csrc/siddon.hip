@@ -10,6 +10,7 @@
 // uses `omp atomic` (source/cpp/projector_functions.h:652-656).
 #include "geom.hpp"
 #include "plane.hpp"
+#include "column.hpp"
 
 #include <utility>
 #include <vector>
@@ -59,6 +60,13 @@ void timing_end(hipStream_t s, hipEvent_t stop) {
 __global__ void k_fill_f32(float* __restrict__ p, uint32_t n, float v) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i < n) p[i] = v;
+}
+
+__global__ void k_clear2(float* __restrict__ p, float* __restrict__ q, uint32_t n) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    p[i] = 0.f;
+    if (q) q[i] = 0.f;
 }
 
 // ---- forward projection -------------------------------------------------------------------------
@@ -683,6 +691,11 @@ static dim3 xy_tiles(const omg_geom* g) { return dim3((g->d.Nx + 31) / 32, (g->d
 // copy measured slower (9.6 ms against 7.4 ms for a C2 forward projection).
 static int generic_fp(const omg_geom* g, int64_t first, int64_t n, const float* img, float* y, hipStream_t s) {
     if (g->d.tof_bins > 1) return tof_forward(g, first, n, img, y, s);
+    if (const ColPlan* pl = col_plan(g, first, n, s)) {
+        bool done = false;
+        const int rc = col_forward(g, pl, first, n, img, y, s, &done);
+        if (rc || done) return rc;
+    }
     const SidArgs a = make_sid_args(g, first, n);
     hipEvent_t stop;
     timing_begin(s, &stop);
@@ -696,6 +709,11 @@ static int generic_fp(const omg_geom* g, int64_t first, int64_t n, const float* 
 static int generic_osem(const omg_geom* g, int64_t first, int64_t n, const float* img, const float* meas, float* rhs,
                         float* sens, float epps, hipStream_t s, const float* add) {
     if (g->d.tof_bins > 1) return tof_osem(g, first, n, img, meas, rhs, sens, epps, s, add);
+    if (const ColPlan* pl = col_plan(g, first, n, s)) {
+        bool done = false;
+        const int rc = col_osem(g, pl, first, n, img, meas, add, rhs, sens, epps, s, &done);
+        if (rc || done) return rc;
+    }
     SidArgs a = make_sid_args(g, first, n);
     a.add = add;
     float *rhs_t = nullptr, *sens_t = nullptr;
@@ -779,6 +797,11 @@ extern "C" int omg_backward_project(const omg_geom* g, int64_t first, int64_t n_
         return launch_planar<false, true, false>(g, first, n_meas, nullptr, y, nullptr, rhs, nullptr, 0.f, s);
     }
     if (g->d.tof_bins > 1) return tof_backward(g, first, n_meas, y, rhs, sens, s);
+    if (const ColPlan* pl = col_plan(g, first, n_meas, s)) {
+        bool done = false;
+        rc = col_backward(g, pl, first, n_meas, y, rhs, sens, s, &done);
+        if (rc || done) return rc;
+    }
     SidArgs a = make_sid_args(g, first, n_meas);
     if (split_layout(g)) {
         // x-major LORs into y-fastest buffers (scratch), added back transposed
@@ -1014,12 +1037,8 @@ int omg_osem_subset_iteration_impl(const omg_geom* g, int64_t first, int64_t n_m
     }
     // one-lane-per-LOR path: rhs (and S) accumulate with global atomics, then the update
     float* rhs = work_ptr(g) + N;
-    hipLaunchKernelGGL(k_fill_f32, dim3(grid_for(N, 256)), dim3(256), 0, s, rhs, N, 0.f);
+    hipLaunchKernelGGL(k_clear2, dim3(grid_for(N, 256)), dim3(256), 0, s, rhs, compute_sens ? S : nullptr, N);
     OMG_CHECK_LAUNCH();
-    if (compute_sens) {
-        hipLaunchKernelGGL(k_fill_f32, dim3(grid_for(N, 256)), dim3(256), 0, s, S, N, 0.f);
-        OMG_CHECK_LAUNCH();
-    }
     if (n_meas > 0 && is_tube(g)) {
         rc = orth_osem(g, first, n_meas, x, meas, rhs, compute_sens ? S : nullptr, epps, s, additive);
         if (rc) return rc;

@@ -46,6 +46,7 @@ struct SidArgs {
     uint32_t pitch;                // row pitch of slice-relative (planar) voxel indices: Nx, or Nx + 1 in LDS
     const uint32_t* __restrict__ index;  // PET sinogram: sinogram bin per measurement (subset types 1-5), or null;
                                          // plane_offset is then the call's first measurement in this table
+    int64_t plane_col = 0;         // column kernels (column.hip): the call's first plane in the z table
     const float* __restrict__ add;  // additive term of the fused ratio (randoms / scatter), call-local, or null
 };
 
@@ -564,8 +565,21 @@ __device__ __forceinline__ bool siddon_gather(const SidArgs& g, int64_t lo, cons
     ax = 0.f;
     Walk w;
     if (!siddon_setup<PLANAR>(g, lo, w, weight, false, ray)) return false;
-    if (w.perp) {
-        perp_walk(w, [&](uint32_t ind, float len) { ax += len * src[ind]; });
+    if (w.perp) {   // kBatch loads in flight here too; the order of the sum is the row's
+        for (uint32_t i0 = w.p_a1; i0 <= w.p_a2; i0 += kBatch) {
+            float len[kBatch], v[kBatch];
+            bool in[kBatch];
+#pragma unroll
+            for (uint32_t k = 0; k < kBatch; k++) {
+                const uint32_t ii = i0 + k, ind = w.p_ind + (ii - w.p_a1) * w.p_stride;
+                in[k] = ii <= w.p_a2 && ind < w.p_lim;
+                len[k] = (w.p_a1 > 0 && ii == w.p_a1) ? w.p_dT1
+                         : (w.p_a2 < w.p_nrun - 1 && ii == w.p_a2) ? w.p_dT2 : w.p_d;
+                v[k] = src[in[k] ? ind : 0u];
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < kBatch; k++) ax = in[k] ? ax + len[k] * v[k] : ax;
+        }
         return true;
     }
     while (w.left > 0u) {

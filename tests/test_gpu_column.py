@@ -1,0 +1,89 @@
+"""3-D sinograms by image columns (column.hip) against the one-lane-per-LOR kernels (omg_geom_desc.reserved[0]).
+
+The forward projection adds the same 32-bit products in the same order, so it is compared bit for bit. The
+backprojection adds the same products in 64-bit fixed point where the other kernels use 32-bit float atomics over at
+most ~5e3 terms per voxel: 2^-24 sqrt(5e3) = 4e-6 relative L2; bar 2e-5. A length between two crossings carries the
+rounding of their parameters, 2^-24 of a LOR of up to ~150 mm (1e-5 mm) each: the updated image is compared where the
+sensitivity is at least 0.5 mm, so that a voxel's own error stays below the bar. Images of one, two and more than two
+registers of slices per lane, odd, non-square and smaller than a tile; plane counts around the 64 of a wave; planes
+far steeper than a voxel, outside the image, and leaving it through an end face.
+"""
+import numpy as np
+import pytest
+
+from omega_amd import _lib, geometry as G
+from tests.hip_helpers import make_geom, ptr, rel_l2
+
+pytestmark = pytest.mark.gpu
+EPPS = 1e-5
+BAR = 2e-5
+
+
+def _scanner(nx, ny, nz, n_radial, n_angles, planes, dz=2.5):
+    fov = 2.5 * max(nx, ny)
+    grid = G.Grid.from_fov(nx, ny, nz, fov, fov, dz * nz)
+    x = G.ring_sinogram_xy(n_radial, n_angles, fov / n_radial, 1.25 * fov)
+    rng = np.random.default_rng(planes)
+    half = 0.5 * dz * nz
+    z = rng.uniform(-half, half, (planes, 2))
+    z[:: 5] = np.repeat(grid.centers()[2][rng.integers(0, nz, len(z[::5]))][:, None], 2, axis=1)   # direct
+    z[1:: 7] *= 6.0                                                                                # through the end faces
+    z[3] = (2.0 * half, 3.0 * half)                                                                # beside the image
+    return grid, x, z.astype(np.float32)
+
+
+def _run(geom, grid, first, n, img, y, meas):
+    import torch
+    out = torch.empty(n, device="cuda")
+    _lib.call("omg_forward_project", geom.handle, first, n, ptr(img), ptr(out), None)
+    back, S = torch.zeros(grid.N, device="cuda"), torch.zeros(grid.N, device="cuda")
+    _lib.call("omg_backward_project", geom.handle, first, n, ptr(y), ptr(back), ptr(S), None)
+    x, Sx = img.clone(), torch.zeros(grid.N, device="cuda")
+    for sens in (1, 0):
+        _lib.call("omg_osem_subset_iteration_ex", geom.handle, first, n, ptr(x), ptr(meas), None, ptr(Sx), sens, EPPS,
+                  0.0, 2.0, 1, None)
+    torch.cuda.synchronize()
+    return [t.cpu().numpy() for t in (out, back, S, x, Sx)]
+
+
+@pytest.mark.parametrize("nx,ny,nz,n_radial,n_angles,planes,first,dz", [
+    (20, 20, 9, 24, 20, 32, 0, 2.5), (33, 21, 15, 29, 23, 63, 1, 2.5), (7, 5, 63, 11, 9, 64, 0, 2.5),
+    (17, 18, 64, 19, 16, 65, 0, 1.0), (16, 32, 127, 20, 12, 40, 0, 0.7), (16, 16, 128, 20, 12, 70, 2, 0.6),
+    (3, 3, 301, 8, 6, 129, 0, 0.3), (40, 40, 2, 32, 32, 130, 0, 9.0)])
+def test_column(cuda, nx, ny, nz, n_radial, n_angles, planes, first, dz):
+    import torch
+    grid, x, z = _scanner(nx, ny, nz, n_radial, n_angles, planes + first, dz)
+    n = planes * n_radial * n_angles
+    rng = np.random.default_rng(1)
+    norm = rng.random(n_radial * n_angles * (planes + first)).astype(np.float32) + 0.5
+    up = lambda a: torch.from_numpy(a.astype(np.float32)).cuda()
+    img, y, meas = up(rng.random(grid.N) + 0.5), up(rng.standard_normal(n)), up(rng.poisson(2.0, n))
+    a, b = (_run(make_geom(grid, x, z, n_radial, n_angles, generic=gen, norm=norm, global_factor=0.9), grid, first, n,
+                 img, y, meas) for gen in (False, True))
+    seen = b[4] > 0.5
+    assert seen.any()
+    a[3], b[3] = a[3][seen], b[3][seen]
+    e = [rel_l2(p, q) for p, q in zip(a, b)]
+    print(f"[column] {nx}x{ny}x{nz} planes={planes} rel-L2 {e}", flush=True)
+    assert np.array_equal(a[0], b[0])
+    assert max(e[1:]) < BAR
+
+
+def test_not_finite(cuda):
+    """A NaN or an infinity in the image or the data goes where the other kernels take it, and nowhere else."""
+    import torch
+    grid, x, z = _scanner(20, 20, 9, 24, 20, 40)
+    n = 40 * 24 * 20
+    rng = np.random.default_rng(2)
+    img, y, meas = rng.random(grid.N) + 0.5, rng.random(n), rng.poisson(2.0, n)
+    img[grid.N // 2 + 3], img[grid.N // 3], y[n // 2], y[n // 3] = np.inf, np.nan, np.nan, np.inf
+    up = lambda a: torch.from_numpy(a.astype(np.float32)).cuda()
+    a, b = (_run(make_geom(grid, x, z, 24, 20, generic=gen), grid, 0, n, up(img), up(y), up(meas))
+            for gen in (False, True))
+    assert np.array_equal(a[0], b[0], equal_nan=True)
+    seen = b[4] > 0.5
+    a[3], b[3] = a[3][seen], b[3][seen]
+    for p, q in zip(a[1:], b[1:]):
+        assert np.array_equal(np.isfinite(p), np.isfinite(q))
+        ok = np.isfinite(q)
+        assert rel_l2(p[ok], q[ok]) < BAR
