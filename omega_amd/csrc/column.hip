@@ -855,36 +855,58 @@ static void col_launch_fp(const ColView& c, const SidArgs& a, uint32_t g0, uint3
     else launch(k_col_fp<MODE, 1, 0>, 4);
 }
 
+struct ColWork {
+    uint32_t nr, pitch, all, pass;
+    uint64_t per;
+    size_t nimg, nrec, nw, need;
+};
+
+static ColWork col_work(const omg_geom* g, const ColPlan* pl, int64_t n, bool img, bool rec, bool sens) {
+    const omg_geom_desc& d = g->d;
+    ColWork w;
+    const bool small = (uint64_t)d.Nx * d.Ny * (d.Nz <= 63 ? 256 : 512) <= 0xffffffffull;   // a buffer's offsets
+    w.nr = !small ? 0 : d.Nz <= 63 ? 1 : d.Nz <= 127 ? 2 : 0;
+    w.pitch = w.nr ? 64 * w.nr : d.Nz + 2;
+    w.all = (uint32_t)((n / pl->bins + kCL - 1) / kCL);
+    w.per = (uint64_t)pl->bins * kCL;
+    w.pass = (uint32_t)std::min<uint64_t>(w.all, std::max<uint64_t>(1, kColRecords / w.per));
+    w.nimg = img ? ((size_t)d.Nx * d.Ny * w.pitch + 3) & ~(size_t)3 : 0;
+    w.nrec = rec ? 4 * w.per * w.pass : 0;
+    w.nw = sens ? w.per * w.pass : 0;
+    w.need = w.nimg + w.nrec + w.nw + w.per * w.pass + 4;
+    return w;
+}
+
+size_t col_osem_work(const omg_geom* g, const ColPlan* pl, int64_t n) { return col_work(g, pl, n, true, true, false).need; }
+
 // The plane groups of a call, pass after pass. yout: forward projection of img. Otherwise rhs (and sens) += the
-// backprojection of the ratios (img given) or of yin (null: ones).
+// backprojection of the ratios (img given) or of yin (null: ones). work: the caller's, or null for the handle's.
 static int col_run(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* img, const float* yin,
-                   float* yout, const float* add, float* rhs, float* sens, float epps, hipStream_t s, bool* done) {
+                   float* yout, const float* add, float* rhs, float* sens, float epps, float* work, hipStream_t s,
+                   bool* done) {
     const omg_geom_desc& d = g->d;
     const ColView c{pl->bins, (uint32_t)(n / pl->bins), pl->tw, pl->th, pl->ntx, pl->max_segs,
                     pl->off, pl->start, pl->ent, pl->seg, pl->item};
     SidArgs a = make_sid_args(g, first, n);
     a.plane_col = g->index_dev ? 0 : first;   // the z table's first plane (an index table's range holds every plane)
     a.add = add;
-    const bool small = (uint64_t)d.Nx * d.Ny * (d.Nz <= 63 ? 256 : 512) <= 0xffffffffull;   // a buffer's offsets
-    const uint32_t nr = !small ? 0 : d.Nz <= 63 ? 1 : d.Nz <= 127 ? 2 : 0, pitch = nr ? 64 * nr : d.Nz + 2;
-    const uint32_t all = (c.planes + kCL - 1) / kCL;
-    const uint64_t per = (uint64_t)c.bins * kCL;
-    const uint32_t pass = (uint32_t)std::min<uint64_t>(all, std::max<uint64_t>(1, kColRecords / per));
-    const size_t nimg = img ? ((size_t)d.Nx * d.Ny * pitch + 3) & ~(size_t)3 : 0, nrec = rhs ? 4 * per * pass : 0;
-    const size_t nw = sens ? per * pass : 0, need = nimg + nrec + nw + per * pass + 4;
+    const ColWork w = col_work(g, pl, n, img != nullptr, rhs != nullptr, sens != nullptr);
+    const uint32_t nr = w.nr, pitch = w.pitch, all = w.all, pass = w.pass;
     *done = false;
-    if (!scratch_fits(g, need)) return OMG_OK;
-    int rc = scratch_reserve(const_cast<omg_geom*>(g), need);
-    if (rc) return rc;
+    if (!work) {
+        if (!scratch_fits(g, w.need)) return OMG_OK;
+        const int rc = scratch_reserve(const_cast<omg_geom*>(g), w.need);
+        if (rc) return rc;
+    }
     *done = true;
-    float* Xz = scratch_ptr(g);
-    float4* rec = reinterpret_cast<float4*>(Xz + nimg);
-    float* wrec = sens ? Xz + nimg + nrec : nullptr;
-    uint32_t* rest = reinterpret_cast<uint32_t*>(Xz + nimg + nrec + nw);
-    uint32_t* state = rest + per * pass;
+    float* Xz = work ? work : scratch_ptr(g);
+    float4* rec = reinterpret_cast<float4*>(Xz + w.nimg);
+    float* wrec = sens ? Xz + w.nimg + w.nrec : nullptr;
+    uint32_t* rest = reinterpret_cast<uint32_t*>(Xz + w.nimg + w.nrec + w.nw);
+    uint32_t* state = rest + w.per * pass;
     const size_t lds = col_lds(c.tw, c.th, d.Nz);
-    hipEvent_t stop;
-    timing_begin(s, &stop);
+    hipEvent_t stop = nullptr;
+    if (!work) timing_begin(s, &stop);
     if (img)
         hipLaunchKernelGGL(k_col_zfast, dim3((d.Nx + 31) / 32, d.Ny, (pitch + 31) / 32), dim3(32, 8), 0, s, img, Xz, d.Nx,
                            d.Ny, d.Nz, pitch, nr ? 0u : 1u, state);
@@ -908,23 +930,23 @@ static int col_run(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t 
         }
         OMG_CHECK_LAUNCH();
     }
-    timing_end(s, stop);
+    if (!work) timing_end(s, stop);
     return OMG_OK;
 }
 
 int col_forward(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* img, float* y,
                 hipStream_t s, bool* done) {
-    return col_run(g, pl, first, n, img, nullptr, y, nullptr, nullptr, nullptr, 0.f, s, done);
+    return col_run(g, pl, first, n, img, nullptr, y, nullptr, nullptr, nullptr, 0.f, nullptr, s, done);
 }
 
 int col_backward(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* y, float* rhs, float* sens,
                  hipStream_t s, bool* done) {
-    return col_run(g, pl, first, n, nullptr, y, nullptr, nullptr, rhs, sens, 0.f, s, done);
+    return col_run(g, pl, first, n, nullptr, y, nullptr, nullptr, rhs, sens, 0.f, nullptr, s, done);
 }
 
 int col_osem(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* img, const float* meas,
-             const float* add, float* rhs, float* sens, float epps, hipStream_t s, bool* done) {
-    return col_run(g, pl, first, n, img, meas, nullptr, add, rhs, sens, epps, s, done);
+             const float* add, float* rhs, float* sens, float epps, float* work, hipStream_t s, bool* done) {
+    return col_run(g, pl, first, n, img, meas, nullptr, add, rhs, sens, epps, work, s, done);
 }
 
 }  // namespace omg

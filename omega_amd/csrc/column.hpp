@@ -19,8 +19,10 @@ int col_forward(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, 
 // rhs += A^T y (y null: A^T 1); with sens also sens += A^T 1.
 int col_backward(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* y, float* rhs, float* sens,
                  hipStream_t s, bool* done);
-// rhs += A^T (meas / (A img + epps (+ add))), NaN and Inf ratios -> epps; with sens also sens += A^T 1.
+// rhs += A^T (meas / (A img + epps (+ add))), NaN and Inf ratios -> epps; with sens also sens += A^T 1. work: null, or
+// col_osem_work floats (calls without sens) that the caller keeps, 16-byte aligned.
+size_t col_osem_work(const omg_geom* g, const ColPlan* pl, int64_t n);
 int col_osem(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* img, const float* meas,
-             const float* add, float* rhs, float* sens, float epps, hipStream_t s, bool* done);
+             const float* add, float* rhs, float* sens, float epps, float* work, hipStream_t s, bool* done);
 
 }  // namespace omg

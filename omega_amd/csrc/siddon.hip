@@ -711,7 +711,7 @@ static int generic_osem(const omg_geom* g, int64_t first, int64_t n, const float
     if (g->d.tof_bins > 1) return tof_osem(g, first, n, img, meas, rhs, sens, epps, s, add);
     if (const ColPlan* pl = col_plan(g, first, n, s)) {
         bool done = false;
-        const int rc = col_osem(g, pl, first, n, img, meas, add, rhs, sens, epps, s, &done);
+        const int rc = col_osem(g, pl, first, n, img, meas, add, rhs, sens, epps, nullptr, s, &done);
         if (rc || done) return rc;
     }
     SidArgs a = make_sid_args(g, first, n);

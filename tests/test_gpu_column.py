@@ -8,6 +8,8 @@ sensitivity is at least 0.5 mm, so that a voxel's own error stays below the bar.
 registers of slices per lane, odd, non-square and smaller than a tile; plane counts around the 64 of a wave; planes
 far steeper than a voxel, outside the image, and leaving it through an end face.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -87,3 +89,44 @@ def test_not_finite(cuda):
         assert np.array_equal(np.isfinite(p), np.isfinite(q))
         ok = np.isfinite(q)
         assert rel_l2(p[ok], q[ok]) < BAR
+
+
+@pytest.mark.parametrize("frames,planes", [(1, 40), (4, 64), (3, 97)])
+def test_frames(cuda, frames, planes):
+    """Two subset steps of a dynamic study, launched and replayed from a graph."""
+    import torch
+    grid, x, z = _scanner(21, 18, 11, 20, 16, planes)
+    n, N = planes * 320, grid.N
+    rng = np.random.default_rng(planes)
+    up = lambda a: torch.from_numpy(a.astype(np.float32)).cuda()
+    meas, x0 = up(rng.poisson(0.3, (frames, n))), up(rng.random((frames, N)) + 0.5)
+    out = []
+    for gen in (False, True):
+        g = make_geom(grid, x, z, 20, 16, generic=gen)
+        S, rhs, xs = torch.empty(N, device="cuda"), torch.zeros(frames, N, device="cuda"), x0.clone()
+        y = torch.empty(frames, n, device="cuda")
+        _lib.call("omg_frames_sensitivity", g.handle, 0, n, ptr(S), EPPS, None)
+        tail = (0.0, 2.0, EPPS, 1, 128, 1, 0)
+        for _ in range(2):
+            _lib.call("omg_frames_osem_step", g.handle, 0, n, frames, ptr(xs), ptr(meas), n, ptr(S), ptr(rhs), None, *tail,
+                      None)
+        _lib.call("omg_frames_forward", g.handle, 0, n, frames, ptr(x0), ptr(y), n, None)
+        torch.cuda.synchronize()
+        res = [S.cpu().numpy(), xs.cpu().numpy(), y.cpu().numpy()]
+        ints = [np.array([v], np.int64) for v in (0, n, 0)]
+        h, xs = C.c_void_p(), x0.clone()
+        torch.cuda.synchronize()
+        _lib.call("omg_frames_graph_create", g.handle, 1, *(v.ctypes.data for v in ints), frames, ptr(xs), ptr(meas), n,
+                  ptr(S), ptr(rhs), None, *tail, C.byref(h))
+        for _ in range(2):
+            _lib.call("omg_graph_launch", h, None)
+            torch.cuda.synchronize()
+            rhs.fill_(7.0)
+        _lib.call("omg_graph_destroy", h)
+        out.append(res + [xs.cpu().numpy()])
+    a, b = out
+    assert np.array_equal(a[2], b[2])
+    seen = b[0] > 0.5
+    assert rel_l2(a[0], b[0]) < BAR
+    for k in (1, 3):
+        assert rel_l2(a[k][:, seen], b[1][:, seen]) < BAR
