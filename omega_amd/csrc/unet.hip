@@ -338,49 +338,44 @@ __global__ __launch_bounds__(256) void k_conv3d_wgrad(const uint16_t* __restrict
 }
 
 // ---- weight gradient on the K = 32 BF16 matrix cores ---------------------------------------------------
-// dW[tap][co][ci] = sum_v dY[v][co] X[v + off(tap)][ci] is a product whose K dimension is the voxels. The
-// MFMA's lanes hold 8 consecutive K values of one row (A) or column (B), so both operands are staged
-// transposed in LDS: dYt[co][voxel] for the block's 32 x 4 x 2 voxels and, for one 16-channel slice of X
-// (blockIdx.y), Xt[dx + 1][ci][halo row][x] -- three copies of the (2 + 2) x (4 + 2) halo rows shifted by
-// dx = -1, 0, 1, so that every operand is one aligned 16-byte LDS read. The 8 waves split the 27 taps
-// (wave w: w, w + 8, w + 16, w + 24) and reuse each row's dY operand across theirs. Blocks persist over
-// the tiles (blockIdx.x, step gridDim.x) and store their sums as one partial per block, added into dW by
-// k_wgrad_reduce (no atomics).
+// dW[tap][co][ci] = sum_v dY[v][co] X[v + off(tap)][ci] is a product whose K dimension is the voxels, and the MFMA's
+// lanes hold several K values of one row (A) or column (B). Both operands lie in LDS as they do in memory, 16
+// channels of a voxel in 32 bytes, and are read by the transposing LDS load: 16 lanes address 4 voxels and lane c
+// receives channel c of them. So a shift along x is an offset of 32 bytes, and a wave's load covers 512 contiguous
+// bytes (no bank conflicts): lane group q holds voxels 4 q + 0..3 and 16 + 4 q + 0..3 of a 32-voxel row, in A and B
+// alike. A block takes 32 x 4 x 2 voxels of dY and one 16-channel slice of X (blockIdx.y) with its halo; its 8 waves
+// split the 27 taps (wave w: w, w + 8, w + 16, w + 24) and reuse each row's dY operand across theirs; the next tile
+// loads into registers meanwhile. Blocks persist over the tiles (blockIdx.x, step gridDim.x) and store their sums
+// as one partial per block, added into dW by k_wgrad_reduce (no atomics). What bounds it: the LDS reads, 432 + 16 MT
+// of 512 bytes per tile and channel slice, behind 216 MT MFMAs. 128 x 128 x 64 voxels, mean of three 16 -> 16 channel
+// layers and one 48 -> 16: 38 us; 104 us with operands transposed by 8-byte LDS writes, three copies for the
+// shifts and one workgroup per CU. 32 outputs at an eighth of the voxels: 22 against 35 us.
 constexpr int kWgTX = 32, kWgTY = 4, kWgTZ = 2, kWgRows = kWgTY * kWgTZ, kWgVox = kWgTX * kWgRows;
-constexpr int kWgHY = kWgTY + 2, kWgHZ = kWgTZ + 2, kWgHRows = kWgHY * kWgHZ, kWgThreads = 512;
-// channel-row strides of the LDS operands, padded by 16 B so that the 16 lanes of a read phase (one
-// channel each, 16 B apart otherwise a multiple of the 256-byte bank cycle) fall on distinct banks
-constexpr int kWgDS = kWgVox + 8, kWgXS = kWgHRows * kWgTX + 8;
+constexpr int kWgHX = kWgTX + 2, kWgHY = kWgTY + 2, kWgHZ = kWgTZ + 2, kWgHRows = kWgHY * kWgHZ, kWgThreads = 512;
 
-// u[e] holds 8 channels of voxel e; channel j's 4 voxels go to dst + j * stride as one 8-byte write.
-__device__ __forceinline__ void wg_store4(uint16_t* dst, size_t stride, const uint4 (&u)[4]) {
-    const uint32_t w[4][4] = {{u[0].x, u[0].y, u[0].z, u[0].w}, {u[1].x, u[1].y, u[1].z, u[1].w},
-                              {u[2].x, u[2].y, u[2].z, u[2].w}, {u[3].x, u[3].y, u[3].z, u[3].w}};
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int sh = 16 * (j & 1), k = j >> 1;
-        const uint32_t lo = ((w[0][k] >> sh) & 0xffffu) | (((w[1][k] >> sh) & 0xffffu) << 16);
-        const uint32_t hi = ((w[2][k] >> sh) & 0xffffu) | (((w[3][k] >> sh) & 0xffffu) << 16);
-        *reinterpret_cast<uint2*>(dst + (size_t)j * stride) = uint2{lo, hi};
-    }
+typedef __attribute__((ext_vector_type(4))) short wg_s4;
+
+// 8 K values of channel lane & 15: `p` is the row's first voxel (in 16-channel units) plus 4 lane elements.
+__device__ __forceinline__ bf8 wg_read(const uint16_t* p) {
+    typedef __attribute__((address_space(3))) wg_s4* lds_ptr;
+    const wg_s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)p);
+    const wg_s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p + 256));
+    return __builtin_bit_cast(bf8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
 template <int MT>
-constexpr size_t wgrad_tile_lds() { return sizeof(uint16_t) * ((size_t)MT * 16 * kWgDS + 3 * 16 * (size_t)kWgXS); }
-
-template <int MT>
-__global__ __launch_bounds__(kWgThreads) void k_conv3d_wgrad_tile(const uint16_t* __restrict__ dY,
-                                                                  const uint16_t* __restrict__ X1, int C1,
-                                                                  const uint16_t* __restrict__ X2, int C2,
-                                                                  float* __restrict__ part, Vol g, int tiles_x,
-                                                                  int tiles_y, int n_tiles) {
+__global__ __launch_bounds__(kWgThreads, MT == 4 ? 2 : 4) void k_conv3d_wgrad_tile(const uint16_t* __restrict__ dY,
+                                                                     const uint16_t* __restrict__ X1, int C1,
+                                                                     const uint16_t* __restrict__ X2, int C2,
+                                                                     float* __restrict__ part, Vol g, int tiles_x,
+                                                                     int tiles_y, int n_tiles) {
     constexpr int Cout = MT * 16;
-    extern __shared__ uint16_t wl[];
-    uint16_t* dYt = wl;                              // [Cout][kWgVox], row stride kWgDS
-    uint16_t* Xt = wl + (size_t)Cout * kWgDS;        // [3][16][kWgHRows][kWgTX], channel stride kWgXS
+    constexpr int kXItems = kWgHRows * kWgHX * 2, kXLoads = (kXItems + kWgThreads - 1) / kWgThreads;   // of 8 channels
+    __shared__ __attribute__((aligned(16))) uint16_t dYt[MT * kWgVox * 16];                            // [m][voxel][16]
+    __shared__ __attribute__((aligned(16))) uint16_t Xt[kXItems * 8];                                  // [halo voxel][16]
     const int Cin = C1 + C2;
     const int n = blockIdx.y;                        // input-channel slice [16 n, 16 n + 16)
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, q = lane >> 4;
     const int ntap = wave < 3 ? 4 : 3;
     f4v acc[4][MT];
@@ -391,59 +386,56 @@ __global__ __launch_bounds__(kWgThreads) void k_conv3d_wgrad_tile(const uint16_t
     const uint16_t* Xs = (n * 16 < C1) ? X1 : X2;    // the slice lies in one input (C1 % 16 == 0)
     const int Cs = (n * 16 < C1) ? C1 : C2;
     const int cs0 = (n * 16 < C1) ? n * 16 : n * 16 - C1;
-    for (int ti = blockIdx.x; ti < n_tiles; ti += gridDim.x) {
+    uint4 fx[kXLoads], fy[MT];
+    auto load = [&](int ti) {
         const int bx = ti % tiles_x, rest = ti / tiles_x;
         const int x0 = bx * kWgTX, y0 = (rest % tiles_y) * kWgTY, z0 = (rest / tiles_y) * kWgTZ;
-        // Transposing fills: an item is 4 consecutive voxels of 8 channels (four 16-byte loads), stored as one
-        // 8-byte LDS write per channel. dY tile:
-        for (int i = threadIdx.x; i < (kWgVox / 4) * (Cout / 8); i += kWgThreads) {
-            const int quad = i / (Cout / 8), c8 = (i - quad * (Cout / 8)) * 8;
-            const int vox = quad * 4;
-            const int vx = vox % kWgTX, r = vox / kWgTX, vy = r % kWgTY, vz = r / kWgTY;
-            const int y = y0 + vy, z = z0 + vz;
-            uint4 u[4];
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int x = x0 + vx + e;
-                u[e] = uint4{0u, 0u, 0u, 0u};
-                if (x < g.W && y < g.H && z < g.D)
-                    u[e] = *reinterpret_cast<const uint4*>(dY + (((size_t)z * g.H + y) * g.W + x) * Cout + c8);
-            }
-            wg_store4(dYt + (size_t)c8 * kWgDS + vox, kWgDS, u);
+        for (int k = 0; k < kXLoads; k++) {
+            const int i = threadIdx.x + k * kWgThreads, v = i >> 1, hrow = v / kWgHX;
+            const int x = x0 + v - hrow * kWgHX - 1, y = y0 + hrow % kWgHY - 1, z = z0 + hrow / kWgHY - 1;
+            fx[k] = uint4{0u, 0u, 0u, 0u};
+            if (i < kXItems && x >= 0 && x < g.W && y >= 0 && y < g.H && z >= 0 && z < g.D)
+                fx[k] = *reinterpret_cast<const uint4*>(Xs + (((size_t)z * g.H + y) * g.W + x) * Cs + cs0 + (i & 1) * 8);
         }
-        // X slice: halo rows, and in copy d the voxels x0 + p + d - 1 at p = 0..31 (x from x0 - 1 to x0 + 32)
-        for (int i = threadIdx.x; i < kWgHRows * (kWgTX / 4) * 2 * 3; i += kWgThreads) {
-            const int d = i % 3, r2 = i / 3;
-            const int c8 = (r2 & 1) * 8, r3 = r2 >> 1;
-            const int xq = r3 % (kWgTX / 4), hrow = r3 / (kWgTX / 4);
-            const int hy = hrow % kWgHY, hz = hrow / kWgHY;
-            const int y = y0 + hy - 1, z = z0 + hz - 1;
-            const bool row_in = y >= 0 && y < g.H && z >= 0 && z < g.D;
-            uint4 u[4];
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int x = x0 + xq * 4 + e + d - 1;
-                u[e] = uint4{0u, 0u, 0u, 0u};
-                if (row_in && x >= 0 && x < g.W)
-                    u[e] = *reinterpret_cast<const uint4*>(Xs + (((size_t)z * g.H + y) * g.W + x) * Cs + cs0 + c8);
-            }
-            wg_store4(Xt + (size_t)(d * 16 + c8) * kWgXS + hrow * kWgTX + xq * 4, kWgXS, u);
+        for (int k = 0; k < MT; k++) {
+            const int i = threadIdx.x + k * kWgThreads, vox = i / (2 * MT);
+            const int x = x0 + vox % kWgTX, y = y0 + vox / kWgTX % kWgTY, z = z0 + vox / (kWgTX * kWgTY);
+            fy[k] = uint4{0u, 0u, 0u, 0u};
+            if (x < g.W && y < g.H && z < g.D)
+                fy[k] = *reinterpret_cast<const uint4*>(dY + (((size_t)z * g.H + y) * g.W + x) * Cout + i % (2 * MT) * 8);
+        }
+    };
+    const uint16_t* tap_at[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const int tap = min(wave + 8 * t, 26);
+        tap_at[t] = Xt + ((tap / 9 * kWgHY + tap / 3 % 3) * kWgHX + tap % 3) * 16 + lane * 4;
+    }
+    if (blockIdx.x < n_tiles) load(blockIdx.x);
+    for (int ti = blockIdx.x; ti < n_tiles; ti += gridDim.x) {
+#pragma unroll
+        for (int k = 0; k < kXLoads; k++) {
+            const int i = threadIdx.x + k * kWgThreads;
+            if (i < kXItems) *reinterpret_cast<uint4*>(Xt + (size_t)i * 8) = fx[k];
+        }
+#pragma unroll
+        for (int k = 0; k < MT; k++) {
+            const int i = threadIdx.x + k * kWgThreads, vox = i / (2 * MT), c = i % (2 * MT);
+            *reinterpret_cast<uint4*>(dYt + ((c >> 1) * kWgVox + vox) * 16 + (c & 1) * 8) = fy[k];
         }
         __syncthreads();
+        if (ti + (int)gridDim.x < n_tiles) load(ti + gridDim.x);
 #pragma unroll
         for (int r = 0; r < kWgRows; r++) {
-            const int ry = r % kWgTY, rz = r / kWgTY;
             bf8 a[MT];
 #pragma unroll
-            for (int m = 0; m < MT; m++)
-                a[m] = *reinterpret_cast<const bf8*>(dYt + (size_t)(m * 16 + col) * kWgDS + r * kWgTX + 8 * q);
+            for (int m = 0; m < MT; m++) a[m] = wg_read(dYt + (m * kWgVox + r * kWgTX) * 16 + lane * 4);
 #pragma unroll
             for (int t = 0; t < 4; t++) {
                 if (t >= ntap) break;
-                const int tap = wave + 8 * t;
-                const int dz = tap / 9, dy = (tap / 3) % 3, dx = tap % 3;   // 0..2: offset + 1
-                const int hrow = (rz + dz) * kWgHY + (ry + dy);
-                const bf8 b = *reinterpret_cast<const bf8*>(Xt + (size_t)(dx * 16 + col) * kWgXS + hrow * kWgTX + 8 * q);
+                const bf8 b = wg_read(tap_at[t] + (r / kWgTY * kWgHY + r % kWgTY) * kWgHX * 16);
 #pragma unroll
                 for (int m = 0; m < MT; m++) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], b, acc[t][m], 0, 0, 0);
             }
@@ -961,7 +953,7 @@ static int launch_wgrad_tile(const uint16_t* dY, const uint16_t* X1, int C1, con
     const int Cin = C1 + C2, NT = Cin / 16;
     const int tiles_x = (g.W + kWgTX - 1) / kWgTX, tiles_y = (g.H + kWgTY - 1) / kWgTY;
     const int n_tiles = tiles_x * tiles_y * ((g.D + kWgTZ - 1) / kWgTZ);
-    const int P = std::max(1, std::min(n_tiles, 256));   // persistent blocks per channel slice
+    const int P = std::max(1, std::min(n_tiles, NT == 1 ? 512 : 256));   // persistent blocks per slice: two per CU
     const size_t per = (size_t)27 * MT * 16 * Cin;
     if ((size_t)P * per > g_wg_floats) {
         OMG_CHECK_HIP(hipStreamSynchronize(s));
@@ -971,14 +963,7 @@ static int launch_wgrad_tile(const uint16_t* dY, const uint16_t* X1, int C1, con
         OMG_CHECK_HIP(hipMalloc(reinterpret_cast<void**>(&g_wg_part), (size_t)P * per * sizeof(float)));
         g_wg_floats = (size_t)P * per;
     }
-    const size_t lds = wgrad_tile_lds<MT>();
-    static bool attr = false;
-    if (!attr) {
-        OMG_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_conv3d_wgrad_tile<MT>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        attr = true;
-    }
-    hipLaunchKernelGGL(k_conv3d_wgrad_tile<MT>, dim3((unsigned)P, (unsigned)NT), dim3(kWgThreads), lds, s, dY, X1, C1,
+    hipLaunchKernelGGL(k_conv3d_wgrad_tile<MT>, dim3((unsigned)P, (unsigned)NT), dim3(kWgThreads), 0, s, dY, X1, C1,
                        X2, C2, g_wg_part, g, tiles_x, tiles_y, n_tiles);
     OMG_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_wgrad_reduce, dim3((unsigned)((per + 63) / 64)), dim3(1024), 0, s, g_wg_part, dW, per, P);

@@ -109,6 +109,24 @@ def test_conv_forward_tile_shapes(cuda, dhw, cins, cout):
     assert np.all(np.abs(got - ref) <= 2.0 ** -8 * np.abs(ref) + acc), np.abs(got - ref).max()
 
 
+@pytest.mark.parametrize("dhw", [(2, 4, 32), (3, 5, 33), (5, 9, 70), (1, 1, 1)])
+@pytest.mark.parametrize("cins,cout", [((16,), 16), ((32, 16), 16), ((16, 32), 32), ((32,), 64)])
+def test_weight_gradient_tiles(cuda, dhw, cins, cout):
+    """Whole, partial and several 32 x 4 x 2 tiles against the float64 oracle; FP32 sums of exact products: at most
+    K 2^-24 of the sum of magnitudes over the K voxels."""
+    import torch
+    rng = np.random.default_rng(sum(dhw) + cout)
+    D, H, W = dhw
+    Xs = [U.bf16_round(rng.normal(size=(D, H, W, c))) for c in cins]
+    X, dY = np.concatenate(Xs, -1), U.bf16_round(rng.normal(size=(D, H, W, cout)))
+    xt, dyt = [_bf(torch, x, cuda) for x in Xs], _bf(torch, dY, cuda)
+    dw = torch.ones((27, cout, sum(cins)), dtype=torch.float32, device=cuda)
+    _lib.call("omg_conv3d_wgrad", _p(dyt), cout, _p(xt[0]), cins[0], _p(xt[1] if len(xt) > 1 else None),
+              cins[1] if len(cins) > 1 else 0, _p(dw), D, H, W, None)
+    ref, mag = U.conv3d_dw(dY, X), U.conv3d_dw(np.abs(dY), np.abs(X))
+    assert np.all(np.abs(dw.cpu().numpy() - 1.0 - ref) <= 2.0 ** -24 * (D * H * W + 2) * (mag + 1.0))
+
+
 def test_network_forward_and_gradients(cuda):
     import torch
     nx = ny = 8
