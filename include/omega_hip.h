@@ -296,6 +296,8 @@ int omg_conv3d_flipT(const uint16_t* W, uint16_t* Wf, int32_t Cout, int32_t Cin,
 int omg_bias_grad(const uint16_t* dY, float* db, int32_t V, int32_t C, void* stream);
 /* dY = 0 where Y <= 0. */
 int omg_relu_backward(const uint16_t* Y, uint16_t* dY, int64_t n, void* stream);
+/* omg_relu_backward, then omg_bias_grad of the masked gradient, in one pass (n = V C elements). */
+int omg_relu_bias_backward(const uint16_t* Y, uint16_t* dY, float* db, int32_t V, int32_t C, void* stream);
 /* 2x2x2 average pooling of the fine grid D x H x W and its adjoint ((+)= into dX). */
 int omg_pool_forward(const uint16_t* X, uint16_t* Y, int32_t D, int32_t H, int32_t W, int32_t C, void* stream);
 int omg_pool_backward(const uint16_t* dY, uint16_t* dX, int32_t D, int32_t H, int32_t W, int32_t C,

@@ -93,6 +93,7 @@ SIGNATURES = {
     "omg_conv3d_flipT": [_P, _P, _I32, _I32, _P],
     "omg_bias_grad": [_P, _P, _I32, _I32, _P],
     "omg_relu_backward": [_P, _P, _I64, _P],
+    "omg_relu_bias_backward": [_P, _P, _P, _I32, _I32, _P],
     "omg_pool_forward": [_P, _P, _I32, _I32, _I32, _I32, _P],
     "omg_pool_backward": [_P, _P, _I32, _I32, _I32, _I32, _I32, _P],
     "omg_upsample_forward": [_P, _P, _I32, _I32, _I32, _I32, _P],

@@ -558,6 +558,61 @@ __global__ void k_relu_bwd8(const uint4* __restrict__ Y, uint4* dY, size_t n8) {
     dY[i] = uint4{dw[0], dw[1], dw[2], dw[3]};
 }
 
+// k_relu_bwd8 and k_bias_grad8 in one pass: dY is masked by Y > 0 in place and its masked sums per channel are added
+// to db. Bound by the memory traffic, so four rows of 16 bytes per thread are in flight; two blocks per CU keep the atomics
+// onto the C sums few. The network's ten (128 x 128 x 64 voxels, 16 to 64
+// channels), mean: 14.5 us against 9.4 + 12.5 us apart.
+constexpr int kRbBatch = 4;
+__global__ __launch_bounds__(256) void k_relu_bias_bwd8(const uint16_t* __restrict__ Y, uint16_t* __restrict__ dY,
+                                                        float* __restrict__ db, int V, int C) {
+    __shared__ float part[2048];
+    const int g8 = C / 8, rows = 256 / g8;
+    const int r = threadIdx.x / g8, c8 = (threadIdx.x - r * g8) * 8;
+    const int64_t step = (int64_t)gridDim.x * rows;
+    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int64_t v0 = (int64_t)blockIdx.x * rows + r; v0 < V; v0 += step * kRbBatch) {
+        uint4 y[kRbBatch], d[kRbBatch];
+#pragma unroll
+        for (int k = 0; k < kRbBatch; k++) {
+            const int64_t v = v0 + k * step;
+            y[k] = d[k] = uint4{0u, 0u, 0u, 0u};
+            if (v < V) {
+                y[k] = *reinterpret_cast<const uint4*>(Y + (size_t)v * C + c8);
+                d[k] = *reinterpret_cast<const uint4*>(dY + (size_t)v * C + c8);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kRbBatch; k++) {
+            const int64_t v = v0 + k * step;
+            if (v >= V) break;
+            const uint32_t yw[4] = {y[k].x, y[k].y, y[k].z, y[k].w};
+            uint32_t dw[4] = {d[k].x, d[k].y, d[k].z, d[k].w};
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (!(bf2f((uint16_t)(yw[j] & 0xffffu)) > 0.f)) dw[j] &= 0xffff0000u;
+                if (!(bf2f((uint16_t)(yw[j] >> 16)) > 0.f)) dw[j] &= 0x0000ffffu;
+                s[2 * j] += bf2f((uint16_t)(dw[j] & 0xffffu));
+                s[2 * j + 1] += bf2f((uint16_t)(dw[j] >> 16));
+            }
+            *reinterpret_cast<uint4*>(dY + (size_t)v * C + c8) = uint4{dw[0], dw[1], dw[2], dw[3]};
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++) part[r * C + c8 + j] = s[j];   // rows * C == 2048
+    __syncthreads();
+    const int c = threadIdx.x % C, q = threadIdx.x / C, fold = 256 / C;
+    float t = 0.f;
+    for (int k = q; k < rows; k += fold) t += part[k * C + c];
+    __syncthreads();
+    part[threadIdx.x] = t;
+    __syncthreads();
+    if (threadIdx.x < C) {
+        float u = 0.f;
+        for (int k = 0; k < fold; k++) u += part[k * C + threadIdx.x];
+        unsafeAtomicAdd(db + threadIdx.x, u);
+    }
+}
+
 // Nearest 2x upsampling, 8 channels (16 bytes) per thread: grid = (ceil(W * C / 8 / 256), H, D) of the fine grid.
 __global__ void k_up_fwd8(const uint16_t* __restrict__ X, uint16_t* __restrict__ Y, Vol g, int C) {
     const int c8n = C / 8;
@@ -1076,6 +1131,18 @@ extern "C" int omg_relu_backward(const uint16_t* Y, uint16_t* dY, int64_t n, voi
                            reinterpret_cast<const uint4*>(Y), reinterpret_cast<uint4*>(dY), (size_t)n / 8);
     else if (n)
         hipLaunchKernelGGL(k_relu_bwd, dim3(blocks((size_t)n)), dim3(256), 0, as_stream(stream), Y, dY, (size_t)n);
+    OMG_CHECK_LAUNCH();
+    return OMG_OK;
+}
+
+extern "C" int omg_relu_bias_backward(const uint16_t* Y, uint16_t* dY, float* db, int32_t V, int32_t C, void* stream) {
+    OMG_REQUIRE(Y && dY && db && V > 0 && (C == 16 || C == 32 || C == 64), "needs V > 0, C in {16, 32, 64}");
+    if ((uintptr_t)Y % 16 || (uintptr_t)dY % 16) {
+        const int rc = omg_relu_backward(Y, dY, (int64_t)V * C, stream);
+        return rc ? rc : omg_bias_grad(dY, db, V, C, stream);
+    }
+    hipLaunchKernelGGL(k_relu_bias_bwd8, dim3((unsigned)std::min<int64_t>(512, ((int64_t)V * C + 8191) / 8192)), dim3(256),
+                       0, as_stream(stream), Y, dY, db, V, C);
     OMG_CHECK_LAUNCH();
     return OMG_OK;
 }

@@ -77,7 +77,10 @@ class UNet3D:
         params = init_params(seed) if params is None else params
         f32 = dict(dtype=torch.float32, device=device)
         self.p = {k: torch.as_tensor(np.ascontiguousarray(v), **f32) for k, v in params.items()}
-        self.g = {k: torch.zeros_like(v) for k, v in self.p.items()}
+        # gradients: views of one buffer (each on a 64-float boundary), so that one launch clears them
+        ends = np.cumsum([0] + [-(-v.numel() // 64) * 64 for v in self.p.values()])
+        self._g_all = torch.zeros(int(ends[-1]), **f32)
+        self.g = {k: self._g_all[int(o):int(o) + v.numel()].view(v.shape) for (k, v), o in zip(self.p.items(), ends)}
         self.m = {k: torch.zeros_like(v) for k, v in self.p.items()}
         self.v = {k: torch.zeros_like(v) for k, v in self.p.items()}
         self.wb = {}    # BF16 weights [27, cout, cin]
@@ -145,10 +148,10 @@ class UNet3D:
         c2 = cins[1] if len(cins) > 1 else 0
         _lib.call("omg_conv3d_wgrad", _p(dY), cout, _p(X1), cins[0], _p(X2), c2, _p(self.g[name + ".w"]),
                   self.D[l], self.H[l], self.W[l], self._s())
-        _lib.call("omg_bias_grad", _p(dY), _p(self.g[name + ".b"]), self.V[l], cout, self._s())
 
-    def _relu_bwd(self, Y, dY):
-        _lib.call("omg_relu_backward", _p(Y), _p(dY), dY.numel(), self._s())
+    def _relu_bwd(self, name, Y, dY):
+        """dY masked by layer ``name``'s output Y; the layer's bias gradient."""
+        _lib.call("omg_relu_bias_backward", _p(Y), _p(dY), _p(self.g[name + ".b"]), Y.shape[0], Y.shape[1], self._s())
 
     def _pool(self, X, Y, l, ch):
         _lib.call("omg_pool_forward", _p(X), _p(Y), self.D[l], self.H[l], self.W[l], ch, self._s())
@@ -185,8 +188,7 @@ class UNet3D:
         return a["out"]
 
     def zero_grad(self):
-        for g in self.g.values():
-            g.zero_()
+        self._g_all.zero_()
 
     def backward(self, gout):
         """Accumulates parameter gradients for d(loss)/d(out) = gout (FP32 [V0])."""
@@ -195,53 +197,53 @@ class UNet3D:
         g_d1 = a["g16_0"]
         _lib.call("omg_head_backward", _p(a["d1"]), _p(self.p["head.w"]), _p(gout), _p(g_d1), _p(self.g["head.w"]),
                   _p(self.g["head.b"]), V0, 16, self._s())
-        self._relu_bwd(a["d1"], g_d1)
+        self._relu_bwd("d1b", a["d1"], g_d1)
         self._wgrad("d1b", g_d1, a["a5"])
         g_a5 = a["g16_0b"]
         self._conv_dx("d1b", g_d1, g_a5)
-        self._relu_bwd(a["a5"], g_a5)
+        self._relu_bwd("d1a", a["a5"], g_a5)
         self._wgrad("d1a", g_a5, a["u1"], a["s1"])
         g_cat1 = a["g48_0"]
         self._conv_dx("d1a", g_a5, g_cat1)
         g_d2 = a["g32_1"]
         _lib.call("omg_upsample_backward", _p(g_cat1), 48, 0, _p(g_d2), self.D[1], self.H[1], self.W[1], 32, self._s())
-        self._relu_bwd(a["d2"], g_d2)
+        self._relu_bwd("d2b", a["d2"], g_d2)
         self._wgrad("d2b", g_d2, a["a4"])
         g_a4 = a["g32_1b"]
         self._conv_dx("d2b", g_d2, g_a4)
-        self._relu_bwd(a["a4"], g_a4)
+        self._relu_bwd("d2a", a["a4"], g_a4)
         self._wgrad("d2a", g_a4, a["u2"], a["s2"])
         g_cat2 = a["g96_1"]
         self._conv_dx("d2a", g_a4, g_cat2)
         g_b3 = a["g64_2"]
         _lib.call("omg_upsample_backward", _p(g_cat2), 96, 0, _p(g_b3), self.D[2], self.H[2], self.W[2], 64, self._s())
-        self._relu_bwd(a["b3"], g_b3)
+        self._relu_bwd("btb", a["b3"], g_b3)
         self._wgrad("btb", g_b3, a["a3"])
         g_a3 = a["g64_2b"]
         self._conv_dx("btb", g_b3, g_a3)
-        self._relu_bwd(a["a3"], g_a3)
+        self._relu_bwd("bta", a["a3"], g_a3)
         self._wgrad("bta", g_a3, a["p2"])
         g_p2 = a["g32_2"]
         self._conv_dx("bta", g_a3, g_p2)
         g_s2 = a["g32_1"]   # g_d2 is consumed
         _lib.call("omg_pool_backward", _p(g_p2), _p(g_s2), self.D[1], self.H[1], self.W[1], 32, 0, self._s())
         _lib.call("omg_take_channels", _p(g_cat2), 96, 64, _p(g_s2), self.V[1], 32, 1, self._s())
-        self._relu_bwd(a["s2"], g_s2)
+        self._relu_bwd("e2b", a["s2"], g_s2)
         self._wgrad("e2b", g_s2, a["a2"])
         g_a2 = a["g32_1b"]
         self._conv_dx("e2b", g_s2, g_a2)
-        self._relu_bwd(a["a2"], g_a2)
+        self._relu_bwd("e2a", a["a2"], g_a2)
         self._wgrad("e2a", g_a2, a["p1"])
         g_p1 = a["g16_1"]
         self._conv_dx("e2a", g_a2, g_p1)
         g_s1 = a["g16_0"]   # g_d1 is consumed
         _lib.call("omg_pool_backward", _p(g_p1), _p(g_s1), self.D[0], self.H[0], self.W[0], 16, 0, self._s())
         _lib.call("omg_take_channels", _p(g_cat1), 48, 32, _p(g_s1), V0, 16, 1, self._s())
-        self._relu_bwd(a["s1"], g_s1)
+        self._relu_bwd("e1b", a["s1"], g_s1)
         self._wgrad("e1b", g_s1, a["a1"])
         g_a1 = a["g16_0b"]
         self._conv_dx("e1b", g_s1, g_a1)
-        self._relu_bwd(a["a1"], g_a1)
+        self._relu_bwd("e1a", a["a1"], g_a1)
         self._wgrad("e1a", g_a1, a["x0"])
 
     def loss(self, target, mask, scale: float):

@@ -127,6 +127,23 @@ def test_weight_gradient_tiles(cuda, dhw, cins, cout):
     assert np.all(np.abs(dw.cpu().numpy() - 1.0 - ref) <= 2.0 ** -24 * (D * H * W + 2) * (mag + 1.0))
 
 
+@pytest.mark.parametrize("V,C", [(1, 16), (1000, 16), (8193, 32), (70001, 64), (300000, 16)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_relu_bias_backward(cuda, V, C, shift):
+    """Mask and bias gradient in one pass: the mask exactly, the sums within V 2^-24 of the sum of magnitudes;
+    ``shift``: pointers that are not 16-byte aligned."""
+    import torch
+    g = torch.Generator(device=cuda).manual_seed(V)
+    Y, dY = (torch.randn(V * C + 8, device=cuda, generator=g).bfloat16() for _ in range(2))
+    y, d = Y[shift:shift + V * C], dY[shift:shift + V * C]
+    ref = torch.where(y > 0, d, torch.zeros_like(d))
+    db = torch.ones(C, device=cuda)
+    _lib.call("omg_relu_bias_backward", _p(y), _p(d), _p(db), V, C, None)
+    assert torch.equal(d, ref)
+    r = ref.double().view(V, C)
+    assert torch.all((db.double() - 1.0 - r.sum(0)).abs() <= 2.0 ** -24 * (V + 2) * (r.abs().sum(0) + 1.0))
+
+
 def test_network_forward_and_gradients(cuda):
     import torch
     nx = ny = 8
