@@ -15,10 +15,10 @@
 // products in double and rounds once.
 //
 // Measured on a 128 x 128 x 63 image, 128 x 160 bins, 8 planes per subset, one subset step (with the sensitivity
-// image / without; the kernels before it in brackets): Siddon 61 / 58 us (141 / 92: slices and accumulators in
-// LDS), with 17 TOF bins 408 us (5968: one lane per LOR, every plane's bin weights evaluated twice), orthogonal
-// 84 / 81 us (964 / 655: tube lists of every plane), interpolation 94 / 78 us (589 / 384). Odd 109 x 97 image,
-// 8 planes of 142 x 91 bins, with prior: 53 us (478: global atomics). The lists take 50 MB (TOF: 340 MB) and are
+// image / without; the kernels before it in brackets): Siddon 55 / 52 us (141 / 92: slices and accumulators in
+// LDS), with 17 TOF bins 362 us (5968: one lane per LOR, every plane's bin weights evaluated twice), orthogonal
+// 73 / 71 us (964 / 655: tube lists of every plane), interpolation 89 / 72 us (589 / 384). Odd 109 x 97 image,
+// 8 planes of 142 x 91 bins, with prior: 50 us (478: global atomics). The lists take 50 MB (TOF: 340 MB) and are
 // built in 0.8 ms (TOF: 2.6 ms), less than the steps of one full iteration save.
 #include "plane.hpp"
 #include "geom.hpp"
@@ -199,15 +199,21 @@ __global__ __launch_bounds__(kPB) void k_plane_fp(PlaneRun a, const float* __res
     } else {
         const uint2* e = a.ent + a.off[g] + row % kLI;
         const uint32_t n = a.len[g];
-        for (uint32_t k = 0; k < n; k += kLUnroll) {
-            uint2 q[kLUnroll];
-            float v[kLUnroll];
+        uint2 q[kLUnroll];
+        float v[kLUnroll];
 #pragma unroll
-            for (uint32_t j = 0; j < kLUnroll; j++) q[j] = e[(k + j) * kLI];
+        for (uint32_t j = 0; j < kLUnroll; j++) q[j] = n ? e[j * kLI] : uint2{0u, 0u};
+        for (uint32_t k = 0; k < n; k += kLUnroll) {
+            uint2 qn[kLUnroll];
+            const uint32_t kn = k + kLUnroll < n ? k + kLUnroll : k;   // the next entries load behind the voxels
 #pragma unroll
             for (uint32_t j = 0; j < kLUnroll; j++) v[j] = X[(size_t)q[j].x * PL];
 #pragma unroll
+            for (uint32_t j = 0; j < kLUnroll; j++) qn[j] = e[(kn + j) * kLI];
+#pragma unroll
             for (uint32_t j = 0; j < kLUnroll; j++) ax += __uint_as_float(q[j].y) * v[j];
+#pragma unroll
+            for (uint32_t j = 0; j < kLUnroll; j++) q[j] = qn[j];
         }
     }
     const bool in = a.slice[plane] >= 0;
@@ -296,7 +302,8 @@ __global__ __launch_bounds__(kPB) void k_plane_tof(PlaneRun a, uint32_t chunk, u
     }
 }
 
-// Sums of one pixel list: rhs of length * R (or of T, TOF), sens of length * W.
+// Sums of one pixel list: rhs of length * R (or of T, TOF), sens of length * W. The entries of the next batch load
+// while the values of this one arrive (they are the chain's two links): 28 -> 23 us without sens, TOF 98 -> 53 us.
 template <int PL, bool TOF, bool SENS>
 __device__ __forceinline__ void plane_sums(const PlaneRun& a, uint32_t pix, const float* __restrict__ R,
                                            const float* __restrict__ W, double& rhs, double& sens) {
@@ -304,22 +311,36 @@ __device__ __forceinline__ void plane_sums(const PlaneRun& a, uint32_t pix, cons
     const size_t o = (size_t)a.coff[g] + pix % kLI;
     const uint2* e = a.cent + o;
     const uint32_t* ep = TOF ? a.cpos + o : nullptr;
-    for (uint32_t k = 0; k < n; k += kLUnroll) {
-        uint2 q[kLUnroll];
-        float v[kLUnroll], u[kLUnroll];
-#pragma unroll
-        for (uint32_t j = 0; j < kLUnroll; j++)
-            if (!TOF || SENS) q[j] = e[(k + j) * kLI];
+    uint2 q[kLUnroll];
+    uint32_t at[kLUnroll];
+    auto fetch = [&](uint32_t k, uint2 (&qq)[kLUnroll], uint32_t (&aa)[kLUnroll]) {
 #pragma unroll
         for (uint32_t j = 0; j < kLUnroll; j++) {
-            v[j] = TOF ? R[(size_t)ep[(k + j) * kLI] * PL] : R[(size_t)q[j].x * PL];
+            if (!TOF || SENS) qq[j] = e[(k + j) * kLI];
+            if (TOF) aa[j] = ep[(k + j) * kLI];
+        }
+    };
+    if (n) fetch(0, q, at);
+    for (uint32_t k = 0; k < n; k += kLUnroll) {
+        uint2 qn[kLUnroll];
+        uint32_t an[kLUnroll];
+        float v[kLUnroll], u[kLUnroll];
+#pragma unroll
+        for (uint32_t j = 0; j < kLUnroll; j++) {
+            v[j] = R[(size_t)(TOF ? at[j] : q[j].x) * PL];
             if (SENS) u[j] = W[(size_t)q[j].x * PL];
         }
+        fetch(k + kLUnroll < n ? k + kLUnroll : k, qn, an);   // the next entries load behind the values
 #pragma unroll
         for (uint32_t j = 0; j < kLUnroll; j++) {
             if (TOF) rhs += (double)v[j];
             else rhs = __builtin_fma((double)__uint_as_float(q[j].y), (double)v[j], rhs);
             if (SENS) sens = __builtin_fma((double)__uint_as_float(q[j].y), (double)u[j], sens);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kLUnroll; j++) {
+            if (!TOF || SENS) q[j] = qn[j];
+            if (TOF) at[j] = an[j];
         }
     }
 }
