@@ -301,7 +301,7 @@ enum { COL_FP = 0, COL_OSEM = 1, COL_BP = 2 };
 // 217 us; 383 us with gathers (16 clocks of the texture address unit each, two per column) and 484 us by one lane per
 // LOR.
 template <int MODE, int BPW, int NR>
-__global__ __launch_bounds__(256, MODE == COL_FP && NR < 2 ? 6 : 4) void k_col_fp(
+__global__ __launch_bounds__(256, MODE == COL_BP || NR > 1 ? 4 : MODE == COL_FP ? 6 : 5) void k_col_fp(
     ColView c, SidArgs a, uint32_t plane0, const float* __restrict__ Xz, const float* __restrict__ yin,
     float* __restrict__ yout, float4* __restrict__ rec, float* __restrict__ wrec, uint32_t* __restrict__ state,
     uint32_t* __restrict__ rest, float epps) {
