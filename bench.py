@@ -6,10 +6,10 @@ Workload (one "step"): a full OSEM reconstruction of the 2-D plane PET data set 
 resident in device memory. value = 32 * steps / wall-seconds of the timed region.
 
 Also reported:
-  roofline      for the dominant kernel (the fused FP/ratio/BP projector launch of iterations >= 1):
-                algorithmic bytes per launch / its average duration, timed with HIP events on the
+  roofline      for the projector launches of a subset step of iterations >= 1 (FP, ratio, BP, update):
+                algorithmic bytes per step / their average duration, timed with HIP events on the
                 launch stream inside the timed region (the library's omg_timing_* hooks).
-                Algorithmic bytes of one such launch = 4 * sum(Np) + 8 * sum(Np, y != 0) + 8 * M_k (4 B gather
+                Algorithmic bytes of one such step = 4 * sum(Np) + 8 * sum(Np, y != 0) + 8 * M_k (4 B gather
                 of x per intersected voxel, 8 B read-modify-write of rhs per voxel of the LORs with counts --
                 a zero ratio is not backprojected --, 4 B measurement + 4 B LOR table per LOR);
                 sum(Np) = exact count of (LOR, voxel) intersections with length > 0.
@@ -32,8 +32,6 @@ if ROOT not in sys.path:
 
 METRIC = "OSEM subset-iters/s; wall-time to plain 40-iter log-lik, learned vs plain"
 HBM_PEAK_GBS = 8000.0
-EXP64_INSTS = 19                                 # FP64 VALU instructions of exp(double) on gfx950
-EXP64_PEAK = 78.6e12 / 2 / EXP64_INSTS          # exp(double) per second at the FP64 vector rate
 
 
 def parse():
@@ -43,9 +41,9 @@ def parse():
     ap.add_argument("--warmup", type=int, default=3)
     ap.add_argument("--cpu-seconds", type=float, default=15.0, help="budget of the CPU baseline sample")
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline leg")
-    ap.add_argument("--traffic", default=os.path.join(ROOT, "profiles", "siddon_planar_pet2d_traffic.txt"),
+    ap.add_argument("--traffic", default=os.path.join(ROOT, "profiles", "plane_lists_pet2d_traffic.txt"),
                     help="summary of the rocprofv3 --pmc HBM traffic of the dominant kernel, if present")
-    ap.add_argument("--issue", default=os.path.join(ROOT, "profiles", "siddon_planar_pet2d_issue.txt"),
+    ap.add_argument("--issue", default=os.path.join(ROOT, "profiles", "plane_lists_pet2d_issue.txt"),
                     help="summary of the rocprofv3 --pmc VALU issue counters of the dominant kernel, if present")
     ap.add_argument("--workload", default="pet2d_osem",
                     choices=["pet2d_osem", "pet3d_frames", "ct_cgls_bdd", "pet2d_orth", "pet2d_volume", "pet3d_autograd",
@@ -144,15 +142,15 @@ def main():
     value = sub_iters * args.steps / dt
     _lib.call("omg_timing_collect", C.byref(tot), C.byref(cnt))
 
-    # dominant kernel: the fused FP -> ratio -> BP projector launch(es) of iterations >= 1, timed with HIP
-    # events on their stream: k_siddon_planar<640, true, true, false> (LDS-atomic BP, the default) or,
-    # opted in, k_planar_fpq + k_planar_vbp (voxel-driven BP, ring sinograms)
+    # the subset step's launches of iterations >= 1 (FP -> ratio -> BP -> update), timed together with HIP events
+    # on their stream: from the shared plane's lists (the default) or, opted in, k_planar_fpq + k_planar_vbp
+    # (voxel-driven BP, ring sinograms)
     kernel_name = "k_planar_fpq<640,false> + k_planar_vbp<false,false>" if args.voxel_bp else \
-        "k_siddon_planar<640,true,true,false>"
+        "k_plane_gather + k_plane_fp + k_plane_bp (with the update)"
     avg_s = tot.value * 1e-3 / max(cnt.value, 1)
     bytes_per_launch = float(np.mean([4.0 * np_sum[k] + 8.0 * np_nz[k] + 8.0 * M[k] for k in range(p.subsets)]))
     achieved = bytes_per_launch / avg_s / 1e9
-    traffic = None if args.voxel_bp else read_traffic(args.traffic)   # the summary covers the LDS kernel
+    traffic = None if args.voxel_bp else read_traffic(args.traffic)   # the summary covers the list kernels
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
                 "kernel": kernel_name, "launches_timed": int(cnt.value),
@@ -304,7 +302,7 @@ def bench_frames(args):
                    "data_gen_s": round(t_data, 1), "tune_s": round(t_tune, 1)},
         "roofline": {"bound": "hbm", "achieved": round(bytes_step / step_s / 1e9, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(bytes_step / step_s / 1e9 / HBM_PEAK_GBS, 4), "traffic": None,
-                     "kernel": f"k_frames_osem<{ft},{rpb}> + k_frames_update", "avg_launch_us": round(step_s * 1e6, 1),
+                     "kernel": "k_col_fp + k_col_bp of every frame + k_frames_update", "avg_launch_us": round(step_s * 1e6, 1),
                      "algorithmic_bytes_per_launch": int(bytes_step)},
         "serial_frames_subset_step_ms": round(serial_step_s * 1e3, 2),
         "batched_subset_step_ms": round(step_s * 1e3, 2),
@@ -507,7 +505,7 @@ def bench_orth(args, volume=False, tof=False):
     elif volume:
         kern = "k_tube_vol_planar (tube lists kept on the device) + update"
     else:
-        kern = "k_orth_osem + update"
+        kern = "k_plane_fp + k_plane_bp (lists of one plane, shared by all) + update"
     _common(args, {
         "metric": "OSEM subset-iters/s, " + ("volume-of-intersection" if volume else "orthogonal distance-based")
                   + " projector" + (" with TOF" if tof else ""), "value": round(p.subsets * args.steps / dt, 2),
@@ -612,7 +610,7 @@ def bench_interp(args, tof=False):
         "roofline": {"bound": "hbm", "achieved": round(byt / s_s / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(byt / s_s / 1e9 / HBM_PEAK_GBS, 4), "traffic": None,
                      "kernel": ("k_interp_tof_fp + ratio + k_interp_tof_bp + update" if tof
-                                else "k_interp_fp_planar + ratio + k_interp_bp_planar (slices in LDS) + update"),
+                                else "k_plane_fp + k_plane_bp (lists of one plane, shared by all) + update"),
                      "avg_launch_us": round(s_s * 1e6, 1), "algorithmic_bytes_per_launch": int(byt)},
         "cpu_baseline": cpu,
     })
@@ -621,9 +619,8 @@ def bench_interp(args, tof=False):
 def bench_tof(args):
     """2-D plane PET OSEM with time of flight and attenuation on the pet2d_osem geometry: 17 TOF bins of
     140 ps (400 ps FWHM), a water cylinder (0.0096 / mm, radius 120 mm) as attenuation image.
-    value = subset-iterations/s (8 subsets x 1 iteration per step). The TOF kernels are bound by the
-    Gaussian's double-precision exponentials (3 per bin and voxel visit: the trapezoid's last point is
-    the next voxel's first), reported as exps/s."""
+    value = subset-iterations/s (8 subsets x 1 iteration per step). The bins' shares of
+    each voxel are kept with the shared plane's lists, so a step streams them and evaluates no exponential."""
     import ctypes as C
     import numpy as np
     import torch
@@ -669,7 +666,6 @@ def bench_tof(args):
     b.record()
     b.synchronize()
     s_s = a.elapsed_time(b) * 1e-3
-    exps = 2.0 * 3.0 * p.nBins * ntr
     byt = 12.0 * ntr + 8.0 * M0 * p.nBins
     cpu = None
     if not args.no_cpu:
@@ -687,14 +683,10 @@ def bench_tof(args):
         # bound: the double-precision exponentials. exp(double) compiles for gfx950 to 19 FP64 VALU
         # instructions (13 FMA, mul, rndne, ldexp, cvt, 2 compares); at the FP64 vector rate of 78.6 TFLOP/s
         # (39.3 T lane-instructions/s) that is 2.07e12 exp/s with no other work
-        "roofline": {"bound": "fp64", "achieved": round(exps / s_s / 1e9, 1), "peak": round(EXP64_PEAK / 1e9, 1),
-                     "unit": "G exp/s", "frac": round(exps / s_s / EXP64_PEAK, 4), "traffic": None,
-                     "peak_basis": f"78.6 TFLOP/s FP64 / 2 = 39.3e12 lane-instructions/s over {EXP64_INSTS} "
-                                   "FP64 instructions per exp(double)",
-                     "kernel": "k_tof_osem + update", "avg_launch_us": round(s_s * 1e6, 1),
-                     "exps_per_launch": int(exps),
-                     "hbm": {"algorithmic_bytes_per_launch": int(byt), "achieved": round(byt / s_s / 1e9, 1),
-                             "frac": round(byt / s_s / 1e9 / HBM_PEAK_GBS, 4)}},
+        "roofline": {"bound": "hbm", "achieved": round(byt / s_s / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                     "frac": round(byt / s_s / 1e9 / HBM_PEAK_GBS, 4), "traffic": None,
+                     "kernel": "k_plane_tof + k_plane_bp + update", "avg_launch_us": round(s_s * 1e6, 1),
+                     "algorithmic_bytes_per_launch": int(byt)},
         "cpu_baseline": cpu,
     })
 
@@ -780,7 +772,7 @@ def bench_autograd(args):
         "fd_voxels": 64, "fd_h": h, "fd_max_rel_error": max(errs), "fd_median_rel_error": float(np.median(errs)),
         "roofline": {"bound": "hbm", "achieved": round(byt / dt / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(byt / dt / 1e9 / HBM_PEAK_GBS, 4), "traffic": None,
-                     "kernel": "forward + backward projection of the pass (k_siddon_* )",
+                     "kernel": "forward + backward projection of the pass (k_col_fp + k_col_bp)",
                      "avg_launch_us": round(dt * 1e6, 1), "algorithmic_bytes_per_launch": int(byt),
                      "visits": visits},
         "cpu_baseline": cpu,
