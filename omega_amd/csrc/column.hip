@@ -704,10 +704,12 @@ static uint32_t col_tpb(uint32_t tw, uint32_t th, uint32_t Nz) {
 static bool col_build(const omg_geom* g, ColPlan* p, hipStream_t s) {
     const omg_geom_desc& d = g->d;
     const uint32_t per = d.size_x * d.size_y;
-    if (!col_tile_size(d.Nz, &p->tw, &p->th) ||
-        hipFuncSetAttribute(reinterpret_cast<const void*>(k_col_bp), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)kColLds) != hipSuccess)
+    if (!col_tile_size(d.Nz, &p->tw, &p->th)) return false;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(k_col_bp), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)kColLds) != hipSuccess) {
+        (void)hipGetLastError();
         return false;
+    }
     p->ntx = (d.Nx + p->tw - 1) / p->tw;
     const uint32_t tiles = p->ntx * ((d.Ny + p->th - 1) / p->th);
     uint32_t *cnt = nullptr, *tile_cnt = nullptr, *tile_off = nullptr;
@@ -795,18 +797,18 @@ static bool col_build(const omg_geom* g, ColPlan* p, hipStream_t s) {
     return ok;
 }
 
-const ColPlan* col_plan(const omg_geom* gc, int64_t first, int64_t n, hipStream_t s) {
+const ColPlan* col_plan(const omg_geom* gc, int64_t first, int64_t n, hipStream_t s, uint32_t min_planes) {
     omg_geom* g = const_cast<omg_geom*>(gc);
     const omg_geom_desc& d = g->d;
-    // fewer planes than half a wave leave most lanes idle; without the ring property a walk's lengths need the
-    // general expression; the records hold z in 15 bits and the steps left in 16
+    // few planes leave lanes idle (min_planes); without the ring property a walk's lengths need the general expression;
+    // the records hold z in 15 bits and the steps left in 16
     if (d.mode != OMG_MODE_PET_SINO || d.projector_type != OMG_PROJ_SIDDON || d.tof_bins > 1 || g->force_generic ||
-        d.reserved[3] != 0 || d.reserved[4] < 0 || !g->ring || d.n_proj < 32 ||
+        d.reserved[3] != 0 || d.reserved[4] < 0 || !g->ring || d.n_proj < min_planes ||
         (uint64_t)d.Nx + d.Ny + d.Nz + 3 > 65535 || d.Nz > 32000 || n > 0xffffffffll ||
         (uint64_t)std::max(d.rays_xy, 1u) * std::max(d.rays_z, 1u) != 1)
         return nullptr;
     const uint64_t per = (uint64_t)d.size_x * d.size_y;
-    if (!g->index_dev && ((uint64_t)n < 32 * per || (uint64_t)n % per)) return nullptr;
+    if (!g->index_dev && ((uint64_t)n < min_planes * per || (uint64_t)n % per)) return nullptr;
     if (!g->columns) {
         if (fixed_region_active()) return nullptr;
         g->columns = new ColCache();

@@ -446,7 +446,7 @@ extern "C" int omg_frames_sensitivity(const omg_geom* g, int64_t first, int64_t 
     OMG_CHECK_LAUNCH();
     if (n_meas > 0) {
         bool done = false;
-        if (const ColPlan* pl = col_plan(g, first, n_meas, s)) {
+        if (const ColPlan* pl = col_plan(g, first, n_meas, s, kColPlanesBack)) {
             const int rc = col_backward(g, pl, first, n_meas, nullptr, S, nullptr, s, &done);
             if (rc) return rc;
         }

@@ -797,7 +797,7 @@ extern "C" int omg_backward_project(const omg_geom* g, int64_t first, int64_t n_
         return launch_planar<false, true, false>(g, first, n_meas, nullptr, y, nullptr, rhs, nullptr, 0.f, s);
     }
     if (g->d.tof_bins > 1) return tof_backward(g, first, n_meas, y, rhs, sens, s);
-    if (const ColPlan* pl = col_plan(g, first, n_meas, s)) {
+    if (const ColPlan* pl = col_plan(g, first, n_meas, s, kColPlanesBack)) {
         bool done = false;
         rc = col_backward(g, pl, first, n_meas, y, rhs, sens, s, &done);
         if (rc || done) return rc;

@@ -5,7 +5,8 @@ backprojection adds the same products in 64-bit fixed point where the other kern
 most ~5e3 terms per voxel: 2^-24 sqrt(5e3) = 4e-6 relative L2; bar 2e-5. A length between two crossings carries the
 rounding of their parameters, 2^-24 of a LOR of up to ~150 mm (1e-5 mm) each: the updated image is compared where the
 sensitivity is at least 0.5 mm, so that a voxel's own error stays below the bar. Images of one, two and more than two
-registers of slices per lane, odd, non-square and smaller than a tile; plane counts around the 64 of a wave; planes
+registers of slices per lane, odd, non-square and smaller than a tile; plane counts around the 64 of a wave, and below the 32 where
+only the backprojection goes by columns; planes
 far steeper than a voxel, outside the image, and leaving it through an end face.
 """
 import ctypes as C
@@ -51,7 +52,7 @@ def _run(geom, grid, first, n, img, y, meas):
 @pytest.mark.parametrize("nx,ny,nz,n_radial,n_angles,planes,first,dz", [
     (20, 20, 9, 24, 20, 32, 0, 2.5), (33, 21, 15, 29, 23, 63, 1, 2.5), (7, 5, 63, 11, 9, 64, 0, 2.5),
     (17, 18, 64, 19, 16, 65, 0, 1.0), (16, 32, 127, 20, 12, 40, 0, 0.7), (16, 16, 128, 20, 12, 70, 2, 0.6),
-    (3, 3, 301, 8, 6, 129, 0, 0.3), (40, 40, 2, 32, 32, 130, 0, 9.0)])
+    (3, 3, 301, 8, 6, 129, 0, 0.3), (20, 18, 11, 24, 20, 12, 1, 2.5), (20, 18, 11, 24, 20, 31, 0, 2.5), (40, 40, 2, 32, 32, 130, 0, 9.0)])
 def test_column(cuda, nx, ny, nz, n_radial, n_angles, planes, first, dz):
     import torch
     grid, x, z = _scanner(nx, ny, nz, n_radial, n_angles, planes + first, dz)
