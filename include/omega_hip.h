@@ -145,6 +145,9 @@ const char* omg_last_error(void);
  * device buffers ProjectorClass::createBuffers makes (source/cpp/ProjectorClass.h). */
 int omg_geom_create(const omg_geom_desc* desc, omg_geom** out);
 int omg_geom_destroy(omg_geom* g);
+/* Calls on g so far (frames counted one by one) that ran from the direct-plane lists and from the transaxial
+ * crossing lists (reserved[4] above); every other call traced its LORs. Either pointer may be NULL. */
+int omg_geom_list_calls(const omg_geom* g, int64_t* plane_calls, int64_t* column_calls);
 
 /* Forward projection y = A_k x for measurements [first, first + n_meas) of the
  * subset-ordered data: first is the subset's first plane/projection (list mode: LOR).

@@ -71,6 +71,7 @@ _U32 = C.c_uint32
 SIGNATURES = {
     "omg_geom_create": [C.POINTER(GeomDesc), C.POINTER(_P)],
     "omg_geom_destroy": [_P],
+    "omg_geom_list_calls": [_P, C.POINTER(C.c_int64), C.POINTER(C.c_int64)],
     "omg_forward_project": [_P, _I64, _I64, _P, _P, _P],
     "omg_backward_project": [_P, _I64, _I64, _P, _P, _P, _P],
     "omg_osem_data_step": [_P, _I64, _I64, _P, _P, _P, _P, _F, _P],

@@ -341,6 +341,13 @@ void bdd_release(omg_geom* g);
 void orth_release(omg_geom* g);
 void vbp_release(omg_geom* g);
 
+extern "C" int omg_geom_list_calls(const omg_geom* g, int64_t* plane_calls, int64_t* column_calls) {
+    OMG_REQUIRE(g != nullptr, "null geometry handle");
+    if (plane_calls) *plane_calls = g->plane_calls.load(std::memory_order_relaxed);
+    if (column_calls) *column_calls = g->column_calls.load(std::memory_order_relaxed);
+    return OMG_OK;
+}
+
 extern "C" int omg_geom_destroy(omg_geom* g) {
     if (!g) return OMG_OK;
     hipFree(g->x_dev);

@@ -901,6 +901,7 @@ static int col_run(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t 
         if (rc) return rc;
     }
     *done = true;
+    g->column_calls.fetch_add(1, std::memory_order_relaxed);
     float* Xz = work ? work : scratch_ptr(g);
     float4* rec = reinterpret_cast<float4*>(Xz + w.nimg);
     float* wrec = sens ? Xz + w.nimg + w.nrec : nullptr;

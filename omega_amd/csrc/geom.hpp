@@ -3,6 +3,7 @@
 #include "common.hpp"
 #include "siddon_device.hpp"
 
+#include <atomic>
 #include <vector>
 
 namespace omg { struct PlanePlan; struct ColCache; }
@@ -44,6 +45,8 @@ struct omg_geom {
     omg::PlanePlan* plane = nullptr;
     // 3-D sinograms: the transaxial crossing lists of column.hip, per measurement range used with an index table.
     omg::ColCache* columns = nullptr;
+    // Calls that ran from either kind of list (omg_geom_list_calls).
+    mutable std::atomic<int64_t> plane_calls{0}, column_calls{0};
     // Workgroups per plane for the planar kernels (omg_geom_desc.reserved[1]; 0 = automatic).
     int32_t planar_groups = 0;
     // Library-owned scratch (floats) for partial images; grown on demand, freed with the handle.

@@ -622,6 +622,7 @@ static int run_planes(omg_geom* g, const PlanePlan* pl, const PlaneRun& a, const
     int rc = scratch_reserve(g, need);
     if (rc) return rc;
     *done = true;
+    g->plane_calls.fetch_add(1, std::memory_order_relaxed);
     float* Xt = scratch_ptr(g);
     float* R = Xt + xt;
     float* W = R + (tof ? tt : rr);

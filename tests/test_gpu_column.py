@@ -15,7 +15,7 @@ import numpy as np
 import pytest
 
 from omega_amd import _lib, geometry as G
-from tests.hip_helpers import make_geom, ptr, rel_l2
+from tests.hip_helpers import list_calls, make_geom, ptr, rel_l2
 
 pytestmark = pytest.mark.gpu
 EPPS = 1e-5
@@ -61,8 +61,9 @@ def test_column(cuda, nx, ny, nz, n_radial, n_angles, planes, first, dz):
     norm = rng.random(n_radial * n_angles * (planes + first)).astype(np.float32) + 0.5
     up = lambda a: torch.from_numpy(a.astype(np.float32)).cuda()
     img, y, meas = up(rng.random(grid.N) + 0.5), up(rng.standard_normal(n)), up(rng.poisson(2.0, n))
-    a, b = (_run(make_geom(grid, x, z, n_radial, n_angles, generic=gen, norm=norm, global_factor=0.9), grid, first, n,
-                 img, y, meas) for gen in (False, True))
+    geoms = [make_geom(grid, x, z, n_radial, n_angles, generic=gen, norm=norm, global_factor=0.9) for gen in (False, True)]
+    a, b = (_run(g, grid, first, n, img, y, meas) for g in geoms)
+    assert [list_calls(g) for g in geoms] == [(0, 4 if planes >= 32 else 1), (0, 0)]
     seen = b[4] > 0.5
     assert seen.any()
     a[3], b[3] = a[3][seen], b[3][seen]
@@ -70,6 +71,44 @@ def test_column(cuda, nx, ny, nz, n_radial, n_angles, planes, first, dz):
     print(f"[column] {nx}x{ny}x{nz} planes={planes} rel-L2 {e}", flush=True)
     assert np.array_equal(a[0], b[0])
     assert max(e[1:]) < BAR
+
+
+def test_several_passes(cuda):
+    """140 planes of 224 x 224 bins: their records take two passes of plane groups, each with LORs off the lists. About
+    1e5 terms per voxel, so the float atomics of the other kernels carry 2^-24 sqrt(1e5) = 2e-5; bar: four times that."""
+    import torch
+    grid, x, z = _scanner(20, 20, 9, 224, 224, 140)
+    n = 140 * 224 * 224
+    rng = np.random.default_rng(4)
+    img = torch.from_numpy((rng.random(grid.N) + 0.5).astype(np.float32)).cuda()
+    y, meas = torch.rand(n, device="cuda") - 0.3, torch.poisson(torch.full((n,), 2.0, device="cuda"))
+    geoms = [make_geom(grid, x, z, 224, 224, generic=gen) for gen in (False, True)]
+    a, b = (_run(g, grid, 0, n, img, y, meas) for g in geoms)
+    assert list_calls(geoms[0]) == (0, 4)
+    assert np.array_equal(a[0], b[0])
+    e = [rel_l2(p, q) for p, q in zip(a[1:], b[1:])]
+    print(f"[column] two passes rel-L2 {e}", flush=True)
+    assert max(e) < 8e-5
+
+
+def test_many_ranges_and_off(cuda):
+    """An index table of 66 ranges keeps 64 lists and traces the others; reserved[3] and reserved[4] < 0 trace all."""
+    import torch
+    planes, per, k = 40, 66 * 7, 66
+    grid, x, z = _scanner(20, 20, 9, 22, 21, planes)
+    bins = np.random.default_rng(5).permutation(per).reshape(k, 7)
+    index = (np.arange(planes)[None, :, None] * per + bins[:, None, :]).astype(np.uint32).ravel()
+    img = torch.rand(grid.N, device="cuda") + 0.5
+    n = planes * 7
+    out = []
+    for kw in ({}, {"generic": True}, {"x_fastest_only": True}, {"tube_budget_mib": -1}):
+        g = make_geom(grid, x, z, 22, 21, meas_index=index, **kw)
+        y = torch.empty(k * n, device="cuda")
+        for s in range(k):
+            _lib.call("omg_forward_project", g.handle, s * n, n, ptr(img), ptr(y[s * n:]), None)
+        out.append(y.cpu().numpy())
+        assert list_calls(g) == (0, 0 if kw else 64)
+        assert np.array_equal(out[-1], out[0])
 
 
 def test_not_finite(cuda):
@@ -125,6 +164,7 @@ def test_frames(cuda, frames, planes):
             rhs.fill_(7.0)
         _lib.call("omg_graph_destroy", h)
         out.append(res + [xs.cpu().numpy()])
+        assert list_calls(g) == (0, 0 if gen else 1 + 4 * frames)   # sensitivity, two steps, forward, captured step
     a, b = out
     assert np.array_equal(a[2], b[2])
     seen = b[0] > 0.5

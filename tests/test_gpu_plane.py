@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 from omega_amd import _lib, geometry as G
-from tests.hip_helpers import make_geom, ptr, rel_l2
+from tests.hip_helpers import list_calls, make_geom, ptr, rel_l2
 
 pytestmark = pytest.mark.gpu
 EPPS = 1e-5
@@ -40,7 +40,7 @@ def _iterate(geom, grid, first, planes, per, meas, add, beta, seed):
     return x.cpu().numpy(), S.cpu().numpy()
 
 
-def _compare(grid, x, z, n_radial, n_angles, first, planes, bins=1, beta=0.0, add=False, **kw):
+def _compare(grid, x, z, n_radial, n_angles, first, planes, bins=1, beta=0.0, add=False, lists=True, **kw):
     import torch
     per = n_radial * n_angles
     rng = np.random.default_rng(planes + grid.Nx)
@@ -51,8 +51,9 @@ def _compare(grid, x, z, n_radial, n_angles, first, planes, bins=1, beta=0.0, ad
         geom = make_geom(grid, x, z, n_radial, n_angles, generic=generic, **kw)
         out.append(_iterate(geom, grid, first, planes, per, meas, a, beta, 3))
         out.append(_iterate(geom, grid, first, planes, per, meas, a, beta, 3)) if not generic else None
+        assert list_calls(geom) == ((0 if generic or not lists else 4), 0)
     (xa, Sa), (xb, _), (xg, Sg) = out
-    if bins <= 32:                  # more bins keep the one-lane-per-LOR kernels and their atomics
+    if lists:                       # the other kernels add with atomics
         assert np.array_equal(xa, xb)   # the lists have a fixed order
     e, es = rel_l2(xa, xg), rel_l2(Sa, Sg)
     print(f"[plane] {grid.Nx}x{grid.Ny}x{grid.Nz} planes={planes} bins={bins} rel-L2 {e:.2e} sens {es:.2e}", flush=True)
@@ -78,6 +79,7 @@ def test_plane_outside_and_shared_slice(cuda):
     gen = make_geom(grid, x, z, 24, 21, generic=True)
     meas = torch.ones(8 * per, device="cuda")
     a = _iterate(geom, grid, 0, 8, per, meas, None, 0.0, 5)[0]
+    assert list_calls(geom) == (0, 0)
     b = _iterate(gen, grid, 0, 8, per, meas, None, 0.0, 5)[0]
     assert rel_l2(a, b) < 5e-6
 
@@ -88,8 +90,8 @@ def test_tof(cuda, bins, planes):
     sigma = G.tof_sigma(300e-12)
     centres = np.linspace(-40.0, 40.0, bins).astype(np.float32)
     atten = np.full(grid.N, 0.004, np.float32)
-    _compare(grid, x, z, 24, 21, 1, planes, bins=bins, add=True, tof=(bins, sigma, centres, EPPS), atten=atten,
-             atten_mode=1)
+    _compare(grid, x, z, 24, 21, 1, planes, bins=bins, add=True, lists=bins <= 32, tof=(bins, sigma, centres, EPPS),
+             atten=atten, atten_mode=1)
 
 
 @pytest.mark.parametrize("n,flags,planes", [(32, 3, 5), (19, 3, 2), (20, 1, 9)])
@@ -105,3 +107,9 @@ def test_interpolation(cuda, nx, ny, dl, atten, planes):
     grid, x, z = _scanner(nx, ny, 10, 24, 20)
     kw = dict(atten=np.full(grid.N, 0.004, np.float32), atten_mode=1) if atten else {}
     _compare(grid, x, z, 24, 20, 0, planes, projector_type=4, interp=(dl, 0.0), beta=0.01, **kw)
+
+
+def test_lists_off(cuda):
+    """A negative budget keeps no lists."""
+    grid, x, z = _scanner(32, 32, 11, 32, 40)
+    _compare(grid, x, z, 32, 40, 0, 5, lists=False, tube_budget_mib=-1)
