@@ -507,8 +507,11 @@ static bool plan_build(const omg_geom* g, PlanePlan* p, hipStream_t s) {
     p->npix = p->nyx + (interp ? d.Nx + 1 : 0);
     if (interp) interp_plane_slices(g, p->slice_host);
     else siddon_plane_slices(g, p->slice_host);
-    uint32_t plane = 0;
-    while (plane < d.n_proj && p->slice_host[plane] < 0) plane++;
+    // The lowest slice: voxels that a walk leaves out behind the image's end are out for every other plane too, so
+    // the lists hold (or refuse, plane_put) all that any plane visits.
+    uint32_t plane = d.n_proj;
+    for (uint32_t q = 0; q < d.n_proj; q++)
+        if (p->slice_host[q] >= 0 && (plane == d.n_proj || p->slice_host[q] < p->slice_host[plane])) plane = q;
     if (plane == d.n_proj || bins == 0) return false;
     const uint64_t budget = plan_budget(g);
 

@@ -113,3 +113,15 @@ def test_lists_off(cuda):
     """A negative budget keeps no lists."""
     grid, x, z = _scanner(32, 32, 11, 32, 40)
     _compare(grid, x, z, 32, 40, 0, 5, lists=False, tube_budget_mib=-1)
+
+
+@pytest.mark.parametrize("descending", [False, True])
+@pytest.mark.parametrize("tof", [False, True])
+def test_rows_past_the_slice(cuda, descending, tof):
+    """Ny > Nx and LORs along x: those step rows by Ny, so their voxels run on into the next slices and, from the last
+    ones, past the image. Whichever plane comes first, the result is the other kernels'."""
+    grid, x, z = _scanner(21, 34, 10, 29, 28)
+    z = z.reshape(-1, 2)[::-1].copy() if descending else z
+    kw = dict(tof=(5, G.tof_sigma(300e-12), np.linspace(-40.0, 40.0, 5).astype(np.float32), EPPS), bins=5) if tof else {}
+    _compare(grid, x, z, 29, 28, 2, 5, lists=False, beta=0.01, **kw)
+    _compare(grid, x, z, 29, 28, 0, 9, lists=False, **kw)
