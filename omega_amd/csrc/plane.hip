@@ -34,9 +34,12 @@ constexpr int kPB = 256;
 struct PlanePlan {
     bool ok = false;
     bool interp = false;
-    uint32_t bins = 0, nyx = 0, npix = 0;    // rows, pixels of a slice, pixel lists
+    // Rows, pixels of a slice, pixel lists. Pixels nyx and up lie in the slices after the plane's own: the far-face
+    // samples of the interpolation projector, and with Ny > Nx the Siddon rows along x, which step by Ny.
+    uint32_t bins = 0, nyx = 0, npix = 0;
+    uint32_t xrows = 0;                      // pixels that the forward projection reads (interpolation: nyx)
     uint64_t nent = 0;                       // entries of `ent`, padding included
-    uint2* ent = nullptr;                    // row lists {pixel, length}; the padding points at pixel nyx
+    uint2* ent = nullptr;                    // row lists {pixel, length}; the padding points at pixel xrows
     uint32_t* off = nullptr;
     uint32_t* len = nullptr;                 // [row groups] padded entries per row
     uint4* samp = nullptr;                   // interpolation projector: forward samples
@@ -108,8 +111,9 @@ __global__ __launch_bounds__(kPB) void k_plane_sort(uint32_t npix, const uint32_
 
 // ---- running -----------------------------------------------------------------------------------------
 struct PlaneRun {
-    uint32_t bins, nyx, npix, planes;        // planes: of this call
+    uint32_t bins, nyx, npix, xrows, planes; // planes: of this call
     uint32_t nx, nz;                         // image row length, slices
+    bool skip0;                              // interpolation projector: nothing is added to voxel 0
     const uint32_t *off, *len, *soff, *slen, *coff, *clen;
     const uint2 *ent, *cent;
     const uint4* samp;
@@ -123,18 +127,19 @@ struct PlaneRun {
     float bz, sz;
 };
 
-// Xt[chunk][pixel][PL]: the planes' slices side by side, and a zero row behind them for the padding entries.
+// Xt[chunk][pixel][PL]: the planes' slices side by side (and what follows them, up to xrows), and a zero row behind
+// them for the padding entries.
 // INTERP: the blend of the two slices that the plane's samples lie between.
 template <int PL, bool INTERP>
 __global__ __launch_bounds__(kPB) void k_plane_gather(PlaneRun a, const float* __restrict__ x, float* __restrict__ Xt) {
     const uint32_t pix = blockIdx.x * kPB + threadIdx.x;
-    if (pix > a.nyx) return;
+    if (pix > a.xrows) return;
     float v[PL];
 #pragma unroll
     for (int p = 0; p < PL; p++) {
         const uint32_t plane = blockIdx.y * PL + p;
         v[p] = 0.f;
-        if (plane < a.planes && pix < a.nyx) {
+        if (plane < a.planes && pix < a.xrows) {
             const int32_t tk = a.slice[plane];
             if (INTERP) {
                 if (tk >= 0) {
@@ -145,11 +150,12 @@ __global__ __launch_bounds__(kPB) void k_plane_gather(PlaneRun a, const float* _
                     v[p] = (1.f - c) * x[(size_t)z0 * a.nyx + pix] + c * x[(size_t)z1 * a.nyx + pix];
                 }
             } else if (tk >= 0) {
-                v[p] = x[(size_t)tk * a.nyx + pix];
+                const size_t n = (size_t)tk * a.nyx + pix;
+                if (n < (size_t)a.nz * a.nyx) v[p] = x[n];
             }
         }
     }
-    float* o = Xt + ((size_t)blockIdx.y * (a.nyx + 1) + pix) * PL;
+    float* o = Xt + ((size_t)blockIdx.y * (a.xrows + 1) + pix) * PL;
 #pragma unroll
     for (int p = 0; p < PL; p++) o[p] = v[p];
 }
@@ -169,7 +175,7 @@ __global__ __launch_bounds__(kPB) void k_plane_fp(PlaneRun a, const float* __res
         if (SENS) W[o] = 0.f;
         return;
     }
-    const float* X = Xt + (size_t)blockIdx.y * (a.nyx + 1) * PL + p;
+    const float* X = Xt + (size_t)blockIdx.y * (a.xrows + 1) * PL + p;
     const uint32_t g = row / kLI;
     float ax = 0.f;
     if (INTERP) {
@@ -242,7 +248,7 @@ __global__ __launch_bounds__(kPB) void k_plane_tof(PlaneRun a, uint32_t chunk, u
         return;
     }
     const bool in = plane < a.planes && a.slice[plane] >= 0;
-    const float* X = Xt + (size_t)chunk * (a.nyx + 1) * PL + p;
+    const float* X = Xt + (size_t)chunk * (a.xrows + 1) * PL + p;
     const uint32_t g = row / kLI, base = a.off[g] + row % kLI, n = a.len[g];
     const float4* sh = reinterpret_cast<const float4*>(a.share) + (size_t)base * NQ;
     float acc[4 * NQ];
@@ -359,11 +365,22 @@ __device__ __forceinline__ int32_t plane_at(const PlaneRun& a, int32_t z) {
     return -1;
 }
 
+// The lists of pixel `pix` of slice z from the planes in the slices before it (pixels nyx and up).
+template <int PL, bool SENS>
+__device__ __forceinline__ void plane_carried(const PlaneRun& a, uint32_t pix, int32_t z, const float* __restrict__ R,
+                                              const float* __restrict__ W, double& rhs, double& sens) {
+    const size_t rows = (size_t)(a.bins + 1) * PL;
+    for (uint32_t q = pix + a.nyx; q < a.npix && z > 0; q += a.nyx) {
+        const int32_t p = plane_at(a, --z);
+        if (p >= 0) plane_sums<PL, false, SENS>(a, q, R + (p / PL) * rows + p % PL, W + (p / PL) * rows + p % PL, rhs, sens);
+    }
+}
+
 // Backprojection and update. The first `bpb` blocks hold the voxels of the call's planes [chunk0, chunk0 +
 // chunks) of PL planes, one lane per (pixel, plane); with OTHERS the blocks behind them update the image's
-// other slices (rhs = 0), 4 * 256 voxels of one slice each. WRAP (interpolation projector): samples on the
-// image's far face carry into the slice after the plane's own (pixel lists nyx and up).
-template <int PL, bool TOF, bool SENS, bool WRAP>
+// other slices (rhs = 0), 4 * 256 voxels of one slice each. CARRY: pixel lists nyx and up exist, whose voxels lie in
+// the slices after their plane's own.
+template <int PL, bool TOF, bool SENS, bool CARRY>
 __global__ __launch_bounds__(kPB) void k_plane_bp(PlaneRun a, uint32_t bpb, uint32_t per_chunk, uint32_t chunk0,
                                                   const float* __restrict__ R, const float* __restrict__ W,
                                                   float* __restrict__ x, float* __restrict__ S,
@@ -378,14 +395,9 @@ __global__ __launch_bounds__(kPB) void k_plane_bp(PlaneRun a, uint32_t bpb, uint
         double rhs = 0.0, sens = 0.0;
         const size_t rows = (size_t)(a.bins + 1) * PL;
         plane_sums<PL, TOF, SENS>(a, pix, R + (TOF ? 0 : ch * rows) + p, W + (TOF ? 0 : ch * rows) + p, rhs, sens);
-        if (WRAP) {
-            if (tk == 0 && pix == 0) { rhs = 0.0; sens = 0.0; }   // the reference skips voxel 0
-            if (pix + a.nyx < a.npix) {
-                const int32_t q = tk > 0 ? plane_at(a, tk - 1) : -1;
-                if (q >= 0)
-                    plane_sums<PL, TOF, SENS>(a, pix + a.nyx, R + (q / PL) * rows + q % PL, W + (q / PL) * rows + q % PL,
-                                              rhs, sens);
-            }
+        if (CARRY) {
+            if (a.skip0 && tk == 0 && pix == 0) { rhs = 0.0; sens = 0.0; }   // the reference skips voxel 0
+            plane_carried<PL, SENS>(a, pix, tk, R, W, rhs, sens);
         }
         const size_t n = (size_t)tk * a.nyx + pix;
         float s;
@@ -402,16 +414,11 @@ __global__ __launch_bounds__(kPB) void k_plane_bp(PlaneRun a, uint32_t bpb, uint
     const uint32_t b = blockIdx.x - bpb, per = (a.nyx + 4 * kPB - 1) / (4 * kPB);
     const int32_t z = (int32_t)(b / per);
     if (plane_at(a, z) >= 0) return;
-    const int32_t prev = WRAP && z > 0 ? plane_at(a, z - 1) : -1;
     for (uint32_t j = 0; j < 4; j++) {
         const uint32_t pix = (b % per) * 4 * kPB + j * kPB + threadIdx.x;
         if (pix >= a.nyx) return;
         double rhs = 0.0, sens = 0.0;
-        if (WRAP && prev >= 0 && pix + a.nyx < a.npix) {
-            const size_t rows = (size_t)(a.bins + 1) * PL;
-            plane_sums<PL, TOF, SENS>(a, pix + a.nyx, R + (prev / PL) * rows + prev % PL, W + (prev / PL) * rows + prev % PL,
-                                      rhs, sens);
-        }
+        if (CARRY) plane_carried<PL, SENS>(a, pix, z, R, W, rhs, sens);
         const size_t n = (size_t)z * a.nyx + pix;
         float s;
         if (SENS) {
@@ -505,6 +512,9 @@ static bool plan_build(const omg_geom* g, PlanePlan* p, hipStream_t s) {
     p->bins = bins;
     p->nyx = d.Nx * d.Ny;
     p->npix = p->nyx + (interp ? d.Nx + 1 : 0);
+    // a row along x starts at its y times Ny (siddon_setup): with Ny > Nx it can end past the slice. The TOF kernels
+    // hold one chunk of planes at a time and take no such rows, nor are lists many times the slice kept for them.
+    if (!interp && !orth && !tof && d.Ny > d.Nx && d.Ny <= 16 * d.Nx && d.Ny < 32768) p->npix = std::max(p->nyx, (d.Ny - 1) * d.Ny + d.Nx);
     if (interp) interp_plane_slices(g, p->slice_host);
     else siddon_plane_slices(g, p->slice_host);
     // The lowest slice: voxels that a walk leaves out behind the image's end are out for every other plane too, so
@@ -544,6 +554,11 @@ static bool plan_build(const omg_geom* g, PlanePlan* p, hipStream_t s) {
              hipMemcpyAsync(&hbad, bad, 4, hipMemcpyDeviceToHost, s) == hipSuccess &&
              hipStreamSynchronize(s) == hipSuccess && !hbad;
     }
+    if (!interp) {       // only as far as the lists go
+        while (p->npix > p->nyx && hp[p->npix - 1] == 0) p->npix--;
+        hp.resize(p->npix);
+    }
+    p->xrows = interp ? p->nyx : p->npix;
     ok = ok && *std::max_element(hp.begin(), hp.end()) <= kMaxPixelList && list_layout(hc, off, len, &p->nent) &&
          list_layout(hp, coff, clen, &nc) && (!interp || list_layout(hs, soff, slen, &ns));
     p->pitch = tof ? (d.tof_bins + 3) / 4 * 4 : 0;
@@ -558,7 +573,7 @@ static bool plan_build(const omg_geom* g, PlanePlan* p, hipStream_t s) {
     if (ok && interp) ok = upload_u32(&p->soff, soff) && upload_u32(&p->slen, slen) && dev_alloc(&p->samp, ns);
     if (ok && tof) ok = dev_alloc(&p->share, p->nent * p->pitch) && dev_alloc(&p->cpos, nc) && dev_alloc(&lsum, p->nent);
     if (ok) {
-        hipLaunchKernelGGL(k_plane_set2, dim3(grid_for((int64_t)p->nent, kPB)), dim3(kPB), 0, s, p->ent, p->nent, p->nyx);
+        hipLaunchKernelGGL(k_plane_set2, dim3(grid_for((int64_t)p->nent, kPB)), dim3(kPB), 0, s, p->ent, p->nent, p->xrows);
         hipLaunchKernelGGL(k_plane_set2, dim3(grid_for((int64_t)nc, kPB)), dim3(kPB), 0, s, p->cent, nc, bins);
         if (tof) fill1(p->cpos, nc, (uint32_t)p->nent);
         if (interp)
@@ -617,7 +632,7 @@ static int run_planes(omg_geom* g, const PlanePlan* pl, const PlaneRun& a, const
                       hipStream_t s, bool* done) {
     const uint32_t chunks = (a.planes + PL - 1) / PL;
     const bool tof = pl->share != nullptr;
-    const size_t xt = (size_t)chunks * (a.nyx + 1) * PL, rr = (size_t)(tof ? 1 : chunks) * (a.bins + 1) * PL;
+    const size_t xt = (size_t)chunks * (a.xrows + 1) * PL, rr = (size_t)(tof ? 1 : chunks) * (a.bins + 1) * PL;
     const size_t tt = tof ? (size_t)(a.nent + 1) * PL : 0;
     const size_t need = xt + (tof ? tt : rr) + (sens ? rr : 0);
     *done = false;
@@ -631,7 +646,7 @@ static int run_planes(omg_geom* g, const PlanePlan* pl, const PlaneRun& a, const
     float* W = R + (tof ? tt : rr);
     hipEvent_t stop;
     timing_begin(s, &stop);
-    const dim3 gg(grid_for((int64_t)a.nyx + 1, kPB), chunks);
+    const dim3 gg(grid_for((int64_t)a.xrows + 1, kPB), chunks);
     if (pl->interp) hipLaunchKernelGGL((k_plane_gather<PL, true>), gg, dim3(kPB), 0, s, a, x, Xt);
     else hipLaunchKernelGGL((k_plane_gather<PL, false>), gg, dim3(kPB), 0, s, a, x, Xt);
     OMG_CHECK_LAUNCH();
@@ -664,19 +679,19 @@ static int run_planes(omg_geom* g, const PlanePlan* pl, const PlaneRun& a, const
         return OMG_OK;
     }
     const dim3 fg(fpb, chunks), bg(per_chunk * chunks + others);
-#define OMG_PLANE(INTERP, SENS)                                                                                       \
-    do {                                                                                                              \
-        hipLaunchKernelGGL((k_plane_fp<PL, INTERP, SENS>), fg, dim3(kPB), 0, s, a, Xt, meas, add, R, W, epps);         \
-        OMG_CHECK_LAUNCH();                                                                                           \
-        hipLaunchKernelGGL((k_plane_bp<PL, false, SENS, INTERP>), bg, dim3(kPB), 0, s, a, per_chunk * chunks, per_chunk, \
-                           0u, R, W, x, S, dU, epps, pos);                                                            \
-        OMG_CHECK_LAUNCH();                                                                                           \
-    } while (0)
-    if (pl->interp && sens) OMG_PLANE(true, true);
-    else if (pl->interp) OMG_PLANE(true, false);
-    else if (sens) OMG_PLANE(false, true);
-    else OMG_PLANE(false, false);
-#undef OMG_PLANE
+    const bool carry = a.npix > a.nyx;
+    auto step = [&](auto fp, auto bp) {
+        hipLaunchKernelGGL(fp, fg, dim3(kPB), 0, s, a, Xt, meas, add, R, W, epps);
+        OMG_CHECK_LAUNCH();
+        hipLaunchKernelGGL(bp, bg, dim3(kPB), 0, s, a, per_chunk * chunks, per_chunk, 0u, R, W, x, S, dU, epps, pos);
+        OMG_CHECK_LAUNCH();
+        return (int)OMG_OK;
+    };
+    if (pl->interp && sens) rc = step(k_plane_fp<PL, true, true>, k_plane_bp<PL, false, true, true>);
+    else if (pl->interp) rc = step(k_plane_fp<PL, true, false>, k_plane_bp<PL, false, false, true>);
+    else if (sens) rc = step(k_plane_fp<PL, false, true>, carry ? k_plane_bp<PL, false, true, true> : k_plane_bp<PL, false, true, false>);
+    else rc = step(k_plane_fp<PL, false, false>, carry ? k_plane_bp<PL, false, false, true> : k_plane_bp<PL, false, false, false>);
+    if (rc) return rc;
     timing_end(s, stop);
     return OMG_OK;
 }
@@ -687,7 +702,8 @@ int plane_subset_iteration(omg_geom* g, const PlanePlan* pl, int64_t first, int6
     const uint32_t planes = (uint32_t)(n / pl->bins);
     const SidArgs sa = make_sid_args(g, first, n);
     PlaneRun a;
-    a.bins = pl->bins; a.nyx = pl->nyx; a.npix = pl->npix; a.planes = planes;
+    a.bins = pl->bins; a.nyx = pl->nyx; a.npix = pl->npix; a.xrows = pl->xrows; a.planes = planes;
+    a.skip0 = pl->interp;
     a.nx = g->d.Nx;
     a.nz = g->d.Nz;
     a.off = pl->off; a.len = pl->len; a.soff = pl->soff; a.slen = pl->slen; a.coff = pl->coff; a.clen = pl->clen;

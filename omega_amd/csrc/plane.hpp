@@ -16,7 +16,7 @@ constexpr uint32_t kLUnroll = 8;
 // Where the tracing kernels put a row's entries. Counting pass: ent null, cnt[row] and the pixels' counts.
 // Filling pass: ent (and for the interpolation projector samp) and the LOR weights of every plane.
 struct PlaneFill {
-    uint32_t npix;               // pixel lists: Nx * Ny, and Nx + 1 more for the interpolation projector
+    uint32_t npix;               // pixel lists: Nx * Ny, and those of the slices behind (PlanePlan)
     uint32_t slice_base;         // linear index of the traced plane's slice
     uint32_t* cnt;               // [rows] entries
     uint32_t* pixcnt;            // [npix] entries

@@ -123,5 +123,7 @@ def test_rows_past_the_slice(cuda, descending, tof):
     grid, x, z = _scanner(21, 34, 10, 29, 28)
     z = z.reshape(-1, 2)[::-1].copy() if descending else z
     kw = dict(tof=(5, G.tof_sigma(300e-12), np.linspace(-40.0, 40.0, 5).astype(np.float32), EPPS), bins=5) if tof else {}
-    _compare(grid, x, z, 29, 28, 2, 5, lists=False, beta=0.01, **kw)
-    _compare(grid, x, z, 29, 28, 0, 9, lists=False, **kw)
+    _compare(grid, x, z, 29, 28, 2, 5, lists=not tof, beta=0.01, **kw)
+    _compare(grid, x, z, 29, 28, 0, 9, lists=not tof, **kw)
+    grid, x, z = _scanner(9, 34, 10, 29, 28)          # over more than one slice
+    _compare(grid, x, z[::-1] if descending else z, 29, 28, 1, 8, lists=not tof, **kw)
