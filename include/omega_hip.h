@@ -153,7 +153,8 @@ int omg_geom_list_calls(const omg_geom* g, int64_t* plane_calls, int64_t* column
  * subset-ordered data: first is the subset's first plane/projection (list mode: LOR).
  * y is overwritten. Replaces projectorClass.forwardProject / projfunctions.forwardProjection
  * (proj.py:1923, projfunctions.py:86) and projectorType123Implementation4(fp=1)
- * (source/cpp/projector_functions.h:1311). */
+ * (source/cpp/projector_functions.h:1311). projector_type 1: calls through one handle may run beside each other, on
+ * several streams and from several threads; captured in a graph they trace their LORs. */
 int omg_forward_project(const omg_geom* g, int64_t first, int64_t n_meas, const float* img, float* y, void* stream);
 
 /* Backprojection rhs += A_k^T y; if sens != NULL also sens += A_k^T 1. rhs/sens are

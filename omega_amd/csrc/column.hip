@@ -23,6 +23,9 @@
 
 #include <algorithm>
 #include <cmath>
+#include <memory>
+#include <mutex>
+#include <new>
 #include <type_traits>
 #include <vector>
 
@@ -664,7 +667,20 @@ __global__ __launch_bounds__(1024, 8) void k_col_bp(ColView c, SidArgs a, uint32
 }
 
 // ---- host ----------------------------------------------------------------------------------------------
-struct ColCache { std::vector<ColPlan*> e; };
+struct ColBuffer {
+    std::mutex mu;                  // held while a call's launches are issued
+    hipStream_t s = nullptr;        // of the calls that used it last; their end is `done`
+    hipEvent_t done = nullptr;      // (the null stream's buffer has none)
+    float* p = nullptr;
+    size_t floats = 0;
+};
+
+struct ColCache {
+    std::vector<ColPlan*> e;
+    std::mutex buffers_mu;
+    std::vector<std::unique_ptr<ColBuffer>> buffers;
+    size_t others = 0;              // of them for streams that are not the null stream
+};
 
 static void col_free(ColPlan* p) {
     hipFree(p->off); hipFree(p->start); hipFree(p->ent); hipFree(p->seg); hipFree(p->item);
@@ -780,15 +796,16 @@ static bool col_build(const omg_geom* g, ColPlan* p, hipStream_t s) {
     ok = ok && p->items > 0 && col_alloc(&p->off, off.size()) && col_alloc(&p->start, p->bins) &&
          col_alloc(&p->ent, total + 4) &&
          col_alloc(&p->seg, segs) && col_alloc(&p->item, items.size()) && col_alloc(&tile_off, tiles) &&
-         hipMemcpy(p->off, off.data(), off.size() * 4, hipMemcpyHostToDevice) == hipSuccess &&
-         hipMemcpy(tile_off, toff.data(), tiles * 4ull, hipMemcpyHostToDevice) == hipSuccess &&
-         hipMemcpy(p->item, items.data(), items.size() * sizeof(ColItem), hipMemcpyHostToDevice) == hipSuccess;
+         hipMemcpyAsync(p->off, off.data(), off.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
+         hipMemcpyAsync(tile_off, toff.data(), tiles * 4ull, hipMemcpyHostToDevice, s) == hipSuccess &&
+         hipMemcpyAsync(p->item, items.data(), items.size() * sizeof(ColItem), hipMemcpyHostToDevice, s) == hipSuccess;
     if (ok) {
         hipLaunchKernelGGL(k_col_zero, dim3(grid_for(tiles, 256)), dim3(256), 0, s, tile_cnt, tiles);
         hipLaunchKernelGGL(k_col_trace, grid, block, 0, s, a, p->bins, p->tw, p->th, p->ntx, tiles, cnt, tile_cnt, p->off,
                            p->start, p->ent, tile_off, p->seg);
         ok = hipGetLastError() == hipSuccess && hipStreamSynchronize(s) == hipSuccess;
     }
+    if (!ok) (void)hipStreamSynchronize(s);      // copies from this function's tables
     hipFree(cnt); hipFree(tile_cnt); hipFree(tile_off);
     if (!ok) {
         (void)hipGetLastError();
@@ -809,20 +826,24 @@ const ColPlan* col_plan(const omg_geom* gc, int64_t first, int64_t n, hipStream_
         return nullptr;
     const uint64_t per = (uint64_t)d.size_x * d.size_y;
     if (!g->index_dev && ((uint64_t)n < min_planes * per || (uint64_t)n % per)) return nullptr;
-    if (!g->columns) {
-        if (fixed_region_active()) return nullptr;
-        g->columns = new ColCache();
+    const std::lock_guard<std::mutex> lock(g->lists_mu);
+    if (g->columns)
+        for (ColPlan* p : g->columns->e)
+            if (!g->index_dev || (p->first == first && p->n == n)) return p->ok ? p : nullptr;
+    if (fixed_region_active() || (g->columns && g->columns->e.size() >= kColPlans) || is_capturing(s)) return nullptr;
+    try {
+        const RelaxedCapture relaxed;
+        if (!g->columns) g->columns = new ColCache();
+        g->columns->e.reserve(kColPlans);
+        std::unique_ptr<ColPlan> p(new ColPlan());
+        p->first = first;
+        p->n = n;
+        p->ok = col_build(g, p.get(), s);
+        g->columns->e.push_back(p.release());
+    } catch (const std::bad_alloc&) {       // no host memory for the tables: trace
+        return nullptr;
     }
-    for (ColPlan* p : g->columns->e)
-        if (!g->index_dev || (p->first == first && p->n == n)) return p->ok ? p : nullptr;
-    if (fixed_region_active() || g->columns->e.size() >= kColPlans) return nullptr;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return nullptr;
-    ColPlan* p = new ColPlan();
-    p->first = first;
-    p->n = n;
-    g->columns->e.push_back(p);
-    p->ok = col_build(g, p, s);
+    const ColPlan* p = g->columns->e.back();
     return p->ok ? p : nullptr;
 }
 
@@ -831,6 +852,10 @@ void col_release(omg_geom* g) {
     for (ColPlan* p : g->columns->e) {
         col_free(p);
         delete p;
+    }
+    for (auto& b : g->columns->buffers) {
+        hipFree(b->p);
+        if (b->done) hipEventDestroy(b->done);
     }
     delete g->columns;
     g->columns = nullptr;
@@ -857,15 +882,15 @@ static void col_launch_fp(const ColView& c, const SidArgs& a, uint32_t g0, uint3
     else launch(k_col_fp<MODE, 1, 0>, 4);
 }
 
-struct ColWork {
+struct ColLayout {
     uint32_t nr, pitch, all, pass;
     uint64_t per;
     size_t nimg, nrec, nw, need;
 };
 
-static ColWork col_work(const omg_geom* g, const ColPlan* pl, int64_t n, bool img, bool rec, bool sens) {
+static ColLayout col_layout(const omg_geom* g, const ColPlan* pl, int64_t n, bool img, bool rec, bool sens) {
     const omg_geom_desc& d = g->d;
-    ColWork w;
+    ColLayout w;
     const bool small = (uint64_t)d.Nx * d.Ny * (d.Nz <= 63 ? 256 : 512) <= 0xffffffffull;   // a buffer's offsets
     w.nr = !small ? 0 : d.Nz <= 63 ? 1 : d.Nz <= 127 ? 2 : 0;
     w.pitch = w.nr ? 64 * w.nr : d.Nz + 2;
@@ -879,37 +904,108 @@ static ColWork col_work(const omg_geom* g, const ColPlan* pl, int64_t n, bool im
     return w;
 }
 
-size_t col_osem_work(const omg_geom* g, const ColPlan* pl, int64_t n) { return col_work(g, pl, n, true, true, false).need; }
+size_t col_work_floats(const omg_geom* g, const ColPlan* pl, int64_t n, bool img, bool rec, bool sens) {
+    return col_layout(g, pl, n, img, rec, sens).need;
+}
+
+// A buffer for stream s, locked: the one that s used last, a new one, or one whose last call has ended. Null: none.
+static ColBuffer* col_buffer(ColCache* c, hipStream_t s) {
+    for (;;) {
+        ColBuffer* own = nullptr;
+        {
+            const std::lock_guard<std::mutex> lock(c->buffers_mu);
+            for (auto& b : c->buffers)
+                if (b->s == s) own = b.get();
+            if (!own && (c->others < kColStreams || !s)) {
+                std::unique_ptr<ColBuffer> b(new ColBuffer());
+                c->buffers.reserve(kColStreams + 1);
+                if (s && hipEventCreateWithFlags(&b->done, hipEventDisableTiming) != hipSuccess) {
+                    (void)hipGetLastError();
+                    return nullptr;
+                }
+                b->mu.lock();
+                b->s = s;
+                c->others += s ? 1 : 0;
+                c->buffers.push_back(std::move(b));
+                return c->buffers.back().get();
+            }
+            for (size_t i = 0; !own && i < c->buffers.size(); i++) {
+                ColBuffer* b = c->buffers[i].get();
+                if (!b->s || !b->mu.try_lock()) continue;
+                if (hipEventQuery(b->done) == hipSuccess) {
+                    b->s = s;
+                    return b;
+                }
+                (void)hipGetLastError();    // not ready
+                b->mu.unlock();
+            }
+        }
+        if (!own) return nullptr;
+        own->mu.lock();             // another thread's call on s: the two come one after the other in any case
+        if (own->s == s) return own;
+        own->mu.unlock();           // given to another stream meanwhile
+    }
+}
+
+ColWork::ColWork(const omg_geom* g, size_t floats, hipStream_t s, bool beside) : s_(s) {
+    if (fixed_region_active() ? !scratch_fits(g, floats) : is_capturing(s)) return;
+    if (fixed_region_active() || !beside) {
+        if (scratch_reserve(const_cast<omg_geom*>(g), floats) == OMG_OK) p_ = scratch_ptr(g);
+        else (void)hipGetLastError();
+        return;
+    }
+    const RelaxedCapture relaxed;
+    try {
+        buf_ = col_buffer(g->columns, s);
+    } catch (const std::bad_alloc&) {
+    }
+    if (!buf_) return;
+    // The event also orders calls of a stream that has this handle's name only by now (hipStreamPerThread in another
+    // thread, a destroyed stream's successor); on the stream itself it is nothing to wait for.
+    bool ok = !buf_->done || hipStreamWaitEvent(s, buf_->done, 0) == hipSuccess;
+    if (ok && buf_->floats < floats) {
+        ok = (buf_->done ? hipEventSynchronize(buf_->done) : hipStreamSynchronize(s)) == hipSuccess;
+        hipFree(buf_->p);
+        buf_->p = nullptr;
+        buf_->floats = 0;
+        ok = ok && hipMalloc(reinterpret_cast<void**>(&buf_->p), floats * sizeof(float)) == hipSuccess;
+        if (ok) buf_->floats = floats;
+    }
+    if (ok) p_ = buf_->p;
+    else (void)hipGetLastError();
+}
+
+ColWork::~ColWork() {
+    if (!buf_) return;
+    if (p_ && buf_->done && hipEventRecord(buf_->done, s_) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipStreamSynchronize(s_);
+    }
+    buf_->mu.unlock();
+}
 
 // The plane groups of a call, pass after pass. yout: forward projection of img. Otherwise rhs (and sens) += the
-// backprojection of the ratios (img given) or of yin (null: ones). work: the caller's, or null for the handle's.
+// backprojection of the ratios (img given) or of yin (null: ones).
 static int col_run(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* img, const float* yin,
                    float* yout, const float* add, float* rhs, float* sens, float epps, float* work, hipStream_t s,
-                   bool* done) {
+                   bool timed) {
     const omg_geom_desc& d = g->d;
     const ColView c{pl->bins, (uint32_t)(n / pl->bins), pl->tw, pl->th, pl->ntx, pl->max_segs,
                     pl->off, pl->start, pl->ent, pl->seg, pl->item};
     SidArgs a = make_sid_args(g, first, n);
     a.plane_col = g->index_dev ? 0 : first;   // the z table's first plane (an index table's range holds every plane)
     a.add = add;
-    const ColWork w = col_work(g, pl, n, img != nullptr, rhs != nullptr, sens != nullptr);
+    const ColLayout w = col_layout(g, pl, n, img != nullptr, rhs != nullptr, sens != nullptr);
     const uint32_t nr = w.nr, pitch = w.pitch, all = w.all, pass = w.pass;
-    *done = false;
-    if (!work) {
-        if (!scratch_fits(g, w.need)) return OMG_OK;
-        const int rc = scratch_reserve(const_cast<omg_geom*>(g), w.need);
-        if (rc) return rc;
-    }
-    *done = true;
     g->column_calls.fetch_add(1, std::memory_order_relaxed);
-    float* Xz = work ? work : scratch_ptr(g);
+    float* Xz = work;
     float4* rec = reinterpret_cast<float4*>(Xz + w.nimg);
     float* wrec = sens ? Xz + w.nimg + w.nrec : nullptr;
     uint32_t* rest = reinterpret_cast<uint32_t*>(Xz + w.nimg + w.nrec + w.nw);
     uint32_t* state = rest + w.per * pass;
     const size_t lds = col_lds(c.tw, c.th, d.Nz);
     hipEvent_t stop = nullptr;
-    if (!work) timing_begin(s, &stop);
+    if (timed) timing_begin(s, &stop);
     if (img)
         hipLaunchKernelGGL(k_col_zfast, dim3((d.Nx + 31) / 32, d.Ny, (pitch + 31) / 32), dim3(32, 8), 0, s, img, Xz, d.Nx,
                            d.Ny, d.Nz, pitch, nr ? 0u : 1u, state);
@@ -933,23 +1029,23 @@ static int col_run(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t 
         }
         OMG_CHECK_LAUNCH();
     }
-    if (!work) timing_end(s, stop);
+    if (timed) timing_end(s, stop);
     return OMG_OK;
 }
 
-int col_forward(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* img, float* y,
-                hipStream_t s, bool* done) {
-    return col_run(g, pl, first, n, img, nullptr, y, nullptr, nullptr, nullptr, 0.f, nullptr, s, done);
+int col_forward(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* img, float* y, float* work,
+                hipStream_t s) {
+    return col_run(g, pl, first, n, img, nullptr, y, nullptr, nullptr, nullptr, 0.f, work, s, true);
 }
 
 int col_backward(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* y, float* rhs, float* sens,
-                 hipStream_t s, bool* done) {
-    return col_run(g, pl, first, n, nullptr, y, nullptr, nullptr, rhs, sens, 0.f, nullptr, s, done);
+                 float* work, hipStream_t s) {
+    return col_run(g, pl, first, n, nullptr, y, nullptr, nullptr, rhs, sens, 0.f, work, s, true);
 }
 
 int col_osem(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t n, const float* img, const float* meas,
-             const float* add, float* rhs, float* sens, float epps, float* work, hipStream_t s, bool* done) {
-    return col_run(g, pl, first, n, img, meas, nullptr, add, rhs, sens, epps, work, s, done);
+             const float* add, float* rhs, float* sens, float epps, float* work, hipStream_t s, bool timed) {
+    return col_run(g, pl, first, n, img, meas, nullptr, add, rhs, sens, epps, work, s, timed);
 }
 
 }  // namespace omg

@@ -40,6 +40,22 @@ void set_error(const char* fmt, ...);
 
 static inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
+// While it lives, this thread may allocate and wait although a stream capture is under way elsewhere (another
+// thread's global capture, or a stream of its own that the call does not touch) without invalidating it.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// True when stream s is being captured, or cannot be asked (the null stream beside a capture that it would join).
+static inline bool is_capturing(hipStream_t s) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 static inline unsigned grid_for(int64_t n, int block) { return (unsigned)((n + block - 1) / block); }
 
 }  // namespace omg

@@ -27,6 +27,7 @@
 #include "rdp_device.hpp"
 
 #include <algorithm>
+#include <optional>
 #include <vector>
 
 namespace omg {
@@ -254,7 +255,8 @@ __global__ __launch_bounds__(256) void k_frames_update_t(uint32_t Nx, uint32_t N
 struct FramesStep {
     const omg_geom* g;
     const ColPlan* columns;   // by image columns; null: one lane per LOR
-    float* work;              // its work memory, or null for the handle's
+    float* work;              // its work memory
+    bool timed;               // record its launches
     int64_t first;
     SidArgs a;
     uint32_t F, N;
@@ -331,15 +333,13 @@ static int launch_step(const FramesStep& st, hipStream_t s) {
                            st.Nz, st.F, st.gamma, st.epps, st.beta);
         OMG_CHECK_LAUNCH();
     }
-    bool done = false;
-    for (uint32_t f = 0; st.columns && f < st.F; f++) {   // the first frame decides: the next ones need no more memory
+    for (uint32_t f = 0; st.columns && f < st.F; f++) {
         const int rc = col_osem(st.g, st.columns, st.first, st.a.nmeas, st.x + (size_t)f * st.N,
                                 st.meas + (size_t)f * st.meas_stride, nullptr, st.rhs + (size_t)f * st.N, nullptr, st.epps,
-                                st.work, s, &done);
+                                st.work, s, st.timed);
         if (rc) return rc;
-        if (!done) break;
     }
-    if (!done) {
+    if (!st.columns) {
         hipError_t e;
         switch (st.rpb) {
             case 64: e = launch_data_ft<64>(st, s); break;
@@ -351,7 +351,7 @@ static int launch_step(const FramesStep& st, hipStream_t s) {
             return OMG_ERR_HIP;
         }
     }
-    if (st.rhs_t && !done) {
+    if (st.rhs_t && !st.columns) {
         const dim3 tg((st.Nx + 31) / 32, (st.Ny + 31) / 32, st.Nz * st.F);
         hipLaunchKernelGGL(k_frames_update_t, tg, dim3(32, 8), 0, s, st.Nx, st.Ny, st.Nz, st.x, st.S, st.rhs, st.rhs_t,
                            st.dU, st.epps, st.pos);
@@ -392,6 +392,7 @@ static int make_step(const omg_geom* g, int64_t first, int64_t n_meas, int32_t n
     st.g = g;
     st.columns = nullptr;
     st.work = nullptr;
+    st.timed = true;
     st.first = first;
     st.a = make_sid_args(g, first, n_meas);
     st.F = (uint32_t)n_frames;
@@ -447,7 +448,9 @@ extern "C" int omg_frames_sensitivity(const omg_geom* g, int64_t first, int64_t 
     if (n_meas > 0) {
         bool done = false;
         if (const ColPlan* pl = col_plan(g, first, n_meas, s, kColPlanesBack)) {
-            const int rc = col_backward(g, pl, first, n_meas, nullptr, S, nullptr, s, &done);
+            const ColWork work(g, col_work_floats(g, pl, n_meas, false, true, false), s, true);
+            done = work.get() != nullptr;
+            const int rc = done ? col_backward(g, pl, first, n_meas, nullptr, S, nullptr, work.get(), s) : OMG_OK;
             if (rc) return rc;
         }
         if (!done) {
@@ -475,13 +478,12 @@ extern "C" int omg_frames_forward(const omg_geom* g, int64_t first, int64_t n_me
     hipStream_t s = as_stream(stream);
     const uint32_t N = g->d.Nx * g->d.Ny * g->d.Nz;
     if (const ColPlan* pl = col_plan(g, first, n_meas, s)) {
-        bool done = false;
-        for (int32_t f = 0; f < n_frames; f++) {
-            const int rc = col_forward(g, pl, first, n_meas, x + (size_t)f * N, yhat + (size_t)f * yhat_stride, s, &done);
+        const ColWork work(g, col_work_floats(g, pl, n_meas, true, false, false), s, true);
+        for (int32_t f = 0; work.get() && f < n_frames; f++) {
+            const int rc = col_forward(g, pl, first, n_meas, x + (size_t)f * N, yhat + (size_t)f * yhat_stride, work.get(), s);
             if (rc) return rc;
-            if (!done) break;
         }
-        if (done) return OMG_OK;
+        if (work.get()) return OMG_OK;
     }
     const SidArgs a = make_sid_args(g, first, n_meas);
     const unsigned gx = grid_for(n_meas, 256);
@@ -517,7 +519,13 @@ extern "C" int omg_frames_osem_step(const omg_geom* g, int64_t first, int64_t n_
     int rc = make_step(g, first, n_meas, n_frames, x, meas, meas_stride, S, rhs, nullptr, dU, beta, gamma, epps,
                        positivity, rays_per_block, frames_per_tile, grid_blocks, st);
     if (rc) return rc;
-    st.columns = n_meas > 0 ? col_plan(g, first, n_meas, s) : nullptr;
+    if (n_meas > 0) st.columns = col_plan(g, first, n_meas, s);
+    std::optional<ColWork> work;
+    if (st.columns) {
+        work.emplace(g, col_work_floats(g, st.columns, n_meas, true, true, false), s, false);
+        st.work = work->get();
+        if (!st.work) st.columns = nullptr;
+    }
     if (!st.columns && frames_split(g)) {
         rc = frames_t_reserve(const_cast<omg_geom*>(g), (size_t)st.N * st.F, s);
         if (rc) return rc;
@@ -563,7 +571,7 @@ extern "C" int omg_frames_graph_create(const omg_geom* g, int32_t n_subsets, con
     size_t work = 0;
     for (FramesStep& st : steps) {
         st.columns = st.a.nmeas > 0 ? col_plan(g, st.first, st.a.nmeas, cs) : nullptr;
-        if (st.columns) work = std::max(work, col_osem_work(g, st.columns, st.a.nmeas));
+        if (st.columns) work = std::max(work, col_work_floats(g, st.columns, st.a.nmeas, true, true, false));
     }
     if (work && hipMalloc(reinterpret_cast<void**>(&h->work), work * sizeof(float)) != hipSuccess) {
         (void)hipGetLastError();
@@ -571,6 +579,7 @@ extern "C" int omg_frames_graph_create(const omg_geom* g, int32_t n_subsets, con
     }
     for (FramesStep& st : steps) {
         st.work = h->work;
+        st.timed = false;
         if (!h->work) st.columns = nullptr;
     }
     hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);

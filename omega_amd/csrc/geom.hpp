@@ -4,6 +4,7 @@
 #include "siddon_device.hpp"
 
 #include <atomic>
+#include <mutex>
 #include <vector>
 
 namespace omg { struct PlanePlan; struct ColCache; }
@@ -40,6 +41,9 @@ struct omg_geom {
     // Projectors 2 and 3: the tube lists of the measurement ranges used so far, kept on the device
     // (orth.hip; omg_geom_desc.reserved[4] sets the budget).
     struct TubeCache* tubes = nullptr;
+    // Guards the two kinds of lists below: calls of several threads through one handle may be the first to need them.
+    // They are published complete.
+    std::mutex lists_mu;
     // Direct-plane sinograms: the one 2-D system's lists (plane.hip), built by the first subset iteration that
     // may allocate.
     omg::PlanePlan* plane = nullptr;

@@ -26,6 +26,8 @@
 
 #include <algorithm>
 #include <cmath>
+#include <memory>
+#include <new>
 
 namespace omg {
 
@@ -467,9 +469,9 @@ static bool list_layout(const std::vector<uint32_t>& cnt, std::vector<uint32_t>&
     return true;
 }
 
-static bool upload_u32(uint32_t** dst, const std::vector<uint32_t>& v) {
+static bool upload_u32(uint32_t** dst, const std::vector<uint32_t>& v, hipStream_t s) {
     return dev_alloc(dst, v.size()) &&
-           hipMemcpy(*dst, v.data(), v.size() * sizeof(uint32_t), hipMemcpyHostToDevice) == hipSuccess;
+           hipMemcpyAsync(*dst, v.data(), v.size() * sizeof(uint32_t), hipMemcpyHostToDevice, s) == hipSuccess;
 }
 
 // Device memory that the lists may take (omg_geom_desc.reserved[4], as the tube lists).
@@ -566,11 +568,11 @@ static bool plan_build(const omg_geom* g, PlanePlan* p, hipStream_t s) {
     if (p->pitch == 12) p->pitch = 16;
     if (p->pitch == 28) p->pitch = 32;
     ok = ok && p->nent * (8 + 4 + 4ull * p->pitch) + nc * (8 + 12 + 4) + ns * 16 + 4ull * bins * d.n_proj <= budget;
-    ok = ok && upload_u32(&p->off, off) && upload_u32(&p->len, len) && upload_u32(&p->coff, coff) &&
-         upload_u32(&p->clen, clen) && dev_alloc(&p->ent, p->nent) && dev_alloc(&p->cent, nc) && dev_alloc(&key, nc) &&
+    ok = ok && upload_u32(&p->off, off, s) && upload_u32(&p->len, len, s) && upload_u32(&p->coff, coff, s) &&
+         upload_u32(&p->clen, clen, s) && dev_alloc(&p->ent, p->nent) && dev_alloc(&p->cent, nc) && dev_alloc(&key, nc) &&
          dev_alloc(&val, nc) && dev_alloc(&p->w, (uint64_t)bins * d.n_proj) && dev_alloc(&p->slice, d.n_proj) &&
-         hipMemcpy(p->slice, p->slice_host.data(), d.n_proj * 4ull, hipMemcpyHostToDevice) == hipSuccess;
-    if (ok && interp) ok = upload_u32(&p->soff, soff) && upload_u32(&p->slen, slen) && dev_alloc(&p->samp, ns);
+         hipMemcpyAsync(p->slice, p->slice_host.data(), d.n_proj * 4ull, hipMemcpyHostToDevice, s) == hipSuccess;
+    if (ok && interp) ok = upload_u32(&p->soff, soff, s) && upload_u32(&p->slen, slen, s) && dev_alloc(&p->samp, ns);
     if (ok && tof) ok = dev_alloc(&p->share, p->nent * p->pitch) && dev_alloc(&p->cpos, nc) && dev_alloc(&lsum, p->nent);
     if (ok) {
         hipLaunchKernelGGL(k_plane_set2, dim3(grid_for((int64_t)p->nent, kPB)), dim3(kPB), 0, s, p->ent, p->nent, p->xrows);
@@ -595,6 +597,7 @@ static bool plan_build(const omg_geom* g, PlanePlan* p, hipStream_t s) {
                            pixcnt, key, val, p->cent, p->cpos);
         ok = ok && hipGetLastError() == hipSuccess && hipStreamSynchronize(s) == hipSuccess;
     }
+    if (!ok) (void)hipStreamSynchronize(s);      // copies from this function's tables
     hipFree(cnt); hipFree(pixcnt); hipFree(scnt); hipFree(bad); hipFree(key); hipFree(val); hipFree(lsum);
     if (interp && ok) {      // the row lists served the transposition only
         hipFree(p->ent);
@@ -609,12 +612,17 @@ static bool plan_build(const omg_geom* g, PlanePlan* p, hipStream_t s) {
 
 const PlanePlan* plane_plan(const omg_geom* gc, hipStream_t s) {
     omg_geom* g = const_cast<omg_geom*>(gc);
+    const std::lock_guard<std::mutex> lock(g->lists_mu);
     if (g->plane) return g->plane->ok ? g->plane : nullptr;
-    if (!plan_applies(g) || fixed_region_active()) return nullptr;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return nullptr;
-    g->plane = new PlanePlan();
-    g->plane->ok = plan_build(g, g->plane, s);
+    if (!plan_applies(g) || fixed_region_active() || is_capturing(s)) return nullptr;
+    try {
+        const RelaxedCapture relaxed;
+        std::unique_ptr<PlanePlan> p(new PlanePlan());
+        p->ok = plan_build(g, p.get(), s);
+        g->plane = p.release();
+    } catch (const std::bad_alloc&) {       // no host memory for the tables: trace
+        return nullptr;
+    }
     return g->plane->ok ? g->plane : nullptr;
 }
 

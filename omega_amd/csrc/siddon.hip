@@ -692,9 +692,8 @@ static dim3 xy_tiles(const omg_geom* g) { return dim3((g->d.Nx + 31) / 32, (g->d
 static int generic_fp(const omg_geom* g, int64_t first, int64_t n, const float* img, float* y, hipStream_t s) {
     if (g->d.tof_bins > 1) return tof_forward(g, first, n, img, y, s);
     if (const ColPlan* pl = col_plan(g, first, n, s)) {
-        bool done = false;
-        const int rc = col_forward(g, pl, first, n, img, y, s, &done);
-        if (rc || done) return rc;
+        const ColWork work(g, col_work_floats(g, pl, n, true, false, false), s, true);
+        if (work.get()) return col_forward(g, pl, first, n, img, y, work.get(), s);
     }
     const SidArgs a = make_sid_args(g, first, n);
     hipEvent_t stop;
@@ -710,9 +709,8 @@ static int generic_osem(const omg_geom* g, int64_t first, int64_t n, const float
                         float* sens, float epps, hipStream_t s, const float* add) {
     if (g->d.tof_bins > 1) return tof_osem(g, first, n, img, meas, rhs, sens, epps, s, add);
     if (const ColPlan* pl = col_plan(g, first, n, s)) {
-        bool done = false;
-        const int rc = col_osem(g, pl, first, n, img, meas, add, rhs, sens, epps, nullptr, s, &done);
-        if (rc || done) return rc;
+        const ColWork work(g, col_work_floats(g, pl, n, true, true, sens != nullptr), s, false);
+        if (work.get()) return col_osem(g, pl, first, n, img, meas, add, rhs, sens, epps, work.get(), s);
     }
     SidArgs a = make_sid_args(g, first, n);
     a.add = add;
@@ -798,9 +796,8 @@ extern "C" int omg_backward_project(const omg_geom* g, int64_t first, int64_t n_
     }
     if (g->d.tof_bins > 1) return tof_backward(g, first, n_meas, y, rhs, sens, s);
     if (const ColPlan* pl = col_plan(g, first, n_meas, s, kColPlanesBack)) {
-        bool done = false;
-        rc = col_backward(g, pl, first, n_meas, y, rhs, sens, s, &done);
-        if (rc || done) return rc;
+        const ColWork work(g, col_work_floats(g, pl, n_meas, false, true, sens != nullptr), s, false);
+        if (work.get()) return col_backward(g, pl, first, n_meas, y, rhs, sens, work.get(), s);
     }
     SidArgs a = make_sid_args(g, first, n_meas);
     if (split_layout(g)) {

@@ -171,3 +171,111 @@ def test_frames(cuda, frames, planes):
     assert rel_l2(a[0], b[0]) < BAR
     for k in (1, 3):
         assert rel_l2(a[k][:, seen], b[1][:, seen]) < BAR
+
+
+def test_first_call_beside_a_capture(cuda):
+    """A handle's first projection, which builds its lists, while another thread captures: neither disturbs the other."""
+    import threading
+    import torch
+    grid, x, z = _scanner(20, 20, 9, 24, 20, 40)
+    n = 40 * 480
+    img, out, want = torch.rand(grid.N, device="cuda"), torch.empty(n, device="cuda"), torch.empty(n, device="cuda")
+    geom, gen = (make_geom(grid, x, z, 24, 20, generic=g) for g in (False, True))
+    _lib.call("omg_forward_project", gen.handle, 0, n, ptr(img), ptr(want), None)
+    side, a = torch.cuda.Stream(), torch.zeros(64, device="cuda")
+    torch.cuda.synchronize()
+    failed = []
+
+    def project():
+        try:
+            torch.cuda.set_device(0)
+            _lib.call("omg_forward_project", geom.handle, 0, n, ptr(img), ptr(out), C.c_void_p(side.cuda_stream))
+        except Exception as e:
+            failed.append(e)
+
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        a.add_(1.0)
+        t = threading.Thread(target=project)
+        t.start()
+        t.join()
+        a.mul_(3.0)
+    assert not failed
+    for k in range(3):
+        a.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float(a.sum()) == 64 * 3.0
+    assert np.array_equal(out.cpu().numpy(), want.cpu().numpy())
+    assert list_calls(geom) == (0, 1)
+
+
+def _operands(grid, n, k):
+    import torch
+    return [torch.rand(grid.N, device="cuda") + 0.5 for _ in range(k)], [torch.empty(n, device="cuda") for _ in range(k)]
+
+
+def test_projections_beside_each_other(cuda):
+    """Forward projections of one handle on six streams and from six threads, with a backprojection between them."""
+    import threading
+    import torch
+    grid, x, z = _scanner(64, 64, 31, 64, 60, 70)
+    n = 70 * 64 * 60
+    img, want = _operands(grid, n, 6)
+    out = [torch.empty(n, device="cuda") for _ in img]
+    y, back, ref = torch.rand(n, device="cuda"), torch.zeros(grid.N, device="cuda"), torch.zeros(grid.N, device="cuda")
+    gen, geom = make_geom(grid, x, z, 64, 60, generic=True), make_geom(grid, x, z, 64, 60)
+    for i, w in zip(img, want):
+        _lib.call("omg_forward_project", gen.handle, 0, n, ptr(i), ptr(w), None)
+    _lib.call("omg_backward_project", gen.handle, 0, n, ptr(y), ptr(ref), None, None)
+    streams = [torch.cuda.Stream() for _ in img]
+    torch.cuda.synchronize()
+
+    def project(k):
+        for _ in range(3):
+            _lib.call("omg_forward_project", geom.handle, 0, n, ptr(img[k]), ptr(out[k]), C.c_void_p(streams[k].cuda_stream))
+
+    for threads in (False, True):
+        for o in out:
+            o.zero_()
+        back.zero_()
+        torch.cuda.synchronize()
+        ts = [threading.Thread(target=project, args=(k,)) for k in range(6)]
+        for k, t in enumerate(ts):
+            t.start() if threads else project(k)
+            if k == 2:
+                _lib.call("omg_backward_project", geom.handle, 0, n, ptr(y), ptr(back), None, None)
+        for t in ts if threads else ():
+            t.join()
+        torch.cuda.synchronize()
+        for o, w in zip(out, want):
+            assert torch.equal(o, w)
+        assert rel_l2(back.cpu().numpy(), ref.cpu().numpy()) < BAR
+
+
+def test_captured_projection_outlives_the_buffers(cuda):
+    """Projections captured on a handle with lists keep nothing of the handle's that later calls may grow and free."""
+    import torch
+    grid, x, z = _scanner(20, 20, 9, 24, 20, 70)
+    n = 70 * 480
+    (img,), (y,) = _operands(grid, n, 1)
+    want = torch.empty(n, device="cuda")
+    geom = make_geom(grid, x, z, 24, 20)
+    side = torch.cuda.Stream()
+    call = lambda out: _lib.call("omg_forward_project", geom.handle, 0, n, ptr(img), ptr(out),
+                                 C.c_void_p(torch.cuda.current_stream().cuda_stream))
+    call(want)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        call(y)
+    back, S = torch.zeros(grid.N, device="cuda"), torch.zeros(grid.N, device="cuda")
+    for k in range(3):
+        _lib.call("omg_backward_project", geom.handle, 0, n, ptr(want), ptr(back), ptr(S), None)   # needs more memory
+        img.mul_(1.5)
+        y.zero_()
+        graph.replay()
+        call(want)
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
+    assert list_calls(geom) == (0, 7)     # the captured one traces
