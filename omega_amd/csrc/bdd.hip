@@ -569,7 +569,7 @@ int bdd_forward(const omg_geom* g, int64_t first, int64_t n, const float* img, f
     uint32_t rb = groups < 256 ? 256 / groups : 1;
     while (rb > 1 && rb * row_lds > 40 * 1024) rb--;
     const bool in_lds = rb * row_lds <= 160 * 1024;
-    int rc = scratch_reserve(const_cast<omg_geom*>(g), sy + sx);
+    int rc = scratch_reserve(const_cast<omg_geom*>(g), sy + sx, s);
     if (rc) return rc;
     float* IY = scratch_ptr(g);
     float* IX = scratch_ptr(g) + sy;
@@ -602,7 +602,7 @@ int bdd_backward(const omg_geom* g, int64_t first, int64_t n, const float* yin, 
     const int64_t per = (int64_t)g->d.size_x * g->d.size_y;
     const uint32_t nproj = (uint32_t)(n / per);
     BddArgs a = make_bdd_args(g, first, nproj);
-    int rc = scratch_reserve(const_cast<omg_geom*>(g), (size_t)(a.nRows + 3) * (a.nCols + 3) * nproj);
+    int rc = scratch_reserve(const_cast<omg_geom*>(g), (size_t)(a.nRows + 3) * (a.nCols + 3) * nproj, s);
     if (rc) return rc;
     float* S = scratch_ptr(g);
     hipLaunchKernelGGL(k_sat_sino_cols, dim3(grid_for(a.nRows, 256), nproj), dim3(256), 0, s, a, yin, S);

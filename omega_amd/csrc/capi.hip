@@ -67,18 +67,27 @@ float* scratch_ptr(const omg_geom* g) { return t_fixed ? t_fixed->base + fixed_w
 float* work_ptr(const omg_geom* g) { return t_fixed ? t_fixed->base : g->work; }
 float* q_ptr(const omg_geom* g) { return t_fixed ? t_fixed->base + fixed_work_floats(g) : g->vbp_q; }
 
-bool scratch_fits(const omg_geom* g, size_t floats) {
-    return !t_fixed || fixed_work_floats(g) + floats <= t_fixed->floats;
+bool scratch_fits(const omg_geom* g, size_t floats, hipStream_t s) {
+    if (t_fixed) return fixed_work_floats(g) + floats <= t_fixed->floats;
+    return g->scratch_floats >= floats || !is_capturing(s);
 }
 
-int scratch_reserve(omg_geom* g, size_t floats) {
+int scratch_reserve(omg_geom* g, size_t floats, hipStream_t s) {
     if (t_fixed) return fixed_need(g, floats, "partial images");
-    if (g->scratch_floats >= floats) return OMG_OK;
+    if (g->scratch_floats >= floats) {
+        g->scratch_captured = g->scratch_captured || is_capturing(s);
+        return OMG_OK;
+    }
     if (g->scratch) {
-        OMG_CHECK_HIP(hipDeviceSynchronize());
-        OMG_CHECK_HIP(hipFree(g->scratch));
+        if (g->scratch_captured) {
+            g->retired.push_back(g->scratch);
+        } else {
+            OMG_CHECK_HIP(hipDeviceSynchronize());
+            OMG_CHECK_HIP(hipFree(g->scratch));
+        }
         g->scratch = nullptr;
         g->scratch_floats = 0;
+        g->scratch_captured = false;
     }
     OMG_CHECK_HIP(hipMalloc(reinterpret_cast<void**>(&g->scratch), floats * sizeof(float)));
     g->scratch_floats = floats;
@@ -360,6 +369,7 @@ extern "C" int omg_geom_destroy(omg_geom* g) {
     hipFree(g->index_dev);
     hipFree(g->frames_t);
     hipFree(g->scratch);
+    for (float* p : g->retired) hipFree(p);
     hipFree(g->work);
     bdd_release(g);
     orth_release(g);

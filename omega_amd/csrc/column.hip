@@ -948,9 +948,9 @@ static ColBuffer* col_buffer(ColCache* c, hipStream_t s) {
 }
 
 ColWork::ColWork(const omg_geom* g, size_t floats, hipStream_t s, bool beside) : s_(s) {
-    if (fixed_region_active() ? !scratch_fits(g, floats) : is_capturing(s)) return;
+    if (fixed_region_active() ? !scratch_fits(g, floats, s) : is_capturing(s)) return;
     if (fixed_region_active() || !beside) {
-        if (scratch_reserve(const_cast<omg_geom*>(g), floats) == OMG_OK) p_ = scratch_ptr(g);
+        if (scratch_reserve(const_cast<omg_geom*>(g), floats, s) == OMG_OK) p_ = scratch_ptr(g);
         else (void)hipGetLastError();
         return;
     }

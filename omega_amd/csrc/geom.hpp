@@ -56,6 +56,8 @@ struct omg_geom {
     // Library-owned scratch (floats) for partial images; grown on demand, freed with the handle.
     float* scratch = nullptr;
     size_t scratch_floats = 0;
+    bool scratch_captured = false;        // a graph may hold it; growth then keeps the old buffer in `retired`
+    std::vector<float*> retired;
     // Library-owned work buffers of the fused OSEM iteration: [dU: N][rhs: N][slice map: Nz int32].
     float* work = nullptr;
     size_t work_floats = 0;
@@ -156,12 +158,14 @@ struct FixedRegionGuard {
 // True while the calling thread holds a fixed region (no device allocation may happen).
 bool fixed_region_active();
 
-// Ensures scratch_ptr(g) holds at least `floats` floats (hipMalloc on growth; synchronises the device then).
-int scratch_reserve(omg_geom* g, size_t floats);
+// Ensures scratch_ptr(g) holds at least `floats` floats for launches on s (hipMalloc on growth; synchronises the
+// device then). A buffer that was handed out while s was being captured is kept until the handle ends.
+int scratch_reserve(omg_geom* g, size_t floats, hipStream_t s);
 float* scratch_ptr(const omg_geom* g);
 
-// False when a held fixed region is too small for scratch_reserve(g, floats).
-bool scratch_fits(const omg_geom* g, size_t floats);
+// False when scratch_reserve(g, floats, s) must fail: a held fixed region is too small, or s is being captured and the
+// scratch would have to grow.
+bool scratch_fits(const omg_geom* g, size_t floats, hipStream_t s);
 
 // Ensures work_ptr(g) holds the fused-iteration buffers for an image of N voxels.
 int work_reserve(omg_geom* g, uint32_t N);

@@ -1258,7 +1258,7 @@ static int orth_launch_planar(const omg_geom* g, int64_t first, int64_t n, const
     float* part = nullptr;
     float* part2 = nullptr;
     if (BP) {
-        const int rc = scratch_reserve(const_cast<omg_geom*>(g), (size_t)sh.blocks * Nyx * (SENS ? 2 : 1));
+        const int rc = scratch_reserve(const_cast<omg_geom*>(g), (size_t)sh.blocks * Nyx * (SENS ? 2 : 1), s);
         if (rc) return rc;
         part = scratch_ptr(g);
         part2 = SENS ? scratch_ptr(g) + (size_t)sh.blocks * Nyx : nullptr;

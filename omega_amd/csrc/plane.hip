@@ -644,8 +644,8 @@ static int run_planes(omg_geom* g, const PlanePlan* pl, const PlaneRun& a, const
     const size_t tt = tof ? (size_t)(a.nent + 1) * PL : 0;
     const size_t need = xt + (tof ? tt : rr) + (sens ? rr : 0);
     *done = false;
-    if (!scratch_fits(g, need)) return OMG_OK;
-    int rc = scratch_reserve(g, need);
+    if (!scratch_fits(g, need, s)) return OMG_OK;
+    int rc = scratch_reserve(g, need, s);
     if (rc) return rc;
     *done = true;
     g->plane_calls.fetch_add(1, std::memory_order_relaxed);

@@ -48,7 +48,7 @@ const PlanePlan* plane_plan(const omg_geom* g, hipStream_t s);
 void plane_release(omg_geom* g);
 
 // One OSEM / OSL-OSEM subset iteration from the lists: planes [first, first + n / bins) of distinct slices.
-// *done false: nothing was launched (work memory short in a no-allocation call).
+// *done false: nothing was launched (work memory short in a no-allocation call or under stream capture).
 int plane_subset_iteration(omg_geom* g, const PlanePlan* pl, int64_t first, int64_t n, float* x, const float* meas,
                            const float* add, float* S, int32_t compute_sens, float epps, const float* dU,
                            int32_t positivity, hipStream_t s, bool* done);

@@ -529,7 +529,7 @@ static int launch_planar(const omg_geom* g, int64_t first, int64_t n, const floa
     const uint32_t Nyx = g->d.Nx * g->d.Ny;
     if (BP) {
         const size_t need = (size_t)sh.blocks * Nyx * (SENS ? 2 : 1);
-        int rc = scratch_reserve(const_cast<omg_geom*>(g), need);
+        int rc = scratch_reserve(const_cast<omg_geom*>(g), need, s);
         if (rc) return rc;
         part = scratch_ptr(g);
         part2 = SENS ? scratch_ptr(g) + (size_t)sh.blocks * Nyx : nullptr;
@@ -717,7 +717,7 @@ static int generic_osem(const omg_geom* g, int64_t first, int64_t n, const float
     float *rhs_t = nullptr, *sens_t = nullptr;
     const uint32_t N = g->d.Nx * g->d.Ny * g->d.Nz;
     if (split_layout(g)) {   // y-fastest accumulators only (see generic_fp)
-        const int rc = scratch_reserve(const_cast<omg_geom*>(g), (size_t)N * (sens ? 2 : 1));
+        const int rc = scratch_reserve(const_cast<omg_geom*>(g), (size_t)N * (sens ? 2 : 1), s);
         if (rc) return rc;
         float* t = scratch_ptr(g);
         hipLaunchKernelGGL(k_fill_f32, dim3(grid_for((int64_t)N * (sens ? 2 : 1), 256)), dim3(256), 0, s, t,
@@ -803,7 +803,7 @@ extern "C" int omg_backward_project(const omg_geom* g, int64_t first, int64_t n_
     if (split_layout(g)) {
         // x-major LORs into y-fastest buffers (scratch), added back transposed
         const uint32_t N = g->d.Nx * g->d.Ny * g->d.Nz;
-        rc = scratch_reserve(const_cast<omg_geom*>(g), (size_t)N * (sens ? 2 : 1));
+        rc = scratch_reserve(const_cast<omg_geom*>(g), (size_t)N * (sens ? 2 : 1), s);
         if (rc) return rc;
         float* rt = scratch_ptr(g);
         float* st = sens ? scratch_ptr(g) + N : nullptr;

@@ -8,6 +8,8 @@ grouping and a second chunk of planes; images that are odd, non-square and small
 outside the image; two planes of one slice (where the lists do not apply); every register group of TOF bins; the
 interpolation projector's far-face samples, which carry into the next slice.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -127,3 +129,40 @@ def test_rows_past_the_slice(cuda, descending, tof):
     _compare(grid, x, z, 29, 28, 0, 9, lists=not tof, **kw)
     grid, x, z = _scanner(9, 34, 10, 29, 28)          # over more than one slice
     _compare(grid, x, z[::-1] if descending else z, 29, 28, 1, 8, lists=not tof, **kw)
+
+
+def test_captured_iterations(cuda):
+    """Iterations captured on a handle with lists: one whose work memory later calls outgrow, and one that would have to
+    grow it while capturing. Replays between eager work give what the same iterations give eagerly."""
+    import torch
+    grid, x, z = _scanner(22, 19, 10, 24, 21)
+    per, bins = 24 * 21, 5
+    geom = make_geom(grid, x, z, 24, 21,
+                     tof=(bins, G.tof_sigma(300e-12), np.linspace(-40.0, 40.0, bins).astype(np.float32), EPPS))
+    meas = torch.poisson(torch.full((9 * per * bins,), 3.0, device="cuda"))
+    side = torch.cuda.Stream()
+
+    def iterate(img, S, planes, sens=1):
+        _lib.call("omg_osem_subset_iteration_ex", geom.handle, 0, planes * per, ptr(img), ptr(meas), None, ptr(S), sens,
+                  EPPS, 0.0, 2.0, 1, C.c_void_p(torch.cuda.current_stream().cuda_stream))
+
+    start = torch.rand(grid.N, device="cuda") + 0.5
+    iterate(start.clone(), torch.zeros(grid.N, device="cuda"), 1)      # lists, and work memory for one plane
+    buf = [(torch.zeros(grid.N, device="cuda"), torch.zeros(grid.N, device="cuda")) for _ in range(2)]
+    torch.cuda.synchronize()
+    graphs = []
+    for (img, S), planes in zip(buf, (1, 9)):                          # the second is captured tracing
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1], stream=side):
+            iterate(img, S, planes)
+    assert list_calls(geom) == (2, 0)
+    for k in range(3):
+        for (img, S), planes, graph in zip(buf, (1, 9), graphs):
+            want, Sw = start.clone(), torch.zeros(grid.N, device="cuda")
+            iterate(want, Sw, planes)                                  # outgrows the memory of the first graph
+            img.copy_(start)
+            S.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert rel_l2(img.cpu().numpy(), want.cpu().numpy()) < 5e-6
+            assert rel_l2(S.cpu().numpy(), Sw.cpu().numpy()) < 5e-6
