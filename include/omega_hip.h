@@ -77,7 +77,8 @@ typedef struct omg_geom_desc {
      * measurement range's voxel indices and table weights, traced once and then streamed by the
      * projections; 0: 16384 MiB, < 0: off, every call traces the tubes), and of the lists that subset
      * iterations of direct-plane sinograms keep (the voxels and lengths of one plane, shared by all planes;
-     * projectors 1, 2 and 4, built by a handle's first iteration that may allocate). Siddon calls on 32 or more
+     * projectors 1, 2 and 4, built by a handle's first iteration that may allocate) together with the work memory
+     * of such an iteration; where those do not fit, or device memory is short, the LORs are traced. Siddon calls on 32 or more
      * planes of a ring sinogram keep the bins' transaxial crossings likewise (at most 2 GiB, per handle and, with
      * meas_index, per range); reserved[3] != 0 or reserved[4] < 0 turns that off.
      * Zero = automatic. */

@@ -474,7 +474,15 @@ static bool upload_u32(uint32_t** dst, const std::vector<uint32_t>& v, hipStream
            hipMemcpyAsync(*dst, v.data(), v.size() * sizeof(uint32_t), hipMemcpyHostToDevice, s) == hipSuccess;
 }
 
-// Device memory that the lists may take (omg_geom_desc.reserved[4], as the tube lists).
+// Work memory of an iteration in floats: gathered slices; ratios (TOF: per entry, a chunk of planes at a time); weights.
+struct PlaneWork { size_t xt, r, w; };
+static PlaneWork plane_work(const PlanePlan* p, uint32_t chunks, uint32_t pl, bool tof) {
+    const size_t rr = (size_t)(tof ? 1 : chunks) * (p->bins + 1) * pl;
+    return PlaneWork{(size_t)chunks * (p->xrows + 1) * pl, tof ? (size_t)(p->nent + 1) * pl : rr, rr};
+}
+
+// Device memory that the lists may take, with the work memory of an iteration on every plane (omg_geom_desc.reserved[4],
+// as the tube lists).
 static uint64_t plan_budget(const omg_geom* g) {
     const int32_t r = g->d.reserved[4];
     if (r < 0) return 0;
@@ -567,7 +575,11 @@ static bool plan_build(const omg_geom* g, PlanePlan* p, hipStream_t s) {
     if (p->pitch == 4) p->pitch = 8;
     if (p->pitch == 12) p->pitch = 16;
     if (p->pitch == 28) p->pitch = 32;
-    ok = ok && p->nent * (8 + 4 + 4ull * p->pitch) + nc * (8 + 12 + 4) + ns * 16 + 4ull * bins * d.n_proj <= budget;
+    if (ok) {
+        const PlaneWork w = plane_work(p, (d.n_proj + 7) / 8, 8, tof);
+        ok = p->nent * (8 + 4 + 4ull * p->pitch) + nc * (8 + 12 + 4) + ns * 16 + 4ull * bins * d.n_proj +
+                 4ull * (w.xt + w.r + w.w) <= budget;
+    }
     ok = ok && upload_u32(&p->off, off, s) && upload_u32(&p->len, len, s) && upload_u32(&p->coff, coff, s) &&
          upload_u32(&p->clen, clen, s) && dev_alloc(&p->ent, p->nent) && dev_alloc(&p->cent, nc) && dev_alloc(&key, nc) &&
          dev_alloc(&val, nc) && dev_alloc(&p->w, (uint64_t)bins * d.n_proj) && dev_alloc(&p->slice, d.n_proj) &&
@@ -640,18 +652,20 @@ static int run_planes(omg_geom* g, const PlanePlan* pl, const PlaneRun& a, const
                       hipStream_t s, bool* done) {
     const uint32_t chunks = (a.planes + PL - 1) / PL;
     const bool tof = pl->share != nullptr;
-    const size_t xt = (size_t)chunks * (a.xrows + 1) * PL, rr = (size_t)(tof ? 1 : chunks) * (a.bins + 1) * PL;
-    const size_t tt = tof ? (size_t)(a.nent + 1) * PL : 0;
-    const size_t need = xt + (tof ? tt : rr) + (sens ? rr : 0);
+    const PlaneWork w = plane_work(pl, chunks, PL, tof);
+    const size_t need = w.xt + w.r + (sens ? w.w : 0);
     *done = false;
     if (!scratch_fits(g, need, s)) return OMG_OK;
-    int rc = scratch_reserve(g, need, s);
-    if (rc) return rc;
+    if (scratch_reserve(g, need, s) != OMG_OK) {   // device memory short: the tracing kernels need less
+        (void)hipGetLastError();
+        return OMG_OK;
+    }
+    int rc = OMG_OK;
     *done = true;
     g->plane_calls.fetch_add(1, std::memory_order_relaxed);
     float* Xt = scratch_ptr(g);
-    float* R = Xt + xt;
-    float* W = R + (tof ? tt : rr);
+    float* R = Xt + w.xt;
+    float* W = R + w.r;
     hipEvent_t stop;
     timing_begin(s, &stop);
     const dim3 gg(grid_for((int64_t)a.xrows + 1, kPB), chunks);

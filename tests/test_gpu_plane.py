@@ -42,6 +42,28 @@ def _iterate(geom, grid, first, planes, per, meas, add, beta, seed):
     return x.cpu().numpy(), S.cpu().numpy()
 
 
+def _entries(grid, x, z, n_radial, n_angles):
+    """Entries of the row lists of one plane: eight rows side by side, each padded to the longest and to a multiple of 8."""
+    import torch
+    per = n_radial * n_angles
+    geom, counts = make_geom(grid, x, z, n_radial, n_angles), torch.zeros(per, dtype=torch.int32, device="cuda")
+    _lib.call("omg_siddon_trace", geom.handle, 0, per, ptr(counts), None, None, None, None)
+    longest = np.pad(counts.cpu().numpy(), (0, -per % 8)).reshape(-1, 8).max(axis=1)
+    return int((-(-longest // 8) * 64).sum())
+
+
+def _lists_fit(grid, x, z, n_radial, n_angles, mib, tof):
+    """Whether an iteration on one plane runs from lists within ``mib``."""
+    import torch
+    per = n_radial * n_angles
+    geom = make_geom(grid, x, z, n_radial, n_angles, tof=tof, tube_budget_mib=mib)
+    img, S, meas = torch.ones(grid.N, device="cuda"), torch.zeros(grid.N, device="cuda"), torch.ones(per * tof[0], device="cuda")
+    _lib.call("omg_osem_subset_iteration_ex", geom.handle, 0, per, ptr(img), ptr(meas), None, ptr(S), 1, EPPS, 0.0, 2.0, 1,
+              None)
+    torch.cuda.synchronize()
+    return list_calls(geom) == (1, 0)
+
+
 def _compare(grid, x, z, n_radial, n_angles, first, planes, bins=1, beta=0.0, add=False, lists=True, **kw):
     import torch
     per = n_radial * n_angles
@@ -166,3 +188,16 @@ def test_captured_iterations(cuda):
             torch.cuda.synchronize()
             assert rel_l2(img.cpu().numpy(), want.cpu().numpy()) < 5e-6
             assert rel_l2(S.cpu().numpy(), Sw.cpu().numpy()) < 5e-6
+
+
+def test_budget_counts_work_memory(cuda):
+    """17 TOF bins of 48 x 63 LORs: the budget holds the lists (92 bytes per entry, and the pixel lists) and an iteration's
+    sums (32 bytes per entry)."""
+    grid, x, z = _scanner(48, 48, 9, 48, 63)
+    kw = dict(bins=17, tof=(17, G.tof_sigma(300e-12), np.linspace(-80.0, 80.0, 17).astype(np.float32), EPPS))
+    sizes = [m for m in range(8, 33) if _lists_fit(grid, x, z, 48, 63, m, kw["tof"])]
+    print(f"[plane] lists and work memory fit from {sizes[0]} MiB", flush=True)
+    nent = _entries(grid, x, z, 48, 63)
+    print(f"[plane] {nent} entries", flush=True)
+    assert sizes == list(range(sizes[0], 33)) and sizes[0] << 20 > nent * (8 + 4 + 4 * 20 + 32)
+    _compare(grid, x, z, 48, 63, 0, 9, lists=False, tube_budget_mib=sizes[0] - 1, **kw)
