@@ -497,7 +497,8 @@ static bool plan_applies(const omg_geom* g) {
     if (d.projector_type == OMG_PROJ_SIDDON) {
         if (tof && d.tof_bins > 32) return false;      // the bins of a LOR are held in registers
     } else if (d.projector_type == OMG_PROJ_ORTH) {
-        if (!orth_plane_ok(g)) return false;
+        uint32_t plane = 0;
+        if (!orth_plane_ok(g, &plane)) return false;
     } else if (d.projector_type == OMG_PROJ_INTERP) {
         if (tof) return false;
     } else {
@@ -527,11 +528,12 @@ static bool plan_build(const omg_geom* g, PlanePlan* p, hipStream_t s) {
     if (!interp && !orth && !tof && d.Ny > d.Nx && d.Ny <= 16 * d.Nx && d.Ny < 32768) p->npix = std::max(p->nyx, (d.Ny - 1) * d.Ny + d.Nx);
     if (interp) interp_plane_slices(g, p->slice_host);
     else siddon_plane_slices(g, p->slice_host);
-    // The lowest slice: voxels that a walk leaves out behind the image's end are out for every other plane too, so
+    // The lowest slice (the orthogonal projector has its own choice, and square images only): voxels that a walk leaves out behind the image's end are out for every other plane too, so
     // the lists hold (or refuse, plane_put) all that any plane visits.
     uint32_t plane = d.n_proj;
     for (uint32_t q = 0; q < d.n_proj; q++)
         if (p->slice_host[q] >= 0 && (plane == d.n_proj || p->slice_host[q] < p->slice_host[plane])) plane = q;
+    if (orth && !orth_plane_ok(g, &plane)) return false;
     if (plane == d.n_proj || bins == 0) return false;
     const uint64_t budget = plan_budget(g);
 

@@ -67,8 +67,8 @@ int interp_plane_weights(const omg_geom* g, float* w, hipStream_t s);
 // Image slices of the planes as the projector's own arithmetic places them (-1: the plane misses the image).
 void siddon_plane_slices(const omg_geom* g, std::vector<int32_t>& out);
 void interp_plane_slices(const omg_geom* g, std::vector<int32_t>& out);
-// True when every tube of a projector-2 direct-plane sinogram stays in its slice and the planes' offsets from
-// their slice centres are the same float.
-bool orth_plane_ok(const omg_geom* g);
+// True when every tube of a projector-2 direct-plane sinogram stays in its slice and the planes lie at the same offset
+// from their slice centres but for rounding; *plane: the one to trace.
+bool orth_plane_ok(const omg_geom* g, uint32_t* plane);
 
 }  // namespace omg

@@ -20,9 +20,9 @@ pytestmark = pytest.mark.gpu
 EPPS = 1e-5
 
 
-def _scanner(nx, ny, nz, n_radial, n_angles, extra_z=()):
+def _scanner(nx, ny, nz, n_radial, n_angles, extra_z=(), dz=2.5):
     fov = 2.5 * max(nx, ny)
-    grid = G.Grid.from_fov(nx, ny, nz, fov, fov, 2.5 * nz)
+    grid = G.Grid.from_fov(nx, ny, nz, fov, fov, dz * nz)
     x = G.ring_sinogram_xy(n_radial, n_angles, fov / n_radial, 1.25 * fov)
     z = G.direct_planes_z(grid)
     if extra_z:
@@ -201,3 +201,26 @@ def test_budget_counts_work_memory(cuda):
     print(f"[plane] {nent} entries", flush=True)
     assert sizes == list(range(sizes[0], 33)) and sizes[0] << 20 > nent * (8 + 4 + 4 * 20 + 32)
     _compare(grid, x, z, 48, 63, 0, 9, lists=False, tube_budget_mib=sizes[0] - 1, **kw)
+
+
+@pytest.mark.parametrize("dz,nz", [(2.027, 109), (2.425, 63), (3.27, 47), (1.775, 83), (2.4, 62)])
+def test_orthogonal_slice_spacing(cuda, dz, nz):
+    """Slices whose thickness is no short binary fraction: the planes' offsets from their slice centres differ by the
+    rounding of the coordinates and of dz, and the lists are of one of them. A weight differs by
+    at most spread / width (1e-4) where a voxel's centre lies on the LOR, and by less than 1e-7 from 0.1 mm on."""
+    grid, x, z = _scanner(20, 20, nz, 24, 20, dz=dz)
+    z = np.repeat((np.arange(nz) + 0.5) * dz - 0.5 * dz * nz, 2).astype(np.float32)
+    f = np.float32
+    tk = (np.abs(z[::2] - f(grid.bz)) / f(grid.dz)).astype(np.int32).astype(f)
+    off = (f(grid.bz) + tk * f(grid.dz) + f(grid.dz) / f(2)) - z[::2]
+    spread = float(off.max() - off.min())
+    assert spread > 0
+    print(f"[plane] {len(set(off.tolist()))} offsets over {spread:.1e} mm", flush=True)
+    _compare(grid, x, z, 24, 20, nz - 9, 9, projector_type=2, orth_width=1.7, orth_flags=3)
+
+
+def test_orthogonal_offsets_apart(cuda):
+    """Planes that lie at different offsets by more than rounding keep lists of their own."""
+    grid, x, z = _scanner(20, 20, 10, 24, 20)
+    z = z + np.repeat(np.arange(10) * 1e-3, 2).astype(np.float32)
+    _compare(grid, x, z, 24, 20, 0, 9, lists=False, projector_type=2, orth_width=1.7, orth_flags=3)
