@@ -584,12 +584,9 @@ int bdd_forward(const omg_geom* g, int64_t first, int64_t n, const float* img, f
                        slab_y);
     OMG_CHECK_LAUNCH();
     const size_t lds = in_lds ? rb * row_lds : 0;
-    static size_t granted = 64 * 1024;
-    if (lds > granted) {
+    if (lds > 64 * 1024)   // every time: a device's attribute, and any thread's call
         OMG_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_bdd_fp<true>),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        granted = lds;
-    }
     const uint32_t per_view = (a.nRows + rb - 1) / rb * ((groups + 255) / 256);
     const uint32_t per_xcd = (uint32_t)(((uint64_t)per_view * nproj + kXcds - 1) / kXcds);
     hipLaunchKernelGGL(in_lds ? k_bdd_fp<true> : k_bdd_fp<false>, dim3(per_xcd * kXcds), dim3(256), lds, s, a, per_xcd,

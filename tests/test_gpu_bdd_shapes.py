@@ -22,6 +22,7 @@ pytestmark = pytest.mark.gpu
     ((20, 24, 30), 11, 2060, 0.05, 4, 1.0),    # 258 column groups; window passed
     ((112, 110, 111), 90, 200, 0.8, 3, 1.0),   # runs of 4
     ((130, 128, 131), 96, 88, 3.0, 2, 1.0),    # runs of 8, last one partial
+    ((4, 5, 5003), 6, 40, 2.0, 2, 0.01),       # rows of more than 64 KB
     ((4, 5, 10301), 6, 40, 2.0, 2, 0.01),      # more slices than LDS rows
 ])
 def test_shapes_match_oracle(cuda, shape, rows, cols, pitch, views, voxel):
