@@ -229,3 +229,14 @@ def test_training_lowers_loss(cuda):
         net.adam_step(lr=2e-3)
     print(f"  loss {losses[0]:.4e} -> {losses[-1]:.4e}", flush=True)
     assert losses[-1] < 0.5 * losses[0]
+
+
+def test_zero_grad_clears_replaced_entries(cuda):
+    """Gradients that a caller has put in place of the network's own (its own buffers, for instance) are cleared too."""
+    import torch
+    net = UN.UNet3D(8, 8, 8, device=cuda)
+    for k in ("d1a.w", "d1a.b"):
+        net.g[k] = torch.full_like(net.g[k], 3.0)
+    net.g["e1a.w"].fill_(2.0)
+    net.zero_grad()
+    assert all(float(g.abs().max()) == 0.0 for g in net.g.values())
