@@ -414,7 +414,8 @@ using namespace omg;
 struct omg_graph {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    float* rhs_t = nullptr;   // the graph's own y-fastest accumulator stack (frames_split), zeroed by the graph
+    float* rhs_t = nullptr;   // the graph's own y-fastest accumulator stack (frames_split), zeroed by the graph; null
+                              // when every step goes by image columns
     float* work = nullptr;    // its own work memory by image columns
 };
 
@@ -548,26 +549,20 @@ extern "C" int omg_frames_graph_create(const omg_geom* g, int32_t n_subsets, con
     OMG_REQUIRE(std::max(g->d.rays_xy, 1u) * std::max(g->d.rays_z, 1u) == 1, "batched frames trace one ray per LOR");
     const uint32_t N = g->d.Nx * g->d.Ny * g->d.Nz;
     OMG_REQUIRE(n_frames >= 1, "n_frames must be >= 1");
-    float* rhs_t = nullptr;
     const size_t NF = (size_t)N * (size_t)n_frames;
-    if (frames_split(g)) OMG_CHECK_HIP(hipMalloc(reinterpret_cast<void**>(&rhs_t), NF * sizeof(float)));
     std::vector<FramesStep> steps((size_t)n_subsets);
     for (int32_t k = 0; k < n_subsets; k++) {
         int rc = meas_offset[k] >= 0 ? OMG_OK : OMG_ERR_ARG;
         if (rc) set_error("negative measurement offset");
         if (!rc)
             rc = make_step(g, first[k], n_meas[k], n_frames, x, meas + meas_offset[k], meas_stride, S + (size_t)k * N,
-                           rhs, rhs_t, dU, beta, gamma, epps, positivity, rays_per_block, frames_per_tile,
+                           rhs, nullptr, dU, beta, gamma, epps, positivity, rays_per_block, frames_per_tile,
                            grid_blocks, steps[(size_t)k]);
-        if (rc) {
-            hipFree(rhs_t);
-            return rc;
-        }
+        if (rc) return rc;
     }
     hipStream_t cs;
     OMG_CHECK_HIP(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
     omg_graph* h = new omg_graph;
-    h->rhs_t = rhs_t;
     size_t work = 0;
     for (FramesStep& st : steps) {
         st.columns = st.a.nmeas > 0 ? col_plan(g, st.first, st.a.nmeas, cs) : nullptr;
@@ -582,12 +577,17 @@ extern "C" int omg_frames_graph_create(const omg_geom* g, int32_t n_subsets, con
         st.timed = false;
         if (!h->work) st.columns = nullptr;
     }
-    hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
+    hipError_t e = hipSuccess;
+    for (const FramesStep& st : steps)
+        if (frames_split(g) && st.a.nmeas > 0 && !st.columns && !h->rhs_t && e == hipSuccess)
+            e = hipMalloc(reinterpret_cast<void**>(&h->rhs_t), NF * sizeof(float));
+    for (FramesStep& st : steps) st.rhs_t = h->rhs_t;
+    if (e == hipSuccess) e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
     int rc = OMG_OK;
     if (e == hipSuccess) {
         hipLaunchKernelGGL(k_frames_fill, dim3((unsigned)((NF + 255) / 256)), dim3(256), 0, cs, rhs, NF, 0.f);
-        if (rhs_t)
-            hipLaunchKernelGGL(k_frames_fill, dim3((unsigned)((NF + 255) / 256)), dim3(256), 0, cs, rhs_t, NF, 0.f);
+        if (h->rhs_t)
+            hipLaunchKernelGGL(k_frames_fill, dim3((unsigned)((NF + 255) / 256)), dim3(256), 0, cs, h->rhs_t, NF, 0.f);
         for (const FramesStep& st : steps) {
             rc = launch_step(st, cs);
             if (rc) break;

@@ -279,3 +279,26 @@ def test_captured_projection_outlives_the_buffers(cuda):
         torch.cuda.synchronize()
         assert torch.equal(y, want)
     assert list_calls(geom) == (0, 7)     # the captured one traces
+
+
+def test_frames_graph_takes_no_stack_it_does_not_use(cuda):
+    """A graph whose steps go by columns holds no accumulator stack of image x frames."""
+    import torch
+    grid, x, z = _scanner(96, 96, 40, 20, 16, 40)
+    frames, n, N = 128, 40 * 320, grid.N
+    g = make_geom(grid, x, z, 20, 16)
+    meas, xs = torch.ones(frames, n, device="cuda"), torch.ones(frames, N, device="cuda")
+    S, rhs = torch.ones(N, device="cuda"), torch.zeros(frames, N, device="cuda")
+    ints = [np.array([v], np.int64) for v in (0, n, 0)]
+    tail = (0.0, 2.0, EPPS, 1, 128, 1, 0)
+    _lib.call("omg_frames_osem_step", g.handle, 0, n, frames, ptr(xs), ptr(meas), n, ptr(S), ptr(rhs), None, *tail, None)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    h = C.c_void_p()
+    _lib.call("omg_frames_graph_create", g.handle, 1, *(v.ctypes.data for v in ints), frames, ptr(xs), ptr(meas), n,
+              ptr(S), ptr(rhs), None, *tail, C.byref(h))
+    took = free - torch.cuda.mem_get_info()[0]
+    _lib.call("omg_graph_destroy", h)
+    print(f"[column] graph took {took >> 20} MiB beside a stack of {rhs.numel() * 4 >> 20} MiB", flush=True)
+    assert list_calls(g) == (0, 2 * frames)
+    assert took < rhs.numel() * 4
