@@ -48,11 +48,14 @@ struct ColPlan {
     uint32_t tw = 0, th = 0, ntx = 0;   // tile width, height; tiles per row
     ColSeg* seg = nullptr;
     ColItem* item = nullptr;
-    uint32_t items = 0, max_segs = 0, tpb = 0;
+    uint32_t items = 0, tpb = 0;
 };
 
+// A bin's records, one group of planes: the largest |value| as float bits, and the sum of the |values|.
+struct ColPeak { uint32_t top; float sum; };
+
 struct ColView {
-    uint32_t bins, planes, tw, th, ntx, max_segs;
+    uint32_t bins, planes, tw, th, ntx;
     const uint32_t* off;
     const ColStart* start;
     const uint2* ent;
@@ -285,6 +288,30 @@ __device__ __forceinline__ void col_pair(ColLane& l, float tc, float tn, uint32_
     }
 }
 
+// A wave's maximum and sum (of values >= 0), in lane 63: rows of 16 lanes first, then lane 15 of rows 0 and 2 into the
+// rows behind, lane 31 into rows 2 and 3.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_or_0(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+}
+template <typename Op>
+__device__ __forceinline__ uint32_t wave_fold(uint32_t v, Op&& op) {
+    v = op(v, dpp_or_0<0x111, 0xf>(v));
+    v = op(v, dpp_or_0<0x112, 0xf>(v));
+    v = op(v, dpp_or_0<0x114, 0xf>(v));
+    v = op(v, dpp_or_0<0x118, 0xf>(v));
+    v = op(v, dpp_or_0<0x142, 0xa>(v));
+    return op(v, dpp_or_0<0x143, 0xc>(v));
+}
+__device__ __forceinline__ ColPeak wave_peak(float v) {
+    v = fabsf(v);
+    const uint32_t top = wave_fold(__float_as_uint(v), [](uint32_t a, uint32_t b) { return max(a, b); });
+    const uint32_t sum = wave_fold(__float_as_uint(v), [](uint32_t a, uint32_t b) {
+        return __float_as_uint(__uint_as_float(a) + __uint_as_float(b));
+    });
+    return ColPeak{top, __uint_as_float(sum)};   // NaN and Inf order above every number
+}
+
 // a * b, and 0 where a factor is 0 whatever the other one is
 __device__ __forceinline__ float mul_or_zero(float a, float b) {
     float r;
@@ -296,8 +323,8 @@ enum { COL_FP = 0, COL_OSEM = 1, COL_BP = 2 };
 
 // One wave per bin and 64 planes, BPW bins one after the other. COL_FP: y = A img. COL_BP: the lanes' records for
 // k_col_bp, {z walk, length, y * weight (weight alone when y is null)}, and with wrec the weights beside them.
-// COL_OSEM: forward projection, ratio, records. state: {largest |value| of the records as float bits, irregular LORs
-// listed in `rest`, largest weight}. Measurements pass through LDS (a wave's lanes are a whole plane apart in
+// COL_OSEM: forward projection, ratio, records. peak, wpeak: each bin's of rec and wrec. state[1]: irregular LORs listed in
+// `rest`. Measurements pass through LDS (a wave's lanes are a whole plane apart in
 // them). A column of up to 64 NR - 1 slices is loaded into the wave's registers, lane z holding slice z, and every
 // lane picks its slices by ds_bpermute; NR 0: lanes gather from memory. What bounds the forward projection: VALU,
 // about 22 operations per column and 64 LORs besides 690 per LOR's set-up. 64 planes of 224 x 224 bins, 128 x 128 x 63:
@@ -306,8 +333,8 @@ enum { COL_FP = 0, COL_OSEM = 1, COL_BP = 2 };
 template <int MODE, int BPW, int NR>
 __global__ __launch_bounds__(256, MODE == COL_BP || NR > 1 ? 4 : MODE == COL_FP ? 6 : 5) void k_col_fp(
     ColView c, SidArgs a, uint32_t plane0, const float* __restrict__ Xz, const float* __restrict__ yin,
-    float* __restrict__ yout, float4* __restrict__ rec, float* __restrict__ wrec, uint32_t* __restrict__ state,
-    uint32_t* __restrict__ rest, float epps) {
+    float* __restrict__ yout, float4* __restrict__ rec, float* __restrict__ wrec, ColPeak* __restrict__ peak,
+    ColPeak* __restrict__ wpeak, uint32_t* __restrict__ state, uint32_t* __restrict__ rest, float epps) {
     constexpr uint32_t NB = 4 * BPW;
     __shared__ float ys[kCL][NB + 1];
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -325,7 +352,6 @@ __global__ __launch_bounds__(256, MODE == COL_BP || NR > 1 ? 4 : MODE == COL_FP 
     const uint32_t zp = NR ? 64u * NR : a.Nz + 2;
     const __amdgpu_buffer_rsrc_t cols = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(Xz), 0, NR ? (int)(a.Nx * a.Ny * 256u * NR) : 0, 0x00027000);
-    uint32_t top = 0, topw = 0;
     for (uint32_t i = 0; i < BPW; i++) {
         const uint32_t b = wave * BPW + i, bin = bin0 + b;
         if (bin >= c.bins) break;
@@ -464,11 +490,13 @@ __global__ __launch_bounds__(256, MODE == COL_BP || NR > 1 ? 4 : MODE == COL_FP 
         const uint32_t steep = reg && col_steep(w) ? 0x8000u : 0u;
         rec[((size_t)blockIdx.y * c.bins + bin) * kCL + lane] =
             make_float4(w.tz0, w.L, keep, __uint_as_float((uint32_t)(w.tk + 1) | steep | w.left << 16));
-        top = max(top, __float_as_uint(keep) & 0x7fffffffu);   // NaN and Inf order above every number
+        const ColPeak pk = wave_peak(keep);
+        if (lane == 63) peak[(size_t)blockIdx.y * c.bins + bin] = pk;
         if (wrec) {
             const float kw = reg ? weight : 0.f;
             wrec[((size_t)blockIdx.y * c.bins + bin) * kCL + lane] = kw;
-            topw = max(topw, __float_as_uint(kw) & 0x7fffffffu);
+            const ColPeak pw = wave_peak(kw);
+            if (lane == 63) wpeak[(size_t)blockIdx.y * c.bins + bin] = pw;
         }
     }
     if (MODE == COL_FP) {
@@ -477,17 +505,7 @@ __global__ __launch_bounds__(256, MODE == COL_BP || NR > 1 ? 4 : MODE == COL_FP 
             const uint32_t b = t % NB, q = t / NB;
             if (bin0 + b < c.bins && pg + q < c.planes) yout[(int64_t)(pg + q) * c.bins + bin0 + b] = ys[q][b];
         }
-        return;
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        top = max(top, (uint32_t)__shfl_xor((int)top, o, 64));
-        topw = max(topw, (uint32_t)__shfl_xor((int)topw, o, 64));
-    }
-    auto raise = [&](uint32_t* at, uint32_t v) {
-        if (lane == 0 && v > __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(at, v);
-    };
-    raise(state, top);
-    if (wrec) raise(state + 2, topw);
 }
 
 // The irregular LORs of a k_col_fp launch, one per lane, by the walk of the one-lane-per-LOR kernels: thread `i` of
@@ -536,9 +554,12 @@ __global__ __launch_bounds__(64) void k_col_rest(SidArgs a, const uint32_t* __re
 // 128 x 128 x 63: 281 us, with the records' launch 355 us; 5690 us by one lane per LOR (global float atomics).
 __global__ __launch_bounds__(1024, 8) void k_col_bp(ColView c, SidArgs a, uint32_t plane0, uint32_t rest_blocks,
                                                     ColRest rest, const float4* __restrict__ rec,
-                                                    const float* __restrict__ wrec,
+                                                    const float* __restrict__ wrec, const ColPeak* __restrict__ peak,
+                                                    const ColPeak* __restrict__ wpeak,
                                                     const uint32_t* __restrict__ state) {
     extern __shared__ unsigned long long acc64[];
+    __shared__ uint32_t most[16], least[16];
+    __shared__ float total[16];
     if (blockIdx.x < rest_blocks) {
         if (blockIdx.y + blockIdx.z == 0)
             col_rest(a, rest, state[1], blockIdx.x * blockDim.x + threadIdx.x, rest_blocks * blockDim.x);
@@ -550,19 +571,47 @@ __global__ __launch_bounds__(1024, 8) void k_col_bp(ColView c, SidArgs a, uint32
     const uint32_t x0 = it.tile % c.ntx * c.tw, y0 = it.tile / c.ntx * c.th;
     const uint32_t zp = a.Nz + 2, cells = c.tw * c.th * zp;
     for (uint32_t i = threadIdx.x; i < cells; i += blockDim.x) acc64[i] = 0ull;
-    const uint32_t pk = state[sens ? 2 : 0];
-    bool finite = pk < 0x7f800000u;
-    // |term| <= peak * voxel diagonal; a segment adds at most two terms to a voxel per lane, and an item holds at
-    // most max_segs segments of 64 lanes
+    // The item's own scale: |term| <= peak * voxel diagonal, and a segment adds at most two terms to a voxel per lane.
+    // One outlying LOR so costs bits where it passes only, and of its own size (the sum of the records bounds a voxel's,
+    // not their number times the largest). Where not even the bins' largest terms keep 20 bits, the item adds floats.
+    uint32_t top = 0, low = ~0u;
+    float sum = 0.f;
+    for (uint32_t q = it.s0 + threadIdx.x; q < it.s1; q += blockDim.x) {
+        const ColPeak pk = (sens ? wpeak : peak)[(size_t)blockIdx.y * c.bins + c.seg[q].bin];
+        top = max(top, pk.top);
+        low = min(low, pk.top ? pk.top : ~0u);
+        sum += pk.sum;
+    }
+    top = wave_fold(top, [](uint32_t a, uint32_t b) { return max(a, b); });
+    low = ~wave_fold(~low, [](uint32_t a, uint32_t b) { return max(a, b); });
+    sum = __uint_as_float(wave_fold(__float_as_uint(sum), [](uint32_t a, uint32_t b) {
+        return __float_as_uint(__uint_as_float(a) + __uint_as_float(b));
+    }));
+    if ((threadIdx.x & 63) == 63) {
+        most[threadIdx.x >> 6] = top;
+        least[threadIdx.x >> 6] = low;
+        total[threadIdx.x >> 6] = sum;
+    }
+    __syncthreads();
+    top = most[0];
+    low = least[0];
+    sum = total[0];
+    for (uint32_t q = 1; q < blockDim.x >> 6; q++) {
+        top = max(top, most[q]);
+        low = min(low, least[q]);
+        sum += total[q];
+    }
+    if (top == 0u) return;
+    bool finite = top < 0x7f800000u;
     double up, down;
     {
         const float diag = sqrtf(a.dx * a.dx + a.dy * a.dy + a.dz * a.dz) * (1.f + 0x1p-10f);
-        const float bt = finite ? __uint_as_float(pk) * diag : 1.f;
-        const float bs = bt * (2.f * kCL * (float)c.max_segs);
+        const float bt = finite ? __uint_as_float(top) * diag : 1.f;
+        const float bs = 2.f * sum * diag * (1.f + 0x1p-10f);
         finite = finite && bs < __builtin_inff();
-        fixed_scale(bt, bs, up, down);
+        fixed_scale(bt, finite ? fmaxf(bs, bt) : 1.f, up, down);
+        finite = finite && (double)(__uint_as_float(low) * diag) * up >= 0x1p20;
     }
-    __syncthreads();
     const uint32_t lane = threadIdx.x & 63, p = plane0 + blockIdx.y * kCL + lane;
     ColLane l;
     float tzi = 0.f;
@@ -789,7 +838,6 @@ static bool col_build(const omg_geom* g, ColPlan* p, hipStream_t s) {
         for (uint32_t q = 0; q < parts; q++) {
             const uint32_t s0 = (uint32_t)((uint64_t)ht[t] * q / parts), s1 = (uint32_t)((uint64_t)ht[t] * (q + 1) / parts);
             items.push_back(ColItem{t, toff[t] + s0, toff[t] + s1});
-            p->max_segs = std::max(p->max_segs, s1 - s0);
         }
     }
     p->items = (uint32_t)items.size();
@@ -862,7 +910,7 @@ void col_release(omg_geom* g) {
 }
 
 // Work memory: [z-fastest image: Nx Ny pitch][records: 4 floats x bins x 64 x plane groups per pass][weights, with
-// sens][irregular LORs][state: 4].
+// sens][the bins' peaks, of the weights too with sens][irregular LORs][state: 4].
 constexpr uint64_t kColRecords = 8ull << 20;      // records per pass (128 MB): plane groups beyond take more passes
 
 // Bins per wave: one where the wave walks (a lane's chain of columns is long, so the last waves would leave the chip
@@ -870,11 +918,11 @@ constexpr uint64_t kColRecords = 8ull << 20;      // records per pass (128 MB): 
 // 73 against 84 us with two).
 template <int MODE>
 static void col_launch_fp(const ColView& c, const SidArgs& a, uint32_t g0, uint32_t groups, uint32_t nr, const float* Xz,
-                          const float* yin, float* yout, float4* rec, float* wrec, uint32_t* state, uint32_t* rest,
-                          float epps, hipStream_t s) {
+                          const float* yin, float* yout, float4* rec, float* wrec, ColPeak* peak,
+                          ColPeak* wpeak, uint32_t* state, uint32_t* rest, float epps, hipStream_t s) {
     auto launch = [&](auto kern, uint32_t nb) {
         hipLaunchKernelGGL(kern, dim3((c.bins + nb - 1) / nb, groups), dim3(256), 0, s, c, a, g0 * kCL, Xz, yin, yout, rec,
-                           wrec, state, rest, epps);
+                           wrec, peak, wpeak, state, rest, epps);
     };
     if (MODE == COL_BP) launch(k_col_fp<MODE, MODE == COL_BP ? 4 : 1, 1>, 16);
     else if (nr == 1) launch(k_col_fp<MODE, 1, 1>, 4);
@@ -885,7 +933,7 @@ static void col_launch_fp(const ColView& c, const SidArgs& a, uint32_t g0, uint3
 struct ColLayout {
     uint32_t nr, pitch, all, pass;
     uint64_t per;
-    size_t nimg, nrec, nw, need;
+    size_t nimg, nrec, nw, npeak, need;
 };
 
 static ColLayout col_layout(const omg_geom* g, const ColPlan* pl, int64_t n, bool img, bool rec, bool sens) {
@@ -900,7 +948,8 @@ static ColLayout col_layout(const omg_geom* g, const ColPlan* pl, int64_t n, boo
     w.nimg = img ? ((size_t)d.Nx * d.Ny * w.pitch + 3) & ~(size_t)3 : 0;
     w.nrec = rec ? 4 * w.per * w.pass : 0;
     w.nw = sens ? w.per * w.pass : 0;
-    w.need = w.nimg + w.nrec + w.nw + w.per * w.pass + 4;
+    w.npeak = rec ? 2 * (size_t)pl->bins * w.pass : 0;   // of one kind
+    w.need = w.nimg + w.nrec + w.nw + (sens ? 2 : 1) * w.npeak + w.per * w.pass + 4;
     return w;
 }
 
@@ -990,7 +1039,7 @@ static int col_run(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t 
                    float* yout, const float* add, float* rhs, float* sens, float epps, float* work, hipStream_t s,
                    bool timed) {
     const omg_geom_desc& d = g->d;
-    const ColView c{pl->bins, (uint32_t)(n / pl->bins), pl->tw, pl->th, pl->ntx, pl->max_segs,
+    const ColView c{pl->bins, (uint32_t)(n / pl->bins), pl->tw, pl->th, pl->ntx,
                     pl->off, pl->start, pl->ent, pl->seg, pl->item};
     SidArgs a = make_sid_args(g, first, n);
     a.plane_col = g->index_dev ? 0 : first;   // the z table's first plane (an index table's range holds every plane)
@@ -1001,7 +1050,9 @@ static int col_run(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t 
     float* Xz = work;
     float4* rec = reinterpret_cast<float4*>(Xz + w.nimg);
     float* wrec = sens ? Xz + w.nimg + w.nrec : nullptr;
-    uint32_t* rest = reinterpret_cast<uint32_t*>(Xz + w.nimg + w.nrec + w.nw);
+    ColPeak* peak = reinterpret_cast<ColPeak*>(Xz + w.nimg + w.nrec + w.nw);
+    ColPeak* wpeak = sens ? peak + w.npeak / 2 : nullptr;
+    uint32_t* rest = reinterpret_cast<uint32_t*>(peak + (sens ? 2 : 1) * (w.npeak / 2));
     uint32_t* state = rest + w.per * pass;
     const size_t lds = col_lds(c.tw, c.th, d.Nz);
     hipEvent_t stop = nullptr;
@@ -1016,16 +1067,16 @@ static int col_run(const omg_geom* g, const ColPlan* pl, int64_t first, int64_t 
             hipLaunchKernelGGL(k_col_zero, dim3(1), dim3(256), 0, s, state, 4u);
             OMG_CHECK_LAUNCH();
         }
-        if (yout) col_launch_fp<COL_FP>(c, a, g0, groups, nr, Xz, yin, yout, rec, wrec, state, rest, epps, s);
-        else if (img) col_launch_fp<COL_OSEM>(c, a, g0, groups, nr, Xz, yin, yout, rec, wrec, state, rest, epps, s);
-        else col_launch_fp<COL_BP>(c, a, g0, groups, nr, Xz, yin, yout, rec, wrec, state, rest, epps, s);
+        if (yout) col_launch_fp<COL_FP>(c, a, g0, groups, nr, Xz, yin, yout, rec, wrec, peak, wpeak, state, rest, epps, s);
+        else if (img) col_launch_fp<COL_OSEM>(c, a, g0, groups, nr, Xz, yin, yout, rec, wrec, peak, wpeak, state, rest, epps, s);
+        else col_launch_fp<COL_BP>(c, a, g0, groups, nr, Xz, yin, yout, rec, wrec, peak, wpeak, state, rest, epps, s);
         OMG_CHECK_LAUNCH();
         const ColRest r{rest, img, yin, yout, rhs, sens, epps};
         if (yout) {
             hipLaunchKernelGGL(k_col_rest, dim3(1024), dim3(64), 0, s, a, state, r);
         } else {
             hipLaunchKernelGGL(k_col_bp, dim3(kColRest + pl->items, groups, sens ? 2 : 1), dim3(pl->tpb), lds, s,
-                               c, a, g0 * kCL, kColRest, r, rec, wrec, state);
+                               c, a, g0 * kCL, kColRest, r, rec, wrec, peak, wpeak, state);
         }
         OMG_CHECK_LAUNCH();
     }

@@ -131,6 +131,32 @@ def test_not_finite(cuda):
         assert rel_l2(p[ok], q[ok]) < BAR
 
 
+@pytest.mark.parametrize("outlier", [2.0 ** 24, 2.0 ** 40, 1e30, 1e-30])
+def test_range_of_values(cuda, outlier):
+    """One LOR whose value is far from the others': the voxels beside it are as good as without it."""
+    import torch
+    grid, x, z = _scanner(33, 40, 15, 32, 30, 70)
+    n = 70 * 960
+    y = np.random.default_rng(6).random(n).astype(np.float32) + 0.5
+    only = np.zeros(n, np.float32)
+    only[37 * 960 + 15 * 32 + 14] = y[37 * 960 + 15 * 32 + 14] = outlier
+    out = []
+    for gen in (False, True):
+        geom = make_geom(grid, x, z, 32, 30, generic=gen)
+        back, path = torch.zeros(grid.N, device="cuda"), torch.zeros(grid.N, device="cuda")
+        for v, to in ((y, back), (only, path)):
+            _lib.call("omg_backward_project", geom.handle, 0, n, ptr(torch.from_numpy(v).cuda()), ptr(to), None, None)
+        torch.cuda.synchronize()
+        out.append((back.cpu().numpy(), path.cpu().numpy()))
+        assert list_calls(geom) == (0, 0 if gen else 2)
+    (a, pa), (b, pb) = out
+    assert rel_l2(pa, pb) < BAR and np.count_nonzero(pb) > 20
+    beside = pb == 0
+    e = rel_l2(a[beside], b[beside]), rel_l2(a[~beside], b[~beside])
+    print(f"[column] outlier {outlier:.1e}: rel-L2 {e}", flush=True)
+    assert max(e) < BAR
+
+
 @pytest.mark.parametrize("frames,planes", [(1, 40), (4, 64), (3, 97)])
 def test_frames(cuda, frames, planes):
     """Two subset steps of a dynamic study, launched and replayed from a graph."""
