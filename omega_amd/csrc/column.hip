@@ -23,6 +23,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <memory>
 #include <mutex>
 #include <new>
@@ -42,7 +43,7 @@ struct ColPlan {
     bool ok = false;
     uint32_t bins = 0;
     const uint32_t* bin_of = nullptr;   // measurement-level subsets: the range's first plane in the index table
-    uint32_t* off = nullptr;            // [bins + 1]
+    uint32_t* off = nullptr;            // [bins + 1]; the allocation that holds the other lists too
     ColStart* start = nullptr;
     uint2* ent = nullptr;               // {x | y << 16, exit parameter}
     uint32_t tw = 0, th = 0, ntx = 0;   // tile width, height; tiles per row
@@ -121,33 +122,37 @@ __device__ __forceinline__ bool col_walk(const SidArgs& a, uint32_t j, ColStart&
 
 // One lane per bin. Counting pass (ent null): entries, and segments per tile. Filling pass: the lists, and the
 // segments in their tiles' ranges. The tiles' counters are shared by every bin, so a workgroup adds its own
-// counts (LDS, up to kTileLds tiles) once.
+// counts (LDS, up to kTileLds tiles) once; they stay in group_cnt [workgroups][tiles] for the filling pass.
 constexpr uint32_t kTileLds = 2048;
 
 __global__ __launch_bounds__(256) void k_col_trace(SidArgs a, uint32_t bins, uint32_t tw, uint32_t th, uint32_t ntx,
                                                    uint32_t tiles, uint32_t* __restrict__ cnt,
-                                                   uint32_t* __restrict__ tile_cnt, const uint32_t* __restrict__ off,
-                                                   ColStart* __restrict__ start, uint2* __restrict__ ent,
-                                                   const uint32_t* __restrict__ tile_off, ColSeg* __restrict__ seg) {
+                                                   uint32_t* __restrict__ tile_cnt, uint32_t* __restrict__ group_cnt,
+                                                   const uint32_t* __restrict__ off, ColStart* __restrict__ start,
+                                                   uint2* __restrict__ ent, const uint32_t* __restrict__ tile_off,
+                                                   ColSeg* __restrict__ seg) {
     __shared__ uint32_t mine[kTileLds];
     const uint32_t j = blockIdx.x * 256 + threadIdx.x;
     const bool shared = tiles <= kTileLds;
-    for (uint32_t i = threadIdx.x; i < (shared ? tiles : 0u); i += 256) mine[i] = 0u;
+    uint32_t* group = group_cnt + (size_t)blockIdx.x * tiles;
+    for (uint32_t i = threadIdx.x; i < (shared ? tiles : 0u); i += 256) mine[i] = ent ? group[i] : 0u;
     __syncthreads();
     ColStart st;
     uint32_t n = 0, tile = 0xffffffffu;
-    if (j < bins && (shared || !ent)) {
+    if (j < bins && !ent) {
         col_walk(a, j, st, [&](uint32_t xy, float) {
             const uint32_t t = col_tile(xy, tw, th, ntx);
             if (t != tile) atomicAdd(shared ? mine + t : tile_cnt + t, 1u);
             tile = t;
             n++;
         });
-        if (!ent) cnt[j] = n;
+        cnt[j] = n;
     }
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < (shared ? tiles : 0u); i += 256)   // counts -> this workgroup's first slot
-        if (mine[i]) mine[i] = atomicAdd(tile_cnt + i, mine[i]);
+    for (uint32_t i = threadIdx.x; i < (shared ? tiles : 0u); i += 256) {
+        if (!ent) group[i] = mine[i];
+        if (mine[i]) mine[i] = atomicAdd(tile_cnt + i, mine[i]);   // filling pass: this workgroup's first slot
+    }
     if (!ent) return;
     __syncthreads();
     if (j >= bins) return;
@@ -732,7 +737,7 @@ struct ColCache {
 };
 
 static void col_free(ColPlan* p) {
-    hipFree(p->off); hipFree(p->start); hipFree(p->ent); hipFree(p->seg); hipFree(p->item);
+    hipFree(p->off);
     p->off = nullptr; p->start = nullptr; p->ent = nullptr; p->seg = nullptr; p->item = nullptr;
 }
 
@@ -777,46 +782,40 @@ static bool col_build(const omg_geom* g, ColPlan* p, hipStream_t s) {
     }
     p->ntx = (d.Nx + p->tw - 1) / p->tw;
     const uint32_t tiles = p->ntx * ((d.Ny + p->th - 1) / p->th);
-    uint32_t *cnt = nullptr, *tile_cnt = nullptr, *tile_off = nullptr;
-    bool ok = true;
     if (g->index_dev) {      // the range has to be the same bins of every plane
         p->bins = d.n_proj && p->n % d.n_proj == 0 ? (uint32_t)(p->n / d.n_proj) : 0u;
         if (p->bins == 0 || p->bins > per) return false;
         p->bin_of = g->index_dev + p->first;
-        int32_t bad = 0;
-        ok = col_alloc(&cnt, 1);
-        if (ok) {
-            hipLaunchKernelGGL(k_col_zero, dim3(1), dim3(256), 0, s, cnt, 1u);
-            hipLaunchKernelGGL(k_col_check, dim3(grid_for(p->n, 256)), dim3(256), 0, s, p->bin_of, (uint64_t)p->n, p->bins,
-                               per, reinterpret_cast<int32_t*>(cnt));
-            ok = hipMemcpyAsync(&bad, cnt, 4, hipMemcpyDeviceToHost, s) == hipSuccess &&
-                 hipStreamSynchronize(s) == hipSuccess && !bad;
-        }
-        hipFree(cnt);
-        cnt = nullptr;
-        if (!ok) return false;
     } else {
         p->bins = per;
     }
-    SidArgs a = make_sid_args(g, g->index_dev ? p->first : 0, p->bins);
-    const dim3 grid(grid_for(p->bins, 256)), block(256);
-    std::vector<uint32_t> hc(p->bins), ht(tiles), off((size_t)p->bins + 1), toff(tiles);
-    ok = col_alloc(&cnt, p->bins) && col_alloc(&tile_cnt, tiles);
+    const uint32_t bins = p->bins;
+    SidArgs a = make_sid_args(g, g->index_dev ? p->first : 0, bins);
+    const dim3 grid(grid_for(bins, 256)), block(256);
+    // counts, read back together: [bins][tiles][bad], and behind them [tiles again, for the filling pass][workgroups][tiles]
+    uint32_t* cnt = nullptr;
+    std::vector<uint32_t> host((size_t)bins + tiles + 1);
+    bool ok = col_alloc(&cnt, (uint64_t)bins + 2ull * tiles + 1 + (tiles <= kTileLds ? (uint64_t)grid.x * tiles : 0));
+    uint32_t *tile_cnt = cnt + bins, *bad = tile_cnt + tiles, *tile_cur = bad + 1, *group_cnt = tile_cur + tiles;
     if (ok) {
-        hipLaunchKernelGGL(k_col_zero, dim3(grid_for(tiles, 256)), dim3(256), 0, s, tile_cnt, tiles);
-        hipLaunchKernelGGL(k_col_trace, grid, block, 0, s, a, p->bins, p->tw, p->th, p->ntx, tiles, cnt, tile_cnt, nullptr,
-                           nullptr, nullptr, nullptr, nullptr);
-        ok = hipMemcpyAsync(hc.data(), cnt, p->bins * 4ull, hipMemcpyDeviceToHost, s) == hipSuccess &&
-             hipMemcpyAsync(ht.data(), tile_cnt, tiles * 4ull, hipMemcpyDeviceToHost, s) == hipSuccess &&
-             hipStreamSynchronize(s) == hipSuccess;
+        hipLaunchKernelGGL(k_col_zero, dim3(grid_for(2ll * tiles + 1, 256)), dim3(256), 0, s, tile_cnt, 2 * tiles + 1);
+        if (g->index_dev)
+            hipLaunchKernelGGL(k_col_check, dim3(grid_for(p->n, 256)), dim3(256), 0, s, p->bin_of, (uint64_t)p->n, bins,
+                               per, reinterpret_cast<int32_t*>(bad));
+        hipLaunchKernelGGL(k_col_trace, grid, block, 0, s, a, bins, p->tw, p->th, p->ntx, tiles, cnt, tile_cnt,
+                           group_cnt, nullptr, nullptr, nullptr, nullptr, nullptr);
+        ok = hipMemcpyAsync(host.data(), cnt, host.size() * 4, hipMemcpyDeviceToHost, s) == hipSuccess &&
+             hipStreamSynchronize(s) == hipSuccess && host.back() == 0;
     }
+    const uint32_t *hc = host.data(), *ht = hc + bins;
+    std::vector<uint32_t> off((size_t)bins + 1), toff(tiles), tables;
     uint64_t total = 0, segs = 0;
-    for (uint32_t j = 0; j < p->bins && ok; j++) {
+    for (uint32_t j = 0; j < bins && ok; j++) {
         off[j] = (uint32_t)total;
         total += hc[j];
         if (total >= 0xFFFFFFF0ull) ok = false;
     }
-    off[p->bins] = (uint32_t)total;
+    off[bins] = (uint32_t)total;
     for (uint32_t t = 0; t < tiles; t++) {
         toff[t] = (uint32_t)segs;
         segs += ht[t];
@@ -841,20 +840,32 @@ static bool col_build(const omg_geom* g, ColPlan* p, hipStream_t s) {
         }
     }
     p->items = (uint32_t)items.size();
-    ok = ok && p->items > 0 && col_alloc(&p->off, off.size()) && col_alloc(&p->start, p->bins) &&
-         col_alloc(&p->ent, total + 4) &&
-         col_alloc(&p->seg, segs) && col_alloc(&p->item, items.size()) && col_alloc(&tile_off, tiles) &&
-         hipMemcpyAsync(p->off, off.data(), off.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
-         hipMemcpyAsync(tile_off, toff.data(), tiles * 4ull, hipMemcpyHostToDevice, s) == hipSuccess &&
-         hipMemcpyAsync(p->item, items.data(), items.size() * sizeof(ColItem), hipMemcpyHostToDevice, s) == hipSuccess;
+    ok = ok && p->items > 0;
     if (ok) {
-        hipLaunchKernelGGL(k_col_zero, dim3(grid_for(tiles, 256)), dim3(256), 0, s, tile_cnt, tiles);
-        hipLaunchKernelGGL(k_col_trace, grid, block, 0, s, a, p->bins, p->tw, p->th, p->ntx, tiles, cnt, tile_cnt, p->off,
-                           p->start, p->ent, tile_off, p->seg);
-        ok = hipGetLastError() == hipSuccess && hipStreamSynchronize(s) == hipSuccess;
+        // one allocation, the tables that the host made in front, uploaded by one copy
+        auto round = [](size_t n) { return (n + 3) & ~(size_t)3; };
+        const size_t at_toff = round(off.size()), at_item = at_toff + round(tiles);
+        const size_t at_start = at_item + round(3 * items.size());
+        const size_t at_ent = at_start + 4 * (size_t)bins, at_seg = at_ent + 2 * (total + 4);
+        tables.assign(at_start, 0u);
+        std::copy(off.begin(), off.end(), tables.begin());
+        std::copy(toff.begin(), toff.end(), tables.begin() + (ptrdiff_t)at_toff);
+        static_assert(sizeof(ColItem) == 12 && sizeof(ColSeg) == 12 && sizeof(ColStart) == 16, "table layout");
+        std::memcpy(tables.data() + at_item, items.data(), items.size() * sizeof(ColItem));
+        ok = col_alloc(&p->off, at_seg + 3 * segs) &&
+             hipMemcpyAsync(p->off, tables.data(), tables.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess;
+        p->item = reinterpret_cast<ColItem*>(p->off + at_item);
+        p->start = reinterpret_cast<ColStart*>(p->off + at_start);
+        p->ent = reinterpret_cast<uint2*>(p->off + at_ent);
+        p->seg = reinterpret_cast<ColSeg*>(p->off + at_seg);
+        if (ok) {
+            hipLaunchKernelGGL(k_col_trace, grid, block, 0, s, a, bins, p->tw, p->th, p->ntx, tiles, cnt, tile_cur,
+                               group_cnt, p->off, p->start, p->ent, p->off + at_toff, p->seg);
+            ok = hipGetLastError() == hipSuccess && hipStreamSynchronize(s) == hipSuccess;
+        }
     }
     if (!ok) (void)hipStreamSynchronize(s);      // copies from this function's tables
-    hipFree(cnt); hipFree(tile_cnt); hipFree(tile_off);
+    hipFree(cnt);
     if (!ok) {
         (void)hipGetLastError();
         col_free(p);

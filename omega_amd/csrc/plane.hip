@@ -18,8 +18,10 @@
 // image / without; the kernels before it in brackets): Siddon 55 / 52 us (141 / 92: slices and accumulators in
 // LDS), with 17 TOF bins 362 us (5968: one lane per LOR, every plane's bin weights evaluated twice), orthogonal
 // 73 / 71 us (964 / 655: tube lists of every plane), interpolation 89 / 72 us (589 / 384). Odd 109 x 97 image,
-// 8 planes of 142 x 91 bins, with prior: 50 us (478: global atomics). The lists take 50 MB (TOF: 340 MB) and are
-// built in 0.8 ms (TOF: 2.6 ms), less than the steps of one full iteration save.
+// 8 planes of 142 x 91 bins, with prior: 50 us (478: global atomics). The lists take 50 MB (TOF: 340 MB). A
+// handle's first call builds them, 0.9 ms with its allocations (orthogonal 1.7, TOF 3.2 ms): two iterations of 8 subsets
+// on a fresh handle take 1.8 ms against 2.05 ms tracing (orthogonal 2.9 against 25, interpolation 2.3 against 7.9, TOF 6.1
+// against 48 ms), one alone takes 0.2 ms more with Siddon.
 #include "plane.hpp"
 #include "geom.hpp"
 #include "siddon_device.hpp"
@@ -55,6 +57,7 @@ struct PlanePlan {
     float* share = nullptr;                  // TOF: [nent][pitch] bin shares
     uint32_t pitch = 0;
     int32_t* slice = nullptr;                // [n_proj]
+    uint32_t* tables = nullptr;              // the allocation of off, len, soff, slen, coff, clen and slice
     std::vector<int32_t> slice_host;
 };
 
@@ -93,21 +96,30 @@ __global__ __launch_bounds__(kPB) void k_plane_transpose(uint32_t bins, const ui
 }
 
 // Orders each pixel's list by key (rank sort, one wave per pixel): the lists do not depend on the order in
-// which k_plane_transpose's atomics retired.
+// which k_plane_transpose's atomics retired. A lane holds one key and counts the smaller ones, 64 others at a time from
+// the wave's registers (128 x 128 pixels, 128 x 160 LORs: 99 us; 328 us with every key read from memory).
 __global__ __launch_bounds__(kPB) void k_plane_sort(uint32_t npix, const uint32_t* __restrict__ coff,
                                                     const uint32_t* __restrict__ count,
                                                     const uint32_t* __restrict__ key, const uint2* __restrict__ val,
                                                     uint2* __restrict__ cent, uint32_t* __restrict__ cpos) {
-    const uint32_t pix = blockIdx.x * (kPB / 64) + (threadIdx.x >> 6);
+    const uint32_t pix = blockIdx.x * (kPB / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (pix >= npix) return;
+    const uint32_t lane = threadIdx.x & 63;
     const size_t o = (size_t)coff[pix / kLI] + pix % kLI;
     const uint32_t n = count[pix];
-    for (uint32_t i = threadIdx.x & 63; i < n; i += 64) {
-        const uint32_t ki = key[o + (size_t)i * kLI];
+    for (uint32_t i0 = 0; i0 < n; i0 += 64) {
+        const uint32_t i = i0 + lane, ki = i < n ? key[o + (size_t)i * kLI] : 0u;
         uint32_t r = 0;
-        for (uint32_t j = 0; j < n; j++) r += key[o + (size_t)j * kLI] < ki ? 1u : 0u;
-        cent[o + (size_t)r * kLI] = val[o + (size_t)i * kLI];
-        if (cpos) cpos[o + (size_t)r * kLI] = ki;
+        for (uint32_t j0 = 0; j0 < n; j0 += 64) {
+            // behind the list: larger than every key (a position below 2^32 - 16)
+            const uint32_t kj = j0 + lane < n ? key[o + (size_t)(j0 + lane) * kLI] : ~0u;
+#pragma unroll
+            for (int t = 0; t < 64; t++) r += (uint32_t)__builtin_amdgcn_readlane((int)kj, t) < ki ? 1u : 0u;
+        }
+        if (i < n) {
+            cent[o + (size_t)r * kLI] = val[o + (size_t)i * kLI];
+            if (cpos) cpos[o + (size_t)r * kLI] = ki;
+        }
     }
 }
 
@@ -436,9 +448,8 @@ __global__ __launch_bounds__(kPB) void k_plane_bp(PlaneRun a, uint32_t bpb, uint
 
 // ---- plan: host ----------------------------------------------------------------------------------------
 static void plan_free(PlanePlan* p) {
-    hipFree(p->ent); hipFree(p->off); hipFree(p->len); hipFree(p->samp); hipFree(p->soff); hipFree(p->slen);
-    hipFree(p->cent); hipFree(p->cpos); hipFree(p->coff); hipFree(p->clen); hipFree(p->w); hipFree(p->share);
-    hipFree(p->slice);
+    hipFree(p->ent); hipFree(p->samp); hipFree(p->cent); hipFree(p->cpos); hipFree(p->w); hipFree(p->share);
+    hipFree(p->tables);
     const std::vector<int32_t> keep = p->slice_host;
     *p = PlanePlan();
     p->slice_host = keep;
@@ -467,11 +478,6 @@ static bool list_layout(const std::vector<uint32_t>& cnt, std::vector<uint32_t>&
     }
     *total = t;
     return true;
-}
-
-static bool upload_u32(uint32_t** dst, const std::vector<uint32_t>& v, hipStream_t s) {
-    return dev_alloc(dst, v.size()) &&
-           hipMemcpyAsync(*dst, v.data(), v.size() * sizeof(uint32_t), hipMemcpyHostToDevice, s) == hipSuccess;
 }
 
 // Work memory of an iteration in floats: gathered slices; ratios (TOF: per entry, a chunk of planes at a time); weights.
@@ -525,11 +531,13 @@ static bool plan_build(const omg_geom* g, PlanePlan* p, hipStream_t s) {
     p->npix = p->nyx + (interp ? d.Nx + 1 : 0);
     // a row along x starts at its y times Ny (siddon_setup): with Ny > Nx it can end past the slice. The TOF kernels
     // hold one chunk of planes at a time and take no such rows, nor are lists many times the slice kept for them.
-    if (!interp && !orth && !tof && d.Ny > d.Nx && d.Ny <= 16 * d.Nx && d.Ny < 32768) p->npix = std::max(p->nyx, (d.Ny - 1) * d.Ny + d.Nx);
+    if (!interp && !orth && !tof && d.Ny > d.Nx && d.Ny <= 16 * d.Nx && d.Ny < 32768)
+        p->npix = std::max(p->nyx, (d.Ny - 1) * d.Ny + d.Nx);
     if (interp) interp_plane_slices(g, p->slice_host);
     else siddon_plane_slices(g, p->slice_host);
-    // The lowest slice (the orthogonal projector has its own choice, and square images only): voxels that a walk leaves out behind the image's end are out for every other plane too, so
-    // the lists hold (or refuse, plane_put) all that any plane visits.
+    // The lowest slice: voxels that a walk leaves out behind the image's end are out for every other plane too, so the
+    // lists hold (or refuse, plane_put) all that any plane visits. The orthogonal projector, whose images are square and
+    // whose tubes stay in their slice, has its own choice.
     uint32_t plane = d.n_proj;
     for (uint32_t q = 0; q < d.n_proj; q++)
         if (p->slice_host[q] >= 0 && (plane == d.n_proj || p->slice_host[q] < p->slice_host[plane])) plane = q;
@@ -540,11 +548,13 @@ static bool plan_build(const omg_geom* g, PlanePlan* p, hipStream_t s) {
     PlaneFill f = {};
     f.npix = p->npix;
     f.slice_base = (uint32_t)p->slice_host[plane] * p->nyx;
-    uint32_t *cnt = nullptr, *pixcnt = nullptr, *scnt = nullptr, *key = nullptr;
-    int32_t* bad = nullptr;
+    // counts, cleared and read back together: [pixels][bad][rows][samples of the rows]
+    const uint64_t npix0 = p->npix, ncount = npix0 + 1 + (interp ? 2 : 1) * (uint64_t)bins;
+    uint32_t *counts = nullptr, *key = nullptr;
     uint2* val = nullptr;
     float* lsum = nullptr;
-    bool ok = dev_alloc(&cnt, bins) && dev_alloc(&pixcnt, p->npix) && dev_alloc(&scnt, bins) && dev_alloc(&bad, 1);
+    bool ok = dev_alloc(&counts, ncount);
+    uint32_t *pixcnt = counts, *cnt = counts + npix0 + 1, *scnt = cnt + bins;
     auto trace = [&](const PlaneFill& q) {
         return (interp ? interp_plane_trace(g, plane, q, s) : orth ? orth_plane_trace(g, plane, q, s)
                 : tof ? tof_plane_trace(g, plane, q, s) : siddon_plane_trace(g, plane, q, s)) == OMG_OK;
@@ -552,20 +562,18 @@ static bool plan_build(const omg_geom* g, PlanePlan* p, hipStream_t s) {
     auto fill1 = [&](uint32_t* q, uint64_t n, uint32_t v) {
         hipLaunchKernelGGL(k_plane_set1, dim3(grid_for((int64_t)n, kPB)), dim3(kPB), 0, s, q, n, v);
     };
-    std::vector<uint32_t> hc(bins), hp(p->npix), hs(bins), off, len, soff, slen, coff, clen;
-    int32_t hbad = 0;
+    std::vector<uint32_t> host(ncount), hc, hp, hs, off, len, soff, slen, coff, clen, tables;
     uint64_t nc = 0, ns = 0;
     if (ok) {
-        fill1(pixcnt, p->npix, 0u);
-        fill1(reinterpret_cast<uint32_t*>(bad), 1, 0u);
-        f.cnt = cnt; f.pixcnt = pixcnt; f.scnt = scnt; f.bad = bad;
-        ok = trace(f) &&
-             hipMemcpyAsync(hc.data(), cnt, bins * 4ull, hipMemcpyDeviceToHost, s) == hipSuccess &&
-             hipMemcpyAsync(hp.data(), pixcnt, p->npix * 4ull, hipMemcpyDeviceToHost, s) == hipSuccess &&
-             (!interp || hipMemcpyAsync(hs.data(), scnt, bins * 4ull, hipMemcpyDeviceToHost, s) == hipSuccess) &&
-             hipMemcpyAsync(&hbad, bad, 4, hipMemcpyDeviceToHost, s) == hipSuccess &&
-             hipStreamSynchronize(s) == hipSuccess && !hbad;
+        fill1(pixcnt, npix0 + 1, 0u);
+        f.cnt = cnt; f.pixcnt = pixcnt; f.scnt = scnt; f.bad = reinterpret_cast<int32_t*>(pixcnt + npix0);
+        ok = trace(f) && hipMemcpyAsync(host.data(), counts, ncount * 4, hipMemcpyDeviceToHost, s) == hipSuccess &&
+             hipStreamSynchronize(s) == hipSuccess && !host[npix0];
     }
+    const auto rows = host.begin() + (ptrdiff_t)npix0 + 1;
+    hp.assign(host.begin(), host.begin() + (ptrdiff_t)npix0);
+    hc.assign(rows, rows + bins);
+    if (interp) hs.assign(rows + bins, host.end());
     if (!interp) {       // only as far as the lists go
         while (p->npix > p->nyx && hp[p->npix - 1] == 0) p->npix--;
         hp.resize(p->npix);
@@ -582,12 +590,19 @@ static bool plan_build(const omg_geom* g, PlanePlan* p, hipStream_t s) {
         ok = p->nent * (8 + 4 + 4ull * p->pitch) + nc * (8 + 12 + 4) + ns * 16 + 4ull * bins * d.n_proj +
                  4ull * (w.xt + w.r + w.w) <= budget;
     }
-    ok = ok && upload_u32(&p->off, off, s) && upload_u32(&p->len, len, s) && upload_u32(&p->coff, coff, s) &&
-         upload_u32(&p->clen, clen, s) && dev_alloc(&p->ent, p->nent) && dev_alloc(&p->cent, nc) && dev_alloc(&key, nc) &&
-         dev_alloc(&val, nc) && dev_alloc(&p->w, (uint64_t)bins * d.n_proj) && dev_alloc(&p->slice, d.n_proj) &&
-         hipMemcpyAsync(p->slice, p->slice_host.data(), d.n_proj * 4ull, hipMemcpyHostToDevice, s) == hipSuccess;
-    if (ok && interp) ok = upload_u32(&p->soff, soff, s) && upload_u32(&p->slen, slen, s) && dev_alloc(&p->samp, ns);
-    if (ok && tof) ok = dev_alloc(&p->share, p->nent * p->pitch) && dev_alloc(&p->cpos, nc) && dev_alloc(&lsum, p->nent);
+    ok = ok && dev_alloc(&p->ent, p->nent) && dev_alloc(&p->cent, nc) && dev_alloc(&key, nc) && dev_alloc(&val, nc) &&
+         dev_alloc(&p->w, (uint64_t)bins * d.n_proj) && (!interp || dev_alloc(&p->samp, ns)) &&
+         (!tof || (dev_alloc(&p->share, p->nent * p->pitch) && dev_alloc(&p->cpos, nc) && dev_alloc(&lsum, p->nent)));
+    if (ok) {                // the small tables in one copy
+        for (const auto* t : {&off, &len, &soff, &slen, &coff, &clen}) tables.insert(tables.end(), t->begin(), t->end());
+        tables.insert(tables.end(), p->slice_host.begin(), p->slice_host.end());
+        ok = dev_alloc(&p->tables, tables.size()) &&
+             hipMemcpyAsync(p->tables, tables.data(), tables.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess;
+        uint32_t* t = p->tables;
+        p->off = t; p->len = t += off.size(); p->soff = t += len.size(); p->slen = t += soff.size();
+        p->coff = t += slen.size(); p->clen = t += coff.size();
+        p->slice = reinterpret_cast<int32_t*>(t += clen.size());
+    }
     if (ok) {
         hipLaunchKernelGGL(k_plane_set2, dim3(grid_for((int64_t)p->nent, kPB)), dim3(kPB), 0, s, p->ent, p->nent, p->xrows);
         hipLaunchKernelGGL(k_plane_set2, dim3(grid_for((int64_t)nc, kPB)), dim3(kPB), 0, s, p->cent, nc, bins);
@@ -603,16 +618,18 @@ static bool plan_build(const omg_geom* g, PlanePlan* p, hipStream_t s) {
         }
         ok = ok && (interp ? interp_plane_weights(g, p->w, s) : orth ? orth_plane_weights(g, p->w, s)
                            : siddon_plane_weights(g, p->w, s)) == OMG_OK;
+    }
+    if (ok) {
         // the second pass over the row counts (the same walk) left cnt as it was
         fill1(pixcnt, p->npix, 0u);
         hipLaunchKernelGGL(k_plane_transpose, dim3((bins + kPB / 64 - 1) / (kPB / 64)), dim3(kPB), 0, s, bins, p->ent,
                            lsum, p->off, cnt, p->coff, pixcnt, key, val);
         hipLaunchKernelGGL(k_plane_sort, dim3((p->npix + kPB / 64 - 1) / (kPB / 64)), dim3(kPB), 0, s, p->npix, p->coff,
                            pixcnt, key, val, p->cent, p->cpos);
-        ok = ok && hipGetLastError() == hipSuccess && hipStreamSynchronize(s) == hipSuccess;
+        ok = hipGetLastError() == hipSuccess && hipStreamSynchronize(s) == hipSuccess;
     }
     if (!ok) (void)hipStreamSynchronize(s);      // copies from this function's tables
-    hipFree(cnt); hipFree(pixcnt); hipFree(scnt); hipFree(bad); hipFree(key); hipFree(val); hipFree(lsum);
+    hipFree(counts); hipFree(key); hipFree(val); hipFree(lsum);
     if (interp && ok) {      // the row lists served the transposition only
         hipFree(p->ent);
         p->ent = nullptr;

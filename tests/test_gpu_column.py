@@ -73,6 +73,24 @@ def test_column(cuda, nx, ny, nz, n_radial, n_angles, planes, first, dz):
     assert max(e[1:]) < BAR
 
 
+def test_many_tiles(cuda):
+    """More tiles than a workgroup counts in LDS."""
+    import torch
+    grid, x, z = _scanner(530, 530, 63, 24, 20, 33)
+    n = 33 * 480
+    img, y = torch.rand(grid.N, device="cuda"), torch.rand(n, device="cuda")
+    out = []
+    for gen in (False, True):
+        geom = make_geom(grid, x, z, 24, 20, generic=gen)
+        p, back = torch.empty(n, device="cuda"), torch.zeros(grid.N, device="cuda")
+        _lib.call("omg_forward_project", geom.handle, 0, n, ptr(img), ptr(p), None)
+        _lib.call("omg_backward_project", geom.handle, 0, n, ptr(y), ptr(back), None, None)
+        out.append((p.cpu().numpy(), back.cpu().numpy()))
+        assert list_calls(geom) == (0, 0 if gen else 2)
+    assert np.array_equal(out[0][0], out[1][0])
+    assert rel_l2(out[0][1], out[1][1]) < BAR
+
+
 def test_several_passes(cuda):
     """140 planes of 224 x 224 bins: their records take two passes of plane groups, each with LORs off the lists. About
     1e5 terms per voxel, so the float atomics of the other kernels carry 2^-24 sqrt(1e5) = 2e-5; bar: four times that."""
