@@ -44,7 +44,7 @@ def parse():
     ap.add_argument("--traffic", default=os.path.join(ROOT, "profiles", "plane_lists_pet2d_traffic.txt"),
                     help="summary of the rocprofv3 --pmc HBM traffic of the dominant kernel, if present")
     ap.add_argument("--issue", default=os.path.join(ROOT, "profiles", "plane_lists_pet2d_issue.txt"),
-                    help="summary of the rocprofv3 --pmc VALU issue counters of the dominant kernel, if present")
+                    help="summary of the rocprofv3 --pmc issue counters of the dominant kernels, if present")
     ap.add_argument("--workload", default="pet2d_osem",
                     choices=["pet2d_osem", "pet3d_frames", "ct_cgls_bdd", "pet2d_orth", "pet2d_volume", "pet3d_autograd",
                              "pet2d_tof", "pet2d_volume_tof", "pet2d_interp", "pet2d_interp_tof", "unet"],
@@ -148,7 +148,11 @@ def main():
     kernel_name = "k_planar_fpq<640,false> + k_planar_vbp<false,false>" if args.voxel_bp else \
         "k_plane_gather + k_plane_fp + k_plane_bp (with the update)"
     avg_s = tot.value * 1e-3 / max(cnt.value, 1)
-    bytes_per_launch = float(np.mean([4.0 * np_sum[k] + 8.0 * np_nz[k] + 8.0 * M[k] for k in range(p.subsets)]))
+    per = p.nRowsD * p.nColsD
+    if args.voxel_bp:
+        bytes_per_launch = float(np.mean([4.0 * np_sum[k] + 8.0 * np_nz[k] + 8.0 * M[k] for k in range(p.subsets)]))
+    else:
+        bytes_per_launch = float(np.mean([_list_bytes(np_sum[k], M[k], per, p.grid.N, 8.0, 8.0) for k in range(p.subsets)]))
     achieved = bytes_per_launch / avg_s / 1e9
     traffic = None if args.voxel_bp else read_traffic(args.traffic)   # the summary covers the list kernels
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
@@ -157,8 +161,8 @@ def main():
                 "avg_launch_us": round(avg_s * 1e6, 2), "algorithmic_bytes_per_launch": int(bytes_per_launch)}
     issue = None if args.voxel_bp else read_issue(args.issue)
     if issue:
-        # the kernel's real limiter: its VALU issue rate, from the committed counter summary
-        roofline["issue_bound"] = issue
+        # what the kernels wait for, from the committed counter summary
+        roofline["issue"] = issue
 
     cpu = None
     if not args.no_cpu:
@@ -485,7 +489,9 @@ def bench_orth(args, volume=False, tof=False):
     b.record()
     b.synchronize()
     s_s = a.elapsed_time(b) * 1e-3
-    byt = 12.0 * ntube + 8.0 * M0 * nb
+    per = p.nRowsD * p.nColsD
+    # the volume projector streams tube lists of every plane; the orthogonal one those of one plane, as the headline does
+    byt = 12.0 * ntube + 8.0 * M0 * nb if volume else _list_bytes(ntube, M0, per, p.grid.N, 8.0, 8.0)
     cpu = None
     if not args.no_cpu:
         from oracle import oracle as O
@@ -529,8 +535,9 @@ def bench_interp(args, tof=False):
     """2-D plane PET OSEM with the interpolation projector (projector type 4, the operator API's default
     interpolation length dL = dx / 2) on the pet2d_osem geometry. value = subset-iterations/s (8 subsets x 1
     iteration per step). tof: with time of flight, 17 bins of 140 ps at 400 ps FWHM. Algorithmic bytes per
-    subset step: 12 per sample (the forward projection's interpolated read, the backprojection's atomic
-    read-modify-write) plus 8 per measurement and bin; the samples are counted from the LORs' chords through
+    subset step: the lists of one plane (16 bytes per forward sample, 8 per backprojected one); with time of flight 12
+    per sample (the forward projection's interpolated read, the backprojection's atomic read-modify-write) plus 8 per
+    measurement and bin; the samples are counted from the LORs' chords through
     the image (chord / dL + 1 per LOR and plane)."""
     import numpy as np
     import torch
@@ -586,7 +593,8 @@ def bench_interp(args, tof=False):
     chord = np.clip(tmax - tmin, 0, None) * np.linalg.norm(v, axis=1)
     per_plane = float(np.sum(np.where(chord > 0, np.floor(chord / dl) + 1, 0)))
     samples = per_plane * (M0 // (sc.n_radial * sc.n_angles))
-    byt = 12.0 * samples + 8.0 * M0 * nb
+    byt = 12.0 * samples + 8.0 * M0 * nb if tof else \
+        _list_bytes(samples, M0, p.nRowsD * p.nColsD, p.grid.N, 16.0, 8.0)
     cpu = None
     if not args.no_cpu:
         from oracle import oracle as O
@@ -656,8 +664,8 @@ def bench_tof(args):
             runner.subset_step(x, k)
     torch.cuda.synchronize()
     dt = time.perf_counter() - t0
-    # one subset step timed alone; its visits give the exponential count (FP and BP each: 3 per bin and
-    # visit, the first point shared with the previous voxel; the BP's weights reused from its sum)
+    # one subset step timed alone; its bytes: the lists of one plane, an entry's shares read for the sums and again for
+    # the ratios
     ntr = _trace_counts(p, 0, dev)
     M0 = int(p.nMeasSubset[0, 0])
     a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
@@ -666,7 +674,7 @@ def bench_tof(args):
     b.record()
     b.synchronize()
     s_s = a.elapsed_time(b) * 1e-3
-    byt = 12.0 * ntr + 8.0 * M0 * p.nBins
+    byt = _list_bytes(ntr, M0, p.nRowsD * p.nColsD, p.grid.N, 8.0 + 8.0 * p.nBins, 4.0, p.nBins)
     cpu = None
     if not args.no_cpu:
         _progress("pet2d_tof: CPU baseline")
@@ -680,9 +688,6 @@ def bench_tof(args):
         "config": {"workload": "pet2d_osem_tof", "image": [128, 128, 63], "sinogram": [128, 160, 63],
                    "tof_bins": p.nBins, "tof_fwhm_ps": 400, "tof_bin_ps": 140, "attenuation": "water cylinder",
                    "subsets": 8, "voxel_visits_subset0": ntr, "geometry_setup_ms": round(setup_ms, 1)},
-        # bound: the double-precision exponentials. exp(double) compiles for gfx950 to 19 FP64 VALU
-        # instructions (13 FMA, mul, rndne, ldexp, cvt, 2 compares); at the FP64 vector rate of 78.6 TFLOP/s
-        # (39.3 T lane-instructions/s) that is 2.07e12 exp/s with no other work
         "roofline": {"bound": "hbm", "achieved": round(byt / s_s / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(byt / s_s / 1e9 / HBM_PEAK_GBS, 4), "traffic": None,
                      "kernel": "k_plane_tof + k_plane_bp + update", "avg_launch_us": round(s_s * 1e6, 1),
@@ -871,21 +876,29 @@ def read_traffic(path):
 
 
 def read_issue(path):
-    """VALU issue figures of the dominant kernel from a committed rocprofv3 --pmc summary, if present:
-    lines 'valu_busy: f' (rocprof's VALUBusy), 'valu_busy_vs_sq_busy: f', 'valu_insts_per_launch: n',
-    'waves_per_simd: w'."""
+    """Issue figures of the dominant kernels from a committed rocprofv3 --pmc summary, if present: lines
+    'valu_busy: f' (VALU issue slots used), 'waves_per_simd: w' (in flight), 'valu_insts_per_launch: n', 'bound: text'."""
     if not os.path.exists(path):
         return None
     out = {}
     for line in open(path):
-        for key in ("valu_busy", "valu_busy_vs_sq_busy", "valu_insts_per_launch", "waves_per_simd"):
-            if line.startswith(key + ":"):
-                out[key] = float(line.split(":", 1)[1])
+        key, _, value = line.partition(":")
+        if key in ("valu_busy", "valu_insts_per_launch", "waves_per_simd"):
+            out[key] = float(value)
+        elif key == "bound":
+            out[key] = value.strip()
     if "valu_busy" not in out:
         return None
-    out["bound"] = "valu_issue"
     out["source"] = os.path.relpath(path, ROOT)
     return out
+
+
+def _list_bytes(visits, M, per, N, forward, backward, bins=1):
+    """Bytes of a subset step from the direct-plane lists: ``forward`` and ``backward`` bytes per entry of one plane's
+    lists (``visits``: LOR x voxel visits of all the step's planes), streamed once for every eight planes, the
+    measurements, the LORs' weights, and the image read and written with its sensitivity."""
+    planes = M // per
+    return visits / planes * -(-planes // 8) * (forward + backward) + 4.0 * M * (bins + 1) + 12.0 * N
 
 
 def cpu_baseline(p, y, x0, budget_s, runner, n_iter, osem_kw=None):
