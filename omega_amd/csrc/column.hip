@@ -575,6 +575,10 @@ __global__ __launch_bounds__(1024, 8) void k_col_bp(ColView c, SidArgs a, uint32
     const ColItem it = c.item[blockIdx.x - rest_blocks];
     const uint32_t x0 = it.tile % c.ntx * c.tw, y0 = it.tile / c.ntx * c.th;
     const uint32_t zp = a.Nz + 2, cells = c.tw * c.th * zp;
+    auto bin_peak = [&](uint32_t q) {
+        return q < it.s1 ? (sens ? wpeak : peak)[(size_t)blockIdx.y * c.bins + c.seg[q].bin] : ColPeak{0u, 0.f};
+    };
+    ColPeak pk = bin_peak(it.s0 + threadIdx.x);        // in flight while the cells are cleared
     for (uint32_t i = threadIdx.x; i < cells; i += blockDim.x) acc64[i] = 0ull;
     // The item's own scale: |term| <= peak * voxel diagonal, and a segment adds at most two terms to a voxel per lane.
     // One outlying LOR so costs bits where it passes only, and of its own size (the sum of the records bounds a voxel's,
@@ -582,10 +586,10 @@ __global__ __launch_bounds__(1024, 8) void k_col_bp(ColView c, SidArgs a, uint32
     uint32_t top = 0, low = ~0u;
     float sum = 0.f;
     for (uint32_t q = it.s0 + threadIdx.x; q < it.s1; q += blockDim.x) {
-        const ColPeak pk = (sens ? wpeak : peak)[(size_t)blockIdx.y * c.bins + c.seg[q].bin];
         top = max(top, pk.top);
         low = min(low, pk.top ? pk.top : ~0u);
         sum += pk.sum;
+        pk = bin_peak(q + blockDim.x);
     }
     top = wave_fold(top, [](uint32_t a, uint32_t b) { return max(a, b); });
     low = ~wave_fold(~low, [](uint32_t a, uint32_t b) { return max(a, b); });

@@ -10,9 +10,15 @@ struct ColPlan;
 
 // The transaxial lists that serve measurements [first, first + n) of g, built on the first call that may allocate
 // and wait; null when they do not apply or do not fit, or with fewer than min_planes planes. A wave's 64 lanes are
-// planes, so its time hardly falls with their number: with 64 the forward projection gains 2.3 times (half of that
-// with kColPlanes), the backprojection 16 times (kColPlanesBack; 1380 -> 209 us
-// with 30 planes of 208 x 128 bins, 123 x 123 x 27 voxels).
+// planes, so its time hardly falls with their number. One lane per LOR / by columns, us, 208 x 128 bins on 123 x 123 x 27
+// voxels and 224 x 224 bins on 128 x 128 x 63:
+//   planes   forward            backward            fused step
+//   8        70/174   102/318   590/263  1174/493   615/392  1157/751
+//   16       105/177  183/322   1132/268 2109/499   1104/397 2117/757
+//   31       170/179  317/322   2050/274 4022/506   2000/404 3934/766
+//   64       310/184  607/331   3962/287 7977/520   3962/414 7864/779
+// So forward projections go by columns from kColPlanes on, backprojections from kColPlanesBack. The fused and frames steps
+// keep the forward projection's line, by these figures a late one (theirs lies at 8).
 constexpr uint32_t kColPlanes = 32, kColPlanesBack = 12;
 const ColPlan* col_plan(const omg_geom* g, int64_t first, int64_t n, hipStream_t s, uint32_t min_planes = kColPlanes);
 void col_release(omg_geom* g);
