@@ -556,7 +556,7 @@ __global__ __launch_bounds__(64) void k_col_rest(SidArgs a, const uint32_t* __re
 // every other block one item: LDS accumulators [tile pixel][Nz + 2], int64 fixed point; the end cells are dropped.
 // blockIdx.z 1: the weights into sens instead of the records' values into rhs. What bounds it: the LDS atomics (64
 // lanes over one column's cells) and about 35 VALU operations per column and 64 LORs. 64 planes of 224 x 224 bins,
-// 128 x 128 x 63: 281 us, with the records' launch 355 us; 5690 us by one lane per LOR (global float atomics).
+// 128 x 128 x 63: 285 us, with the records' launch 355 us; 5690 us by one lane per LOR (global float atomics).
 __global__ __launch_bounds__(1024, 8) void k_col_bp(ColView c, SidArgs a, uint32_t plane0, uint32_t rest_blocks,
                                                     ColRest rest, const float4* __restrict__ rec,
                                                     const float* __restrict__ wrec, const ColPeak* __restrict__ peak,

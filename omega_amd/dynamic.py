@@ -159,7 +159,8 @@ class FramesTuner:
     Every candidate runs ``reps`` eager subset steps (subset ``k``) on a scratch copy of the image
     stack after one warm-up step; the median event-timed step wins. Results are cached per key
     (image size, measurements of the subset, frame count) in memory and, when ``path`` is given, in a
-    JSON file.
+    JSON file. Where the steps go by image columns (3-D ring sinograms of 32 or more planes per subset) the launch
+    shape does not enter them, and the candidates differ by noise only.
     """
 
     def __init__(self, path: str | None = None):
