@@ -894,16 +894,18 @@ const ColPlan* col_plan(const omg_geom* gc, int64_t first, int64_t n, hipStream_
         for (ColPlan* p : g->columns->e)
             if (!g->index_dev || (p->first == first && p->n == n)) return p->ok ? p : nullptr;
     if (fixed_region_active() || (g->columns && g->columns->e.size() >= kColPlans) || is_capturing(s)) return nullptr;
+    std::unique_ptr<ColPlan> built;
     try {
         const RelaxedCapture relaxed;
         if (!g->columns) g->columns = new ColCache();
         g->columns->e.reserve(kColPlans);
-        std::unique_ptr<ColPlan> p(new ColPlan());
-        p->first = first;
-        p->n = n;
-        p->ok = col_build(g, p.get(), s);
-        g->columns->e.push_back(p.release());
+        built.reset(new ColPlan());
+        built->first = first;
+        built->n = n;
+        built->ok = col_build(g, built.get(), s);
+        g->columns->e.push_back(built.release());
     } catch (const std::bad_alloc&) {       // no host memory for the tables: trace
+        if (built) col_free(built.get());
         return nullptr;
     }
     const ColPlan* p = g->columns->e.back();

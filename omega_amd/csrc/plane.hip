@@ -645,13 +645,15 @@ const PlanePlan* plane_plan(const omg_geom* gc, hipStream_t s) {
     omg_geom* g = const_cast<omg_geom*>(gc);
     const std::lock_guard<std::mutex> lock(g->lists_mu);
     if (g->plane) return g->plane->ok ? g->plane : nullptr;
-    if (!plan_applies(g) || fixed_region_active() || is_capturing(s)) return nullptr;
+    std::unique_ptr<PlanePlan> p;
     try {
+        if (!plan_applies(g) || fixed_region_active() || is_capturing(s)) return nullptr;
         const RelaxedCapture relaxed;
-        std::unique_ptr<PlanePlan> p(new PlanePlan());
+        p.reset(new PlanePlan());
         p->ok = plan_build(g, p.get(), s);
         g->plane = p.release();
     } catch (const std::bad_alloc&) {       // no host memory for the tables: trace
+        if (p) plan_free(p.get());
         return nullptr;
     }
     return g->plane->ok ? g->plane : nullptr;
