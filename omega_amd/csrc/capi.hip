@@ -331,7 +331,7 @@ extern "C" int omg_geom_create(const omg_geom_desc* d, omg_geom** out) {
         g->planar = d->meas_index == nullptr && d->tof_bins <= 1 && rays <= 1;
         for (uint32_t p = 0; p < d->n_proj && g->planar; p++) g->planar = d->z[2 * p] == d->z[2 * p + 1];
     }
-    if (!rc && d->mode == OMG_MODE_PET_SINO) g->ring = ring_table(*d, d->x, g->bmaxx, g->bmaxy);
+    if (!rc && g->planar) g->ring = ring_table(*d, d->x, g->bmaxx, g->bmaxy);
     if (!rc && d->mode == OMG_MODE_PET_SINO) rc = vbp_prepare(g, d->x);
     if (!rc && d->projector_type == OMG_PROJ_BDD) rc = bdd_prepare(g);
     if (!rc && d->projector_type == OMG_PROJ_VOLUME) rc = upload(d->vol_V, d->vol_len, &g->vol_dev);

@@ -120,12 +120,35 @@ __device__ __forceinline__ bool col_walk(const SidArgs& a, uint32_t j, ColStart&
     return true;
 }
 
+// Bin j's LOR misses the image, or enters it after 1e-3 of its way and leaves it before 1 - 1e-3: every crossing parameter
+// of its walk then lies in [0, 1], and a length is a parameter step times the LOR's (as ring_table asks of all LORs of
+// a direct-plane sinogram).
+__device__ __forceinline__ bool col_ring(const SidArgs& a, uint32_t j) {
+    Ray r;
+    fetch_ray_base(a, j, r);
+    double t0 = 0.0, t1 = 1.0;
+    bool miss = false;
+    auto clip = [&](double s, double e, double lo, double hi) {
+        const double dd = e - s;
+        if (dd == 0.0) {
+            miss = miss || s < lo || s > hi;
+            return;
+        }
+        const double ta = (lo - s) / dd, tb = (hi - s) / dd;
+        t0 = fmax(t0, fmin(ta, tb));
+        t1 = fmin(t1, fmax(ta, tb));
+    };
+    clip(r.xs, r.xd, a.bx, a.bmaxx);
+    clip(r.ys, r.yd, a.by, a.bmaxy);
+    return miss || t0 >= t1 || !(t0 < 1e-3 || t1 > 1.0 - 1e-3);
+}
+
 // One plan's arrays while it is built (blockIdx.y of the launches below).
 struct ColTrace {
     int64_t first;               // index table: the range's first measurement
     uint32_t* cnt;               // [bins] entries
     uint32_t* tile_cnt;          // [tiles] segments
-    int32_t* bad;                // the range is not the same bins of every plane
+    int32_t* bad;                // not the same bins in every plane, or a LOR that starts or ends in the image
     uint32_t* group_cnt;         // [workgroups][tiles]
     uint32_t* tile_cur;          // [tiles] segments placed so far
     // filling pass; null: no plan
@@ -165,6 +188,7 @@ __global__ __launch_bounds__(256) void k_col_trace(SidArgs a, uint32_t bins, uin
             n++;
         });
         q.cnt[j] = n;
+        if (!col_ring(a, j)) *q.bad = 1;
     }
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < (shared ? tiles : 0u); i += 256) {
@@ -944,10 +968,9 @@ static void col_build(const omg_geom* g, const std::vector<ColPlan*>& ps, hipStr
 const ColPlan* col_plan(const omg_geom* gc, int64_t first, int64_t n, hipStream_t s, uint32_t min_planes) {
     omg_geom* g = const_cast<omg_geom*>(gc);
     const omg_geom_desc& d = g->d;
-    // few planes leave lanes idle (min_planes); without the ring property a walk's lengths need the general expression;
-    // the records hold z in 15 bits and the steps left in 16
+    // few planes leave lanes idle (min_planes); the records hold z in 15 bits and the steps left in 16
     if (d.mode != OMG_MODE_PET_SINO || d.projector_type != OMG_PROJ_SIDDON || d.tof_bins > 1 || g->force_generic ||
-        d.reserved[3] != 0 || d.reserved[4] < 0 || !g->ring || d.n_proj < min_planes ||
+        d.reserved[3] != 0 || d.reserved[4] < 0 || d.n_proj < min_planes ||
         (uint64_t)d.Nx + d.Ny + d.Nz + 3 > 65535 || d.Nz > 32000 || n > 0xffffffffll ||
         (uint64_t)std::max(d.rays_xy, 1u) * std::max(d.rays_z, 1u) != 1)
         return nullptr;

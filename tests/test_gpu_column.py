@@ -73,6 +73,20 @@ def test_column(cuda, nx, ny, nz, n_radial, n_angles, planes, first, dz):
     assert max(e[1:]) < BAR
 
 
+def test_detectors_within_the_image(cuda):
+    """LORs that start in the image are traced: their lengths are not the crossings' steps."""
+    import torch
+    fov = 50.0
+    grid = G.Grid.from_fov(20, 20, 9, fov, fov, 22.5)
+    x = G.ring_sinogram_xy(24, 20, 1.5, 20.0)
+    z = np.random.default_rng(1).uniform(-10.0, 10.0, (40, 2)).astype(np.float32)
+    n = 40 * 480
+    img, y, meas = torch.rand(grid.N, device="cuda"), torch.rand(n, device="cuda"), torch.rand(n, device="cuda")
+    geoms = [make_geom(grid, x, z, 24, 20, generic=gen) for gen in (False, True)]
+    a, b = (_run(g, grid, 0, n, img, y, meas) for g in geoms)
+    assert list_calls(geoms[0]) == (0, 0) and np.array_equal(a[0], b[0]) and rel_l2(a[1], b[1]) < BAR
+
+
 def test_many_tiles(cuda):
     """More tiles than a workgroup counts in LDS."""
     import torch
