@@ -57,7 +57,7 @@ struct PlanePlan {
     float* share = nullptr;                  // TOF: [nent][pitch] bin shares
     uint32_t pitch = 0;
     int32_t* slice = nullptr;                // [n_proj]
-    uint32_t* tables = nullptr;              // the allocation of off, len, soff, slen, coff, clen and slice
+    char* block = nullptr;                   // the allocation that holds all of these
     std::vector<int32_t> slice_host;
 };
 
@@ -448,8 +448,7 @@ __global__ __launch_bounds__(kPB) void k_plane_bp(PlaneRun a, uint32_t bpb, uint
 
 // ---- plan: host ----------------------------------------------------------------------------------------
 static void plan_free(PlanePlan* p) {
-    hipFree(p->ent); hipFree(p->samp); hipFree(p->cent); hipFree(p->cpos); hipFree(p->w); hipFree(p->share);
-    hipFree(p->tables);
+    hipFree(p->block);
     const std::vector<int32_t> keep = p->slice_host;
     *p = PlanePlan();
     p->slice_host = keep;
@@ -590,18 +589,37 @@ static bool plan_build(const omg_geom* g, PlanePlan* p, hipStream_t s) {
         ok = p->nent * (8 + 4 + 4ull * p->pitch) + nc * (8 + 12 + 4) + ns * 16 + 4ull * bins * d.n_proj +
                  4ull * (w.xt + w.r + w.w) <= budget;
     }
-    ok = ok && dev_alloc(&p->ent, p->nent) && dev_alloc(&p->cent, nc) && dev_alloc(&key, nc) && dev_alloc(&val, nc) &&
-         dev_alloc(&p->w, (uint64_t)bins * d.n_proj) && (!interp || dev_alloc(&p->samp, ns)) &&
-         (!tof || (dev_alloc(&p->share, p->nent * p->pitch) && dev_alloc(&p->cpos, nc) && dev_alloc(&lsum, p->nent)));
-    if (ok) {                // the small tables in one copy
+    char* temp = nullptr;
+    if (ok) {                // one allocation for the lists, one for what only their building needs
         for (const auto* t : {&off, &len, &soff, &slen, &coff, &clen}) tables.insert(tables.end(), t->begin(), t->end());
         tables.insert(tables.end(), p->slice_host.begin(), p->slice_host.end());
-        ok = dev_alloc(&p->tables, tables.size()) &&
-             hipMemcpyAsync(p->tables, tables.data(), tables.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess;
-        uint32_t* t = p->tables;
+        size_t keep = 0, work = 0;
+        auto take = [](size_t& at, uint64_t bytes) {
+            const size_t o = at;
+            at += ((size_t)bytes + 255) & ~(size_t)255;
+            return o;
+        };
+        const size_t at_tables = take(keep, tables.size() * 4), at_cent = take(keep, nc * 8);
+        const size_t at_w = take(keep, 4ull * bins * d.n_proj), at_samp = take(keep, ns * 16);
+        const size_t at_share = take(keep, tof ? 4 * p->nent * p->pitch : 0), at_cpos = take(keep, tof ? 4 * nc : 0);
+        // the interpolation projector's row lists serve the transposition only
+        const size_t at_ent = take(interp ? work : keep, p->nent * 8);
+        const size_t at_key = take(work, nc * 4), at_val = take(work, nc * 8), at_lsum = take(work, tof ? 4 * p->nent : 0);
+        ok = dev_alloc(&p->block, keep) && dev_alloc(&temp, work) &&
+             hipMemcpyAsync(p->block + at_tables, tables.data(), tables.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess;
+        uint32_t* t = reinterpret_cast<uint32_t*>(p->block + at_tables);
         p->off = t; p->len = t += off.size(); p->soff = t += len.size(); p->slen = t += soff.size();
         p->coff = t += slen.size(); p->clen = t += coff.size();
         p->slice = reinterpret_cast<int32_t*>(t += clen.size());
+        p->cent = reinterpret_cast<uint2*>(p->block + at_cent);
+        p->w = reinterpret_cast<float*>(p->block + at_w);
+        if (interp) p->samp = reinterpret_cast<uint4*>(p->block + at_samp);
+        if (tof) p->share = reinterpret_cast<float*>(p->block + at_share);
+        if (tof) p->cpos = reinterpret_cast<uint32_t*>(p->block + at_cpos);
+        if (tof) lsum = reinterpret_cast<float*>(temp + at_lsum);
+        p->ent = reinterpret_cast<uint2*>((interp ? temp : p->block) + at_ent);
+        key = reinterpret_cast<uint32_t*>(temp + at_key);
+        val = reinterpret_cast<uint2*>(temp + at_val);
     }
     if (ok) {
         hipLaunchKernelGGL(k_plane_set2, dim3(grid_for((int64_t)p->nent, kPB)), dim3(kPB), 0, s, p->ent, p->nent, p->xrows);
@@ -629,11 +647,8 @@ static bool plan_build(const omg_geom* g, PlanePlan* p, hipStream_t s) {
         ok = hipGetLastError() == hipSuccess && hipStreamSynchronize(s) == hipSuccess;
     }
     if (!ok) (void)hipStreamSynchronize(s);      // copies from this function's tables
-    hipFree(counts); hipFree(key); hipFree(val); hipFree(lsum);
-    if (interp && ok) {      // the row lists served the transposition only
-        hipFree(p->ent);
-        p->ent = nullptr;
-    }
+    hipFree(counts); hipFree(temp);
+    if (interp) p->ent = nullptr;
     if (!ok) {
         (void)hipGetLastError();
         plan_free(p);
