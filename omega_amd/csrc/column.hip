@@ -982,8 +982,8 @@ const ColPlan* col_plan(const omg_geom* gc, int64_t first, int64_t n, hipStream_
             if (!g->index_dev || (p->first == first && p->n == n)) return p->ok ? p : nullptr;
     if (fixed_region_active() || (g->columns && g->columns->e.size() >= kColPlans) || is_capturing(s)) return nullptr;
     // Where an index table divides into ranges of this size, the caller goes through all of them: they are built together
-    // (a plan of 576 bins takes 130 us, three more beside it 30 us each), with up to 8 at the first range, which a caller of
-    // a single range pays for, with more at the second.
+    // (four plans of 576 bins take 220 us, one after the other 520 us), up to 8 at the first range, for which a caller of a
+    // single range pays little, more at the second.
     std::vector<int64_t> firsts{first};
     const int64_t ranges = g->index_dev && n > 0 && first % n == 0 && d.meas_index_len % n == 0 ? d.meas_index_len / n : 0;
     const ColPlan* one = g->columns && g->columns->e.size() == 1 ? g->columns->e[0] : nullptr;

@@ -19,9 +19,9 @@
 // LDS), with 17 TOF bins 362 us (5968: one lane per LOR, every plane's bin weights evaluated twice), orthogonal
 // 73 / 71 us (964 / 655: tube lists of every plane), interpolation 89 / 72 us (589 / 384). Odd 109 x 97 image,
 // 8 planes of 142 x 91 bins, with prior: 50 us (478: global atomics). The lists take 50 MB (TOF: 340 MB). A
-// handle's first call builds them, 0.9 ms with its allocations (orthogonal 1.7, TOF 3.2 ms): two iterations of 8 subsets
-// on a fresh handle take 1.8 ms against 2.05 ms tracing (orthogonal 2.9 against 25, interpolation 2.3 against 7.9, TOF 6.1
-// against 48 ms), one alone takes 0.2 ms more with Siddon.
+// handle's first call builds them, 0.8 ms with its allocations (interpolation 0.7, orthogonal 1.6, TOF 2.9 ms): two
+// iterations of 8 subsets on a fresh handle take 1.7 ms against 2.0 ms tracing (orthogonal 2.8 against 25, interpolation
+// 2.1 against 7.9, TOF 5.9 against 48 ms); one alone takes 0.1 ms more with Siddon.
 #include "plane.hpp"
 #include "geom.hpp"
 #include "siddon_device.hpp"
@@ -124,27 +124,30 @@ __global__ __launch_bounds__(kPB) void k_plane_sort(uint32_t npix, const uint32_
 }
 
 // ---- running -----------------------------------------------------------------------------------------
+// (Every argument of k_plane_bp within 256 bytes, and what k_plane_fp waits for first together: a further line of them
+// costs 0.1 us.)
 struct PlaneRun {
-    uint32_t bins, nyx, npix, xrows, planes; // planes: of this call
+    uint32_t bins, xrows, nyx, npix;
+    uint32_t planes;                         // of this call
     uint32_t nx, nz;                         // image row length, slices
-    bool skip0;                              // interpolation projector: nothing is added to voxel 0
+    uint32_t nent;
     const uint32_t *off, *len, *soff, *slen, *coff, *clen;
     const uint2 *ent, *cent;
     const uint4* samp;
     const uint32_t* cpos;
     const float* w;                          // of the call's first plane
     const int32_t* slice;                    // of the call's first plane
-    uint64_t nent;
     const float* share;
-    // interpolation projector: the planes' z table and the grid's z axis
+    // interpolation projector: the planes' z table and the grid's z axis (others: null)
     const float* z;
     float bz, sz;
 };
 
 // Xt[chunk][pixel][PL]: the planes' slices side by side (and what follows them, up to xrows), and a zero row behind
-// them for the padding entries.
-// INTERP: the blend of the two slices that the plane's samples lie between.
-template <int PL, bool INTERP>
+// them for the padding entries. GATHER_BEHIND: xrows reach past the slice, to the image's end at most.
+// GATHER_INTERP: the blend of the two slices that the plane's samples lie between.
+enum { GATHER_SLICE = 0, GATHER_INTERP = 1, GATHER_BEHIND = 2 };
+template <int PL, int MODE>
 __global__ __launch_bounds__(kPB) void k_plane_gather(PlaneRun a, const float* __restrict__ x, float* __restrict__ Xt) {
     const uint32_t pix = blockIdx.x * kPB + threadIdx.x;
     if (pix > a.xrows) return;
@@ -155,7 +158,7 @@ __global__ __launch_bounds__(kPB) void k_plane_gather(PlaneRun a, const float* _
         v[p] = 0.f;
         if (plane < a.planes && pix < a.xrows) {
             const int32_t tk = a.slice[plane];
-            if (INTERP) {
+            if (MODE == GATHER_INTERP) {
                 if (tk >= 0) {
                     const float u = ((0.f + a.z[2 * plane]) - a.bz) * a.sz * (float)a.nz - 0.5f;
                     const float f = floorf(u), c = u - f;
@@ -165,7 +168,7 @@ __global__ __launch_bounds__(kPB) void k_plane_gather(PlaneRun a, const float* _
                 }
             } else if (tk >= 0) {
                 const size_t n = (size_t)tk * a.nyx + pix;
-                if (n < (size_t)a.nz * a.nyx) v[p] = x[n];
+                if (MODE != GATHER_BEHIND || n < (size_t)a.nz * a.nyx) v[p] = x[n];
             }
         }
     }
@@ -410,7 +413,7 @@ __global__ __launch_bounds__(kPB) void k_plane_bp(PlaneRun a, uint32_t bpb, uint
         const size_t rows = (size_t)(a.bins + 1) * PL;
         plane_sums<PL, TOF, SENS>(a, pix, R + (TOF ? 0 : ch * rows) + p, W + (TOF ? 0 : ch * rows) + p, rhs, sens);
         if (CARRY) {
-            if (a.skip0 && tk == 0 && pix == 0) { rhs = 0.0; sens = 0.0; }   // the reference skips voxel 0
+            if (a.z && tk == 0 && pix == 0) { rhs = 0.0; sens = 0.0; }   // the interpolation reference skips voxel 0
             plane_carried<PL, SENS>(a, pix, tk, R, W, rhs, sens);
         }
         const size_t n = (size_t)tk * a.nyx + pix;
@@ -595,15 +598,15 @@ static bool plan_build(const omg_geom* g, PlanePlan* p, hipStream_t s) {
         tables.insert(tables.end(), p->slice_host.begin(), p->slice_host.end());
         size_t keep = 0, work = 0;
         auto take = [](size_t& at, uint64_t bytes) {
-            const size_t o = at;
-            at += ((size_t)bytes + 255) & ~(size_t)255;
+            const size_t unit = bytes >= (1u << 20) ? 2u << 20 : 256u, o = (at + unit - 1) & ~(unit - 1);
+            at = o + (size_t)bytes;
             return o;
         };
+        const size_t at_ent = take(interp ? work : keep, p->nent * 8);
         const size_t at_tables = take(keep, tables.size() * 4), at_cent = take(keep, nc * 8);
         const size_t at_w = take(keep, 4ull * bins * d.n_proj), at_samp = take(keep, ns * 16);
         const size_t at_share = take(keep, tof ? 4 * p->nent * p->pitch : 0), at_cpos = take(keep, tof ? 4 * nc : 0);
         // the interpolation projector's row lists serve the transposition only
-        const size_t at_ent = take(interp ? work : keep, p->nent * 8);
         const size_t at_key = take(work, nc * 4), at_val = take(work, nc * 8), at_lsum = take(work, tof ? 4 * p->nent : 0);
         ok = dev_alloc(&p->block, keep) && dev_alloc(&temp, work) &&
              hipMemcpyAsync(p->block + at_tables, tables.data(), tables.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess;
@@ -705,8 +708,8 @@ static int run_planes(omg_geom* g, const PlanePlan* pl, const PlaneRun& a, const
     hipEvent_t stop;
     timing_begin(s, &stop);
     const dim3 gg(grid_for((int64_t)a.xrows + 1, kPB), chunks);
-    if (pl->interp) hipLaunchKernelGGL((k_plane_gather<PL, true>), gg, dim3(kPB), 0, s, a, x, Xt);
-    else hipLaunchKernelGGL((k_plane_gather<PL, false>), gg, dim3(kPB), 0, s, a, x, Xt);
+    hipLaunchKernelGGL((pl->interp ? k_plane_gather<PL, GATHER_INTERP> : a.xrows > a.nyx ? k_plane_gather<PL, GATHER_BEHIND>
+                        : k_plane_gather<PL, GATHER_SLICE>), gg, dim3(kPB), 0, s, a, x, Xt);
     OMG_CHECK_LAUNCH();
     const uint32_t per_chunk = grid_for((int64_t)a.nyx * PL, kPB);
     const uint32_t others = (a.nyx + 4 * kPB - 1) / (4 * kPB) * a.nz;
@@ -761,16 +764,15 @@ int plane_subset_iteration(omg_geom* g, const PlanePlan* pl, int64_t first, int6
     const SidArgs sa = make_sid_args(g, first, n);
     PlaneRun a;
     a.bins = pl->bins; a.nyx = pl->nyx; a.npix = pl->npix; a.xrows = pl->xrows; a.planes = planes;
-    a.skip0 = pl->interp;
     a.nx = g->d.Nx;
     a.nz = g->d.Nz;
     a.off = pl->off; a.len = pl->len; a.soff = pl->soff; a.slen = pl->slen; a.coff = pl->coff; a.clen = pl->clen;
     a.ent = pl->ent; a.cent = pl->cent; a.samp = pl->samp; a.cpos = pl->cpos;
     a.w = pl->w + (size_t)first * pl->bins;
     a.slice = pl->slice + first;
-    a.nent = pl->nent;
+    a.nent = (uint32_t)pl->nent;      // below 2^32 (list_layout)
     a.share = pl->share;
-    a.z = g->z_dev + 2 * first;
+    a.z = pl->interp ? g->z_dev + 2 * first : nullptr;
     a.bz = g->d.bz;
     a.sz = (float)(1.0 / ((double)g->d.dz * g->d.Nz));
     *done = false;

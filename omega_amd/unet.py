@@ -81,7 +81,7 @@ class UNet3D:
         ends = np.cumsum([0] + [-(-v.numel() // 64) * 64 for v in self.p.values()])
         self._g_all = torch.zeros(int(ends[-1]), **f32)
         self.g = {k: self._g_all[int(o):int(o) + v.numel()].view(v.shape) for (k, v), o in zip(self.p.items(), ends)}
-        self._g_at = {k: g.data_ptr() for k, g in self.g.items()}
+        self._g_at = [g.data_ptr() for g in self.g.values()]
         self.m = {k: torch.zeros_like(v) for k, v in self.p.items()}
         self.v = {k: torch.zeros_like(v) for k, v in self.p.items()}
         self.wb = {}    # BF16 weights [27, cout, cin]
@@ -190,8 +190,9 @@ class UNet3D:
 
     def zero_grad(self):
         self._g_all.zero_()
-        for k, g in self.g.items():   # an entry that the caller has put in place of its view
-            if g.data_ptr() != self._g_at[k]:
+        at = list(map(self.torch.Tensor.data_ptr, self.g.values()))
+        if at != self._g_at:          # entries that the caller has put in place of their views
+            for g in self.g.values():
                 g.zero_()
 
     def backward(self, gout):

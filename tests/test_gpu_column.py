@@ -73,6 +73,33 @@ def test_column(cuda, nx, ny, nz, n_radial, n_angles, planes, first, dz):
     assert max(e[1:]) < BAR
 
 
+@pytest.mark.parametrize("k", [1, 3, 8, 14, 21])
+def test_ranges_built_together(cuda, k):
+    """Index tables of k equal ranges, called from the middle on: up to 8 are built at the first call, more at the second
+    in batches of 8. One range is not the same bins in every plane, and is traced."""
+    import torch
+    planes, per = 40, 21 * 16
+    grid, x, z = _scanner(20, 20, 9, 21, 16, planes)
+    b = per // k
+    bins = np.random.default_rng(k).permutation(per)[:k * b].reshape(k, b)
+    index = (np.arange(planes)[None, :, None] * per + bins[:, None, :]).astype(np.uint32)
+    odd = k - 1
+    index[odd, 7] = index[odd, 7][::-1]
+    img, n = torch.rand(grid.N, device="cuda") + 0.5, planes * b
+    out = []
+    for gen in (False, True):
+        g = make_geom(grid, x, z, 21, 16, meas_index=index.ravel(), generic=gen)
+        y = torch.empty(k * n, device="cuda")
+        back = torch.zeros(grid.N, device="cuda")
+        for r in [(i + k // 2) % k for i in range(k)]:
+            _lib.call("omg_forward_project", g.handle, r * n, n, ptr(img), ptr(y[r * n:]), None)
+            _lib.call("omg_backward_project", g.handle, r * n, n, ptr(y[r * n:]), ptr(back), None, None)
+        out.append((y.cpu().numpy(), back.cpu().numpy()))
+        assert list_calls(g) == (0, 0 if gen else 2 * (k - 1))
+    assert np.array_equal(out[0][0], out[1][0])
+    assert rel_l2(out[0][1], out[1][1]) < BAR
+
+
 def test_detectors_within_the_image(cuda):
     """LORs that start in the image are traced: their lengths are not the crossings' steps."""
     import torch
